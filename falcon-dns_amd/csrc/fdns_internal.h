@@ -253,7 +253,6 @@ void launch_solve(const RunDesc* runs, int nrun, const SolvePlan& pl, const Shap
 // (nothing launched) above that size
 bool launch_solve_T_m0(const RunDesc* runs, int nrun, const SolvePlan& pl, const Shape& sh, int stage, hipStream_t st);
 void launch_m0(const RunDesc* runs, int nrun, const Shape& sh, hipStream_t st);
-size_t solve_lds(const Shape& sh, int w);
 void launch_asm_T(double* A, const double* t, const double* D, const double* D2, const Shape& sh, int m0, int count,
                   double wtdt, double Pr, hipStream_t st);
 void launch_asm_F(double* A, const double* t, const double* D, const double* D2, const Shape& sh, int m0, int count,

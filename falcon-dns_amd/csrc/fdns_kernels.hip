@@ -742,6 +742,17 @@ __device__ __forceinline__ double rdl(double v, int l)
     return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned int)lo);
 }
 
+// Broadcast lane C of each quad of lanes to the quad (DPP quad_perm on both
+// halves): stays in vector registers, where v_readlane goes through scalar ones.
+template <int C>
+__device__ __forceinline__ double bcast4(double v)
+{
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)(b & 0xffffffffll), C * 0x55, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), C * 0x55, 0xf, 0xf, true);
+    return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned int)lo);
+}
+
 // Buffer resources (raw, stride 0): loads outside [0, bytes) return zero, so
 // the K padding of a product's last k-step and rows past the end of an array
 // read zeros without a bounds test.
@@ -753,6 +764,12 @@ __device__ __forceinline__ BRes bres(const void* base, size_t bytes)
 __device__ __forceinline__ double bload(BRes r, int off)
 {
     return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0));
+}
+// the same with a uniform part of the offset, s <= bytes (the range check is
+// off < bytes - s)
+__device__ __forceinline__ double2 bload2(BRes r, int off, int s)
+{
+    return __builtin_bit_cast(double2, __builtin_amdgcn_raw_buffer_load_b128(r, off, s, 0));
 }
 __device__ __forceinline__ double2 bload2(BRes r, int off)
 {
@@ -909,13 +926,12 @@ __device__ void lu_solve_k(double2* x, double2* xs, const double* __restrict__ A
     }
 }
 
-// lu_solve_k with the GEMV rows of a thread loaded one at a time (KR = 1,
-// the radial kernels, whose registers are spoken for) or two at a time.
-template <int NT, int NB, int KR = 1>
+// lu_solve_k with the GEMV rows of a thread loaded one at a time (the radial
+// kernels, whose registers are spoken for).
+template <int NT, int NB>
 __device__ void lu_solve(double2* x, double2* xs, const double* __restrict__ A, const int* __restrict__ perm, const int n)
 {
-    if (KR == 1 || n <= NT + NB) lu_solve_k<NT, NB, 1>(x, xs, A, perm, n);
-    else lu_solve_k<NT, NB, 2>(x, xs, A, perm, n);
+    lu_solve_k<NT, NB, 1>(x, xs, A, perm, n);
 }
 
 constexpr int SOLVE_NB = 8;    // column block of lu_solve
@@ -1013,6 +1029,273 @@ __device__ void lu_solve_wave(double (&xr)[SLOTS], Col col, const int n)
     if constexpr (SLOTS > 2) lu_wave_bwd<2, SLOTS, D>(xr, col, n);
     if constexpr (SLOTS > 1) lu_wave_bwd<1, SLOTS, D>(xr, col, n);
     lu_wave_bwd<0, SLOTS, D>(xr, col, n);
+}
+
+// ---- dgetrs('N', n, nrhs=1) with x in registers (the solves of LU mode)
+// One workgroup per right-hand side; thread t keeps rows 2t and 2t + 1 of x
+// (complex) for the whole solve, a wavefront 128 adjacent rows.  The sweeps go
+// by column blocks of eight: the block's eight values of x are finished by the
+// quad of lanes that holds those rows (lux_diag), published in LDS (two
+// buffers, so one barrier per block), and applied by every thread to its rows
+// below (above).  Each x(i) receives its column updates in dgetrs' column
+// order, the arithmetic of lu_solve.
+// What bounds it: the factor's bytes, read once, at many right-hand sides per
+// CU; the load instructions of the CU (about 27 cycles each) and the chain of
+// blocks at few.  So a load takes two adjacent rows (16 B per lane), a
+// wavefront whose rows are done only keeps the barriers, and the factor
+// entries of the next two blocks are always in flight in two register buffers
+// (loads without branches: the wait for one block leaves the other's out).
+//
+// Leading zeros: a column whose x(j) is zero updates nothing, so the forward
+// sweep starts at the block of the first non-zero entry of the permuted
+// right-hand side (as the reference BLAS's dtrsm skips them).  In the
+// vorticity-streamfunction system the psi rows and the wall rows, whose
+// right-hand sides are zero, are the pivot rows of the first N columns
+// (nothing else has entries there), so the first N of its 2N columns are never
+// read: 2.5 N^2 entries of the factor instead of 4 N^2.
+//
+// Measured per launch of all modes of one run, against x in LDS with one
+// wavefront solving the diagonal blocks (same results bit for bit):
+//   257 x 768   temperature 277 -> 123 us, coupled 620 -> 257 us
+//   513 x 1536  temperature 977 -> 675 us, coupled 2965 -> 1620 us (5.0 TB/s of
+//               the factor entries it has to read; a plain read takes 6.2)
+// Five wavefronts per SIMD (96 VGPRs) against four: 257 x 768 coupled 268 ->
+// 220 us in a loop of its own, 513 x 1536 within 4 % either way.  Three rows a
+// thread, 8-byte loads, every wavefront in every block: 294 and 2053 us; the
+// diagonal block's steps masked and divided by the compiler's divide, x_j by
+// v_readlane: 325 and 2936 us; 16-column blocks spill (1430 us).
+constexpr int LUX_NB = 8;      // columns per block
+constexpr int LUX_ROWS = 128;  // rows per wavefront
+__host__ __device__ constexpr int lux_waves(int n) { return (n + LUX_ROWS - 1) / LUX_ROWS; }
+constexpr int LUX_MAXT = 64 * lux_waves(2 * MAX_N);
+
+// Barrier of the LDS buffers only: the factor loads in flight stay in flight.
+__device__ __forceinline__ void lds_barrier()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// x / d by the reciprocal rcp = 1 / d (rounded): quotient, remainder,
+// correction (Markstein), which gives the correctly rounded quotient where
+// neither the reciprocal nor the remainder leaves the normal range.
+__device__ __forceinline__ double div_by(double x, double d, double rcp)
+{
+    const double q = x * rcp;
+    return fma(fma(-q, d, x), rcp, q);
+}
+
+// The 8 x 8 diagonal block of a sweep on a quad of lanes: lane l of the quad
+// holds rows 2l and 2l + 1 of x and of the block (a0, a1); jb rows are inside
+// the matrix.  Columns ascending (LOW: unit lower triangle) or descending, each
+// x_j divided by U_jj.  Entries on the wrong side of the diagonal count as
+// zero, so that a step of the chain is the broadcast of x_j and one fma per
+// row and part, without a mask or a branch; the division is three
+// multiply-adds by a reciprocal formed ahead of the chain, on every lane at
+// once, and the divided values are formed again for all lanes at the end.
+// Called by a whole wavefront, mine: the lane is in the block's quad; the
+// other lanes' x is left as it is.
+template <bool LOW>
+__device__ __forceinline__ void lux_diag(double2& x0, double2& x1, const double (&a0)[LUX_NB],
+                                         const double (&a1)[LUX_NB], const int jb, const bool mine)
+{
+    constexpr int NB = LUX_NB;
+    // rows l and l + 1 of the block; a lane that is not in it has no entries
+    const int l = mine ? 2 * ((int)threadIdx.x & 3) : jb;
+    auto fold = [&](auto J, double xr, double xm) {
+        constexpr int j = decltype(J)::value;
+        const double m0 = (LOW ? j < l : j > l && j < jb) && l < jb ? a0[j] : 0.0;
+        const double m1 = (LOW ? j < l + 1 : j > l + 1 && j < jb) && l + 1 < jb ? a1[j] : 0.0;
+        x0.x = fma(-xr, m0, x0.x);
+        x0.y = fma(-xm, m0, x0.y);
+        x1.x = fma(-xr, m1, x1.x);
+        x1.y = fma(-xm, m1, x1.y);
+    };
+    if constexpr (LOW) {
+        auto step = [&](auto J) {
+            constexpr int j = decltype(J)::value;
+            fold(J, bcast4<j / 2>(j & 1 ? x1.x : x0.x), bcast4<j / 2>(j & 1 ? x1.y : x0.y));
+        };
+        step(std::integral_constant<int, 0>{});
+        step(std::integral_constant<int, 1>{});
+        step(std::integral_constant<int, 2>{});
+        step(std::integral_constant<int, 3>{});
+        step(std::integral_constant<int, 4>{});
+        step(std::integral_constant<int, 5>{});
+        step(std::integral_constant<int, 6>{});
+    } else {
+        double d0 = 1.0, d1 = 1.0;
+#pragma unroll
+        for (int j = 0; j < NB; j += 2) {
+            d0 = (j == l && l < jb) ? a0[j] : d0;
+            d1 = (j == l && l + 1 < jb) ? a1[j + 1] : d1;
+        }
+        const double r0 = 1.0 / d0, r1 = 1.0 / d1;
+        auto sweep = [&](auto div) {
+            auto step = [&](auto J) {
+                constexpr int j = decltype(J)::value;
+                fold(J, bcast4<j / 2>(j & 1 ? div(x1.x, d1, r1) : div(x0.x, d0, r0)),
+                     bcast4<j / 2>(j & 1 ? div(x1.y, d1, r1) : div(x0.y, d0, r0)));
+            };
+            step(std::integral_constant<int, 7>{});
+            step(std::integral_constant<int, 6>{});
+            step(std::integral_constant<int, 5>{});
+            step(std::integral_constant<int, 4>{});
+            step(std::integral_constant<int, 3>{});
+            step(std::integral_constant<int, 2>{});
+            step(std::integral_constant<int, 1>{});
+            // the lanes and rows that are not in the block have d = r = 1
+            x0 = mk(div(x0.x, d0, r0), div(x0.y, d0, r0));
+            x1 = mk(div(x1.x, d1, r1), div(x1.y, d1, r1));
+        };
+        // a diagonal out of the range where the reciprocal is safe: divide
+        const auto safe = [](double d) { return fabs(d) > 0x1p-900 && fabs(d) < 0x1p900; };
+        if (__any(!(safe(d0) && safe(d1)))) sweep([](double x, double d, double) { return x / d; });
+        else sweep([](double x, double d, double r) { return div_by(x, d, r); });
+    }
+}
+
+// x0, x1: rows 2 tid and 2 tid + 1 of the permuted right-hand side (zero past
+// n), then of the solution; blockDim.x = 64 lux_waves(n); pub: 2 LUX_NB entries.
+__device__ __forceinline__ void lu_solve_reg(double2& x0, double2& x1, const double* __restrict__ A, const int n,
+                                             double2* pub)
+{
+    constexpr int NB = LUX_NB, WB = LUX_ROWS / LUX_NB;   // blocks per wavefront
+    const int tid = threadIdx.x, lane = tid & 63, r = 2 * tid;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int nblk = (n + NB - 1) / NB;
+    __shared__ int first;
+    // first block with a non-zero right-hand side
+    if (tid == 0) first = nblk;
+    __syncthreads();
+    if (r < n && !(x0.x == 0.0 && x0.y == 0.0 && x1.x == 0.0 && x1.y == 0.0)) atomicMin(&first, r / NB);
+    __syncthreads();
+    const int b0 = __builtin_amdgcn_readfirstlane(first);
+
+    // block b's columns of this thread's rows (LOW: rows >= j0; else rows
+    // < j0 + 8); rows and columns that are not wanted read past the end of the
+    // resource, zero, without a branch
+    double p0[NB], p1[NB], q0[NB], q1[NB];
+    const BRes Ar = bres(A, sizeof(double) * (size_t)n * n);
+    auto load = [&](double (&a0)[NB], double (&a1)[NB], int b, auto low) {
+        const int j0 = b * NB;
+        const bool want = b >= 0 && r < n && (decltype(low)::value ? r >= j0 : r < j0 + NB);
+        const int off = want ? 8 * r : 0x40000000;
+#pragma unroll
+        for (int j = 0; j < NB; ++j) {
+            const double2 v = bload2(Ar, off, 8 * n * min(max(j0 + j, 0), n));
+            a0[j] = v.x;
+            a1[j] = v.y;
+        }
+    };
+    // the diagonal block b, by the wavefront that holds its rows
+    auto diag = [&](const double (&a0)[NB], const double (&a1)[NB], int b, auto low) {
+        if (b < 0 || b >= nblk || b / WB != wv) return;
+        const bool in = (lane >> 2) == b % WB;
+        lux_diag<decltype(low)::value>(x0, x1, a0, a1, n - b * NB, in);
+        if (in) {
+            lstore(pub + NB * (b & 1) + 2 * (lane & 3), x0);
+            lstore(pub + NB * (b & 1) + 2 * (lane & 3) + 1, r + 1 < n ? x1 : mk(0.0, 0.0));
+        }
+    };
+    // block b (its x published): the other rows' updates, the next diagonal
+    // block, then the loads of block b + 2 (or b - 2) into b's buffer; blocks
+    // past either end update nothing
+    auto block = [&](double (&a0)[NB], double (&a1)[NB], const double (&n0)[NB], const double (&n1)[NB], int b, auto low) {
+        constexpr bool LOW = decltype(low)::value;
+        lds_barrier();
+        const int j0 = b * NB;
+        if (LOW ? (r >= j0 + NB && r < n) : r < j0) {
+#pragma unroll
+            for (int jj = 0; jj < NB; ++jj) {
+                const int j = LOW ? jj : NB - 1 - jj;
+                const double2 xj = lload(pub + NB * (b & 1) + j);
+                x0.x = fma(-xj.x, a0[j], x0.x);
+                x0.y = fma(-xj.y, a0[j], x0.y);
+                x1.x = fma(-xj.x, a1[j], x1.x);
+                x1.y = fma(-xj.y, a1[j], x1.y);
+            }
+        }
+        diag(n0, n1, LOW ? b + 1 : b - 1, low);
+        load(a0, a1, LOW ? b + 2 : b - 2, low);
+    };
+    // each sweep goes in pairs of blocks; a wavefront takes part up to its last
+    // (first) block and keeps the barriers after that
+    {
+        constexpr auto low = std::true_type{};
+        const int pairs = (nblk - b0 + 1) / 2, mine = min(pairs, max(0, (WB * wv + WB - b0 + 1) / 2));
+        if (mine > 0) {
+            load(p0, p1, b0, low);
+            load(q0, q1, b0 + 1, low);
+            diag(p0, p1, b0, low);
+            for (int k = 0; k < mine; ++k) {
+                block(p0, p1, q0, q1, b0 + 2 * k, low);
+                block(q0, q1, p0, p1, b0 + 2 * k + 1, low);
+            }
+        }
+        for (int k = 2 * mine; k < 2 * pairs; ++k) lds_barrier();
+    }
+    {
+        constexpr auto up = std::false_type{};
+        const int bt = nblk - 1;
+        const int pairs = (bt + 2) / 2, mine = (bt - WB * wv + 2) / 2;
+        load(p0, p1, bt, up);
+        load(q0, q1, bt - 1, up);
+        lds_barrier();   // every read of the forward sweep's last values is done
+        diag(p0, p1, bt, up);
+        for (int k = 0; k < mine; ++k) {
+            block(p0, p1, q0, q1, bt - 2 * k, up);
+            block(q0, q1, p0, p1, bt - 2 * k - 1, up);
+        }
+        for (int k = 2 * mine; k < 2 * pairs; ++k) lds_barrier();
+    }
+}
+
+// The implicit solves of one phase in LU mode (fdns_params.solver): one
+// workgroup per (run, mode), dgetrs in its operation order.  Modes go round
+// the XCDs and a mode's runs, which may share its factor, stay on one XCD's
+// L2.
+template <int phase>
+__global__ __launch_bounds__(LUX_MAXT) __attribute__((amdgpu_waves_per_eu(5))) void k_solve_lu(
+    const RunDesc* __restrict__ runs, const int nrun, const Shape sh, const int stage)
+{
+    __shared__ double2 pub[2 * LUX_NB];
+    const int N = sh.N, tid = threadIdx.x;
+    const int k = (int)blockIdx.x >> 3;
+    const int m = 8 * (k / nrun) + ((int)blockIdx.x & 7), ri = k % nrun;
+    if (m >= sh.Nm1) return;
+    const RunDesc& R = runs[ri];
+    const size_t MS = 2 * (size_t)N;     // solve-area entries per mode
+    const double2* v = (const double2*)R.sx + (size_t)m * MS;
+    double2* y = (double2*)R.sy + (size_t)m * MS;
+    // o: the system's row 0 in the solve area; z: rows below z have zero
+    // right-hand sides (the psi rows of the coupled system)
+    const double* A;
+    const int* perm;
+    int n = N, o = 0, z = 0;
+    if (phase == 0) {
+        A = R.TiS[stage] + (size_t)m * N * N;
+        perm = R.pTS[stage] + (size_t)m * N;
+    } else if (m == 0) {
+        A = R.UiS[stage];
+        perm = R.pUS[stage];
+        o = N;
+    } else {
+        A = R.FiS[stage] + (size_t)(m - 1) * 4 * N * N;
+        perm = R.pFS[stage] + (size_t)(m - 1) * 2 * N;
+        n = 2 * N;
+        z = N;
+    }
+    auto rhs = [&](int r) {
+        const int p = r < n ? gload(perm + r) : -1;
+        return p >= z ? gload(v + o + p) : mk(0.0, 0.0);
+    };
+    double2 x0 = rhs(2 * tid), x1 = rhs(2 * tid + 1);
+    lu_solve_reg(x0, x1, A, n, pub);
+    const bool real_out = phase == 1 && m == 0;
+    if (2 * tid < n) gstore(y + o + 2 * tid, mk(x0.x, real_out ? 0.0 : x0.y));
+    if (2 * tid + 1 < n) gstore(y + o + 2 * tid + 1, mk(x1.x, real_out ? 0.0 : x1.y));
 }
 
 constexpr int SOLVE_KC = 16;   // MFMA k-steps (4 columns of A each) loaded ahead per wavefront
@@ -1169,9 +1452,9 @@ __device__ void m0_solve(const RunDesc& R, const Shape& sh, double2* smem)
 //   (phase 0, inverse mode) the launch's first blocks solve it for runs
 //   0..m0n-1 (m0_solve), the rest do the batched solves; otherwise k_m0
 //   solves it beside this kernel.
-template <int phase, bool LU>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(LU ? 3 : 1))) void k_solve(const RunDesc* __restrict__ runs, const int nrun, const SolvePlan pl,
-                                              const Shape sh, const int stage, const int m0n)
+template <int phase>
+__global__ __launch_bounds__(NT) void k_solve(const RunDesc* __restrict__ runs, const SolvePlan pl, const Shape sh,
+                                              const int m0n)
 {
     extern __shared__ double2 smem[];
     __shared__ const double2* sxp[SOLVE_RHS];
@@ -1179,36 +1462,6 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(LU ? 3 : 1))
     const int N = sh.N, Nm1 = sh.Nm1, tid = threadIdx.x;
     const size_t MS = 2 * (size_t)N;     // solve-area entries per mode
     int w;
-    auto lu_one = [&](const RunDesc& R, const int m) {
-        double2* x = smem;
-        double2* xs = smem + 2 * N;
-        const double2* v = (const double2*)R.sx + (size_t)m * MS;
-        double2* y = (double2*)R.sy + (size_t)m * MS;
-        if (phase == 0) {
-            for (int i = tid; i < N; i += NT) lstore(x + i, gload(v + i));
-            __syncthreads();
-            lu_solve<NT, SOLVE_NB, 2>(x, xs, R.TiS[stage] + (size_t)m * N * N, R.pTS[stage] + (size_t)m * N, N);
-            for (int i = tid; i < N; i += NT) gstore(y + i, lload(x + i));
-        } else if (m == 0) {
-            for (int i = tid; i < N; i += NT) lstore(x + i, gload(v + N + i));
-            __syncthreads();
-            lu_solve<NT, SOLVE_NB, 2>(x, xs, R.UiS[stage], R.pUS[stage], N);
-            for (int i = tid; i < N; i += NT) gstore(y + N + i, mk(lload(x + i).x, 0.0));
-        } else {
-            for (int i = tid; i < 2 * N; i += NT) lstore(x + i, i < N ? mk(0.0, 0.0) : gload(v + i));
-            __syncthreads();
-            lu_solve<NT, SOLVE_NB, 2>(x, xs, R.FiS[stage] + (size_t)(m - 1) * 4 * N * N,
-                                      R.pFS[stage] + (size_t)(m - 1) * 2 * N, 2 * N);
-            for (int i = tid; i < 2 * N; i += NT) gstore(y + i, lload(x + i));
-        }
-    };
-    if constexpr (LU) {
-        if (!map_work(nrun * Nm1, w)) return;
-        int m, ri;
-        split_mode_major(w, nrun, m, ri);
-        lu_one(runs[ri], m);
-        return;
-    }
     int b0 = 0;   // blocks before b0: the m = 0 solves (a multiple of 8)
     if constexpr (phase == 0) {
         if (m0n > 0) {
@@ -3512,8 +3765,7 @@ int kernels_init()
     SETLDS4(k_rkx_init) SETLDS4(k_rkx_update) SETLDS4(k_rkx_rhs) SETLDS4(k_budget_dr) SETLDS4(k_budget)
     SETLDS4(k_spectra)
 #undef SETLDS4
-    SETLDS(k_lu) SETLDS((k_solve<0, false>)) SETLDS((k_solve<1, false>)) SETLDS((k_solve<0, true>))
-    SETLDS((k_solve<1, true>)) SETLDS(k_m0)
+    SETLDS(k_lu) SETLDS(k_solve<0>) SETLDS(k_solve<1>) SETLDS(k_m0)
 #define SETTILE(k) SETLDS((k<4, true, false>)) SETLDS((k<8, true, false>))
 #define SETTILEPF(k) SETTILE(k) SETLDS((k<4, true, true>)) SETLDS((k<8, true, true>)) \
     SETLDS((k<4, false, true>)) SETLDS((k<8, false, true>))
@@ -3673,13 +3925,9 @@ void launch_rkx_rhs(const RunDesc* runs, int nrun, const Shape& sh, int s, hipSt
     RADIAL_LAUNCH(k_rkx_rhs, s);
 }
 
-// LDS of k_solve: the two 2N vectors of dgetrs, or the staged right-hand
-// sides of the widest chunk (w real columns) of a batched phase.
-size_t solve_lds(const Shape& sh, int w)
-{
-    const size_t k4 = 4 * (((size_t)sh.N + 3) / 4);
-    return std::max(sizeof(double2) * 4 * (size_t)sh.N, sizeof(double) * k4 * (size_t)w);
-}
+// LDS of k_solve: the staged right-hand sides of the widest chunk (w real
+// columns) of a batched phase.
+static size_t solve_lds(const Shape& sh, int w) { return sizeof(double) * 4 * (((size_t)sh.N + 3) / 4) * (size_t)w; }
 
 void launch_m0(const RunDesc* runs, int nrun, const Shape& sh, hipStream_t st)
 {
@@ -3689,23 +3937,20 @@ void launch_m0(const RunDesc* runs, int nrun, const Shape& sh, hipStream_t st)
 void launch_solve(const RunDesc* runs, int nrun, const SolvePlan& pl, const Shape& sh, int phase, int lu,
                   int stage, hipStream_t st, int m0n)
 {
-    const int b0 = (m0n + 7) & ~7;
-    int total;
-    if (lu) total = nrun * sh.Nm1;
-    else if (phase == 0) total = pl.nchT * sh.Nm * solve_groups(sh.N, 0);
-    else total = pl.nchF * sh.Nm1 * solve_groups(sh.N, 1);
-    size_t lds = solve_lds(sh, lu ? 0 : (phase == 0 ? pl.wT : pl.wF));
-    if (m0n > 0) lds = std::max(lds, sizeof(double2) * (size_t)sh.N + sizeof(double) * (64 * (size_t)sh.N + 128));
-    // the dgetrs-order solves in a kernel of their own, so that their
-    // registers do not cost the batched inverse products occupancy
-    const dim3 g(b0 + padded_grid(total));
     if (lu) {
-        if (phase == 0) hipLaunchKernelGGL((k_solve<0, true>), g, dim3(NT), lds, st, runs, nrun, pl, sh, stage, 0);
-        else hipLaunchKernelGGL((k_solve<1, true>), g, dim3(NT), lds, st, runs, nrun, pl, sh, stage, 0);
-    } else {
-        if (phase == 0) hipLaunchKernelGGL((k_solve<0, false>), g, dim3(NT), lds, st, runs, nrun, pl, sh, stage, m0n);
-        else hipLaunchKernelGGL((k_solve<1, false>), g, dim3(NT), lds, st, runs, nrun, pl, sh, stage, 0);
+        // the dgetrs-order solves: modes round the XCDs, a mode's runs together
+        const dim3 g(8 * ((sh.Nm1 + 7) / 8) * nrun);
+        if (phase == 0) hipLaunchKernelGGL((k_solve_lu<0>), g, dim3(64 * lux_waves(sh.N)), 0, st, runs, nrun, sh, stage);
+        else hipLaunchKernelGGL((k_solve_lu<1>), g, dim3(64 * lux_waves(2 * sh.N)), 0, st, runs, nrun, sh, stage);
+        return;
     }
+    const int b0 = (m0n + 7) & ~7;
+    const int total = phase == 0 ? pl.nchT * sh.Nm * solve_groups(sh.N, 0) : pl.nchF * sh.Nm1 * solve_groups(sh.N, 1);
+    size_t lds = solve_lds(sh, phase == 0 ? pl.wT : pl.wF);
+    if (m0n > 0) lds = std::max(lds, sizeof(double2) * (size_t)sh.N + sizeof(double) * (64 * (size_t)sh.N + 128));
+    const dim3 g(b0 + padded_grid(total));
+    if (phase == 0) hipLaunchKernelGGL((k_solve<0>), g, dim3(NT), lds, st, runs, pl, sh, m0n);
+    else hipLaunchKernelGGL((k_solve<1>), g, dim3(NT), lds, st, runs, pl, sh, 0);
 }
 
 bool launch_solve_T_m0(const RunDesc* runs, int nrun, const SolvePlan& pl, const Shape& sh, int stage, hipStream_t st)
