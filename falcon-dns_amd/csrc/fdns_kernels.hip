@@ -20,7 +20,8 @@
 //   k_asm_*     operator matrices of mat_build / mat_build_IRK /
 //               mat_build_uphibar (mat_assembly.F90:68-413), one workgroup per
 //               (mode, column), a chunk of modes per launch.
-//   k_lu        one workgroup per matrix: blocked right-looking LU with
+//   k_lu, k_lu_small
+//               one workgroup per matrix: blocked right-looking LU with
 //               partial pivoting whose per-element arithmetic is dgetf2's.
 //   k_inv       the needed columns of each operator's inverse from its LU
 //               factor (dgetrs on unit vectors), a wavefront per block of
@@ -774,6 +775,12 @@ __device__ __forceinline__ double2 bload2(BRes r, int off, int s)
 __device__ __forceinline__ double2 bload2(BRes r, int off)
 {
     return __builtin_bit_cast(double2, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
+}
+// Store inside [0, bytes); a store outside does nothing.
+__device__ __forceinline__ void bstore(BRes r, int off, double v)
+{
+    typedef int i2 __attribute__((ext_vector_type(2)));
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(i2, v), r, off, 0, 0);
 }
 // LDS-direct load (buffer_load_dwordx4 ... lds): each lane's 16 bytes at
 // byte offset off of r land in LDS at lds + 16 * lane (lds uniform over the
@@ -3217,130 +3224,567 @@ __global__ __launch_bounds__(NT) void k_asm_U(double* __restrict__ A, const doub
 }
 
 // ------------------------------------------------------------------ LU factor
-constexpr int LU_NB = 8;
+// LU with partial pivoting of one n x n column-major matrix per workgroup,
+// column panels of 16, right-looking.  Each element sees exactly dgetf2's
+// sequence of operations (pivot = first max |a|, column scaled by the
+// reciprocal pivot, a(i,k) = fma(-l(i,j), u(j,k), a(i,k)) for j = 0, 1, ...):
+// the trailing update is v_mfma_f64_16x16x4f64, whose outputs are that chain
+// of fma in ascending j.
+//
+// With the few hundred matrices of an operator set each CU has one or two, so
+// the chain of columns bounds it, then the trailing matrix's passes through
+// L2.  Hence:
+//   - the panel is factored in registers, a row per thread, with one barrier
+//     per column: every wavefront publishes its best candidate with its whole
+//     panel row, and each thread then picks the pivot among them;
+//   - rows stay where they are (no interchanges); what dgetf2's interchanges
+//     would have made of them is kept as a position per row (it decides ties
+//     between equal candidates), and one pass at the end puts the factor's
+//     rows in order;
+//   - the panel's multipliers (zero for rows that are done) and the 16 rows of
+//     U feed the matrix cores from LDS, and every 16 x 16 tile of the trailing
+//     matrix is read and written once per panel, the next tile's loads in
+//     flight during the products.
+// Measured (time of one launch, against panels of 8 in LDS with a tree over
+// the workgroup per pivot search; same factors bit for bit): 97 matrices of
+// n = 65 214 -> 54 us (k_lu_small), 96 of 130 700 -> 140, 256 of 194 1810 ->
+// 430, 128 of 258 2900 -> 770, 768 of 514 38.9 -> 26 ms, 1536 of 1026 640 ->
+// 264 ms.
+constexpr int LU_NB = 16;
+constexpr int LU_PITCH = LU_NB + 1;
+constexpr int LU_CAND = LU_NB + 4;   // doubles of a wavefront's pivot candidate
 constexpr int LU_MAXN = 2 * MAX_N;
-
-// Blocked right-looking LU with partial pivoting of one n x n column-major
-// matrix per workgroup.  Each element sees exactly dgetf2's sequence of
-// operations (pivot = first max |a|, column scaled by the reciprocal pivot,
-// a(i,k) = fma(-l(i,j), u(j,k), a(i,k)) for j = 0, 1, ...); the panel of
-// LU_NB columns lives in LDS and the trailing matrix is streamed once per
-// panel.  Writes the net row permutation of dgetrs' interchanges.
-__global__ __launch_bounds__(NT) void k_lu(double* __restrict__ A_all, int* __restrict__ perm_all, const int n,
-                                           const size_t stride)
+__host__ __device__ constexpr int lu_n16(int n) { return (n + 15) & ~15; }
+// columns of U staged at a time: all of them up to n = 512, then what is left
+// of 160 KiB beside the panel
+__host__ __device__ constexpr int lu_chunk(int n) { return n <= 512 ? lu_n16(n) : 64; }
+__host__ __device__ constexpr size_t lu_lds(int n, int waves)
 {
-    extern __shared__ double P[];          // rows x LU_NB
-    __shared__ int ipiv[LU_MAXN];
-    __shared__ double redv[NT];
-    __shared__ int redi[NT];
+    return sizeof(double) * ((size_t)lu_n16(n) * LU_PITCH + (size_t)LU_NB * (lu_chunk(n) + 16) + LU_NB * LU_PITCH +
+                             2 * (size_t)waves * LU_CAND) +
+           sizeof(int) * ((size_t)lu_n16(n) + lu_n16(n) / 16);
+}
+
+// The larger of two numbers (a NaN loses), one instruction.
+__device__ __forceinline__ double vmax(double a, double b)
+{
+    double r;
+    asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+
+// Largest value over the wavefront (no NaN), in every lane.
+__device__ __forceinline__ double wave_max(double v)
+{
+    auto step = [&](auto ctrl, auto rows) {
+        const long long b = __double_as_longlong(v);
+        const int x = (int)(b & 0xffffffffll), y = (int)(b >> 32);
+        const int lo = __builtin_amdgcn_update_dpp(x, x, decltype(ctrl)::value, decltype(rows)::value, 0xf, false);
+        const int hi = __builtin_amdgcn_update_dpp(y, y, decltype(ctrl)::value, decltype(rows)::value, 0xf, false);
+        v = vmax(v, __longlong_as_double(((long long)hi << 32) | (long long)(unsigned int)lo));
+    };
+    step(std::integral_constant<int, 0x111>{}, std::integral_constant<int, 0xf>{});   // row_shr 1, 2, 4, 8
+    step(std::integral_constant<int, 0x112>{}, std::integral_constant<int, 0xf>{});
+    step(std::integral_constant<int, 0x114>{}, std::integral_constant<int, 0xf>{});
+    step(std::integral_constant<int, 0x118>{}, std::integral_constant<int, 0xf>{});
+    step(std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xa>{});   // row_bcast 15, 31
+    step(std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xc>{});
+    return rdl(v, 63);
+}
+
+template <int T, int RQ>
+__global__ __launch_bounds__(T) void k_lu(double* __restrict__ A_all, int* __restrict__ perm_all, const int n,
+                                          const size_t stride)
+{
+    constexpr int NB = LU_NB, W = T / 64, CD = LU_CAND;
+    extern __shared__ double sm[];
+    const int n16 = lu_n16(n), CB = lu_chunk(n), LDU = CB + 16, nrt = n16 >> 4;
+    double* const Lp = sm;                          // [row][16], pitch 17: multipliers of the panel
+    double* const Us = Lp + (size_t)n16 * LU_PITCH; // [16][LDU]: rows of U, a chunk of columns
+    double* const T11 = Us + NB * LDU;              // [16][17]: the panel's unit lower triangle
+    double* const cand = T11 + NB * LU_PITCH;       // [2][W]{value, position, reciprocal, -, 16 entries}
+    int* const prow = (int*)(cand + 2 * W * CD);   // row of pivot k
+    int* const left = prow + n16;                   // rows not yet done per 16-row tile
     double* A = A_all + (size_t)blockIdx.x * stride;
     int* perm = perm_all + (size_t)blockIdx.x * n;
-    const int tid = threadIdx.x;
-    const int wave = tid >> 6, lane = tid & 63;
-    const size_t ld = (size_t)n;
-    for (int k0 = 0; k0 < n; k0 += LU_NB) {
-        const int kb = min(LU_NB, n - k0);
-        const int rows = n - k0;
-        for (int idx = tid; idx < rows * kb; idx += NT) {
-            const int c = idx / rows, r = idx - c * rows;
-            P[r + rows * c] = A[(size_t)(k0 + r) + ld * (size_t)(k0 + c)];
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int li = lane & 15, lk = lane >> 4;
+    const BRes Ar = bres(A, sizeof(double) * (size_t)n * n);
+    int pos[RQ];          // position of this thread's rows under dgetf2's interchanges
+    bool act[RQ];         // not a pivot row yet
+#pragma unroll
+    for (int q = 0; q < RQ; ++q) {
+        pos[q] = tid + q * T;
+        act[q] = pos[q] < n;
+    }
+    for (int i = tid; i < n16 * LU_PITCH; i += T) Lp[i] = 0.0;   // rows past n stay zero
+    for (int i = tid; i < nrt; i += T) left[i] = min(16, n - 16 * i);
+    __syncthreads();
+    for (int k0 = 0; k0 < n; k0 += NB) {
+        const int kb = min(NB, n - k0);
+        // ---- the panel, rows in registers
+        double a[RQ][NB];
+        bool in[RQ];      // rows of the panel: those not done before it
+#pragma unroll
+        for (int q = 0; q < RQ; ++q) {
+            const int r = tid + q * T;
+            in[q] = act[q];
+            const int off = act[q] ? 8 * r : 0x40000000;
+#pragma unroll
+            for (int c = 0; c < NB; ++c) a[q][c] = bload(Ar, off + 8 * n * min(k0 + c, n));
+        }
+        // one column: the candidates, the pivot, its row on the others
+        auto column = [&](auto CC) {
+            constexpr int c = decltype(CC)::value;
+            if (c >= kb) return;
+            const int k = k0 + c;
+            double* const cd = cand + (size_t)(c & 1) * W * CD;
+            // this thread's candidate: the largest |a|, the first position on ties; a NaN is
+            // chosen only if there is nothing else
+            double v = -1.0, row[NB];
+            int p = 0x7fffffff;
+#pragma unroll
+            for (int j = 0; j < NB; ++j) row[j] = a[0][j];
+#pragma unroll
+            for (int q = 0; q < RQ; ++q) {
+                const double m0 = fabs(a[q][c]);
+                const double m = act[q] ? (m0 >= 0.0 ? m0 : -0.5) : -1.0;
+                const bool t = q == 0 || m > v || (m == v && act[q] && pos[q] < p);
+                v = t ? m : v;
+                p = t ? pos[q] : p;
+                if (q > 0) {
+#pragma unroll
+                    for (int j = 0; j < NB; ++j) {
+                        const double x = a[q][j];
+                        row[j] = t ? x : row[j];
+                    }
+                }
+            }
+            const double rc = 1.0 / row[c];   // off the chain: every candidate's reciprocal
+            const double vm = wave_max(v);
+            unsigned long long mask = __ballot(v == vm);
+            int best = __ffsll((long long)mask) - 1;
+            if (vm >= -0.5 && (mask & (mask - 1))) {   // equal candidates: the first position
+                int pb = __builtin_amdgcn_readlane(p, best);
+                for (mask &= mask - 1; mask; mask &= mask - 1) {
+                    const int l = __ffsll((long long)mask) - 1, pl = __builtin_amdgcn_readlane(p, l);
+                    if (pl < pb) { pb = pl; best = l; }
+                }
+            }
+            if (lane == best) {
+                double2* o = (double2*)(cd + wv * CD);
+                lstore(o, mk(v, (double)p));
+                lstore(o + 1, mk(rc, 0.0));
+#pragma unroll
+                for (int j = 0; j < NB; j += 2) lstore(o + 2 + j / 2, mk(row[j], row[j + 1]));
+            }
+            lds_barrier();
+            // the pivot among the wavefronts' candidates
+            double2 bv = lload((const double2*)cd);
+            int bw = 0;
+#pragma unroll
+            for (int w = 1; w < W; ++w) {
+                const double2 v2 = lload((const double2*)(cd + w * CD));
+                const bool t = v2.x > bv.x || (v2.x == bv.x && v2.y < bv.y);
+                bv = csel(t, v2, bv);
+                bw = t ? w : bw;
+            }
+            const double2* u = (const double2*)(cd + bw * CD);
+            const int pp = (int)bv.y;
+            const double rcp = lload(u + 1).x;
+            double ur[NB];
+#pragma unroll
+            for (int j = c & ~1; j < NB; j += 2) {
+                const double2 x = lload(u + 2 + j / 2);
+                ur[j] = x.x;
+                ur[j + 1] = x.y;
+            }
+            if (tid < NB) T11[c * LU_PITCH + tid] = (cd + bw * CD)[4 + tid];
+            const double piv = ur[c];
+            const bool byrcp = fabs(piv) >= DBL_MIN || piv == 0.0;   // uniform
+#pragma unroll
+            for (int q = 0; q < RQ; ++q) {
+                if (act[q] && pos[q] == pp) {      // the pivot row
+                    act[q] = false;
+                    pos[q] = k;
+                    prow[k] = tid + q * T;
+                    atomicSub(&left[(tid + q * T) >> 4], 1);
+                } else if (act[q]) {
+                    if (pos[q] == k) pos[q] = pp;  // the row it displaces
+                    const double l = byrcp ? (piv == 0.0 ? a[q][c] : a[q][c] * rcp) : a[q][c] / piv;
+                    a[q][c] = l;
+#pragma unroll
+                    for (int j = c + 1; j < NB; ++j) a[q][j] = fma(-l, ur[j], a[q][j]);
+                }
+            }
+        };
+        column(std::integral_constant<int, 0>{});
+        column(std::integral_constant<int, 1>{});
+        column(std::integral_constant<int, 2>{});
+        column(std::integral_constant<int, 3>{});
+        column(std::integral_constant<int, 4>{});
+        column(std::integral_constant<int, 5>{});
+        column(std::integral_constant<int, 6>{});
+        column(std::integral_constant<int, 7>{});
+        column(std::integral_constant<int, 8>{});
+        column(std::integral_constant<int, 9>{});
+        column(std::integral_constant<int, 10>{});
+        column(std::integral_constant<int, 11>{});
+        column(std::integral_constant<int, 12>{});
+        column(std::integral_constant<int, 13>{});
+        column(std::integral_constant<int, 14>{});
+        column(std::integral_constant<int, 15>{});
+        // the panel back to memory; its multipliers, zero for the rows that are done, to LDS
+#pragma unroll
+        for (int q = 0; q < RQ; ++q) {
+            const int r = tid + q * T;
+            if (in[q]) {
+#pragma unroll
+                for (int c = 0; c < NB; ++c)
+                    if (c < kb) gstore(A + (size_t)r + (size_t)n * (k0 + c), a[q][c]);
+#pragma unroll
+                for (int c = 0; c < NB; ++c) Lp[r * LU_PITCH + c] = act[q] ? a[q][c] : 0.0;
+            }
         }
         __syncthreads();
-        for (int c = 0; c < kb; ++c) {
-            double best = -1.0;
-            int bidx = 0x7fffffff;
-            for (int r = c + tid; r < rows; r += NT) {
-                const double v = fabs(P[r + rows * c]);
-                if (v > best) { best = v; bidx = r; }
-            }
-            redv[tid] = best;
-            redi[tid] = bidx;
-            __syncthreads();
-            for (int k = NT / 2; k > 0; k >>= 1) {
-                if (tid < k) {
-                    const double v2 = redv[tid + k];
-                    const int i2 = redi[tid + k];
-                    if (v2 > redv[tid] || (v2 == redv[tid] && i2 < redi[tid])) { redv[tid] = v2; redi[tid] = i2; }
+        // ---- the rows of U and the trailing update, a chunk of columns at a time
+        for (int j0 = k0 + NB; j0 < n; j0 += CB) {
+            const int nc = min(CB, n - j0);
+            for (int jj = tid; jj < CB; jj += T) {
+                double y[NB];
+                const bool ok = jj < nc;
+                const int co = 8 * n * (j0 + jj);
+#pragma unroll
+                for (int i = 0; i < NB; ++i) y[i] = bload(Ar, ok ? 8 * prow[k0 + i] + co : 0x40000000);
+#pragma unroll
+                for (int i = 0; i < NB - 1; ++i) {
+#pragma unroll
+                    for (int i2 = i + 1; i2 < NB; ++i2) y[i2] = fma(-T11[i2 * LU_PITCH + i], y[i], y[i2]);
+                    asm volatile("" ::: "memory");   // one column of the triangle in registers at a time
                 }
-                __syncthreads();
-            }
-            const int p = redi[0];
-            if (tid == 0) ipiv[k0 + c] = k0 + p;
-            const double pv = P[p + rows * c];
-            __syncthreads();
-            if (pv != 0.0) {
-                if (p != c && tid < kb) {
-                    const double a = P[c + rows * tid];
-                    P[c + rows * tid] = P[p + rows * tid];
-                    P[p + rows * tid] = a;
-                }
-                __syncthreads();
-                const double piv = P[c + rows * c];
-                if (fabs(piv) >= DBL_MIN) {
-                    const double rcp = 1.0 / piv;
-                    for (int r = c + 1 + tid; r < rows; r += NT) P[r + rows * c] = P[r + rows * c] * rcp;
-                } else {
-                    for (int r = c + 1 + tid; r < rows; r += NT) P[r + rows * c] = P[r + rows * c] / piv;
+#pragma unroll
+                for (int i = 0; i < NB; ++i) {
+                    if (ok) gstore(A + (size_t)prow[k0 + i] + (size_t)n * (j0 + jj), y[i]);
+                    Us[i * LDU + jj] = y[i];
                 }
             }
             __syncthreads();
-            for (int cc = c + 1; cc < kb; ++cc) {
-                const double u = P[c + rows * cc];
-                for (int r = c + 1 + tid; r < rows; r += NT) P[r + rows * cc] = fma(-P[r + rows * c], u, P[r + rows * cc]);
+            const int nct = (nc + 15) >> 4, nt = nrt * nct;
+            // tile t: rows 16 (t % nrt).., columns 16 (t / nrt)..; lane (lk, li) rows 4 r + lk of column li
+            auto at = [&](int t, int r) {
+                const int rt = t % nrt, ct = t / nrt;
+                const int row = 16 * rt + 4 * r + lk, col = j0 + 16 * ct + li;
+                return (t < nt && row < n && col < n) ? 8 * (row + n * col) : 0x40000000;
+            };
+            auto next = [&](int t) {   // this wavefront's next tile with rows left
+                while (t < nt && left[t % nrt] == 0) t += W;
+                return t;
+            };
+            dbl4 cur, nx;
+            int t = next(wv);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) cur[r] = bload(Ar, at(t, r));
+            while (t < nt) {
+                const int tn = next(t + W);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) nx[r] = bload(Ar, at(tn, r));
+                const int rt = t % nrt, ct = t / nrt;
+#pragma unroll
+                for (int s = 0; s < NB / 4; ++s)
+                    cur = __builtin_amdgcn_mfma_f64_16x16x4f64(-Lp[(16 * rt + li) * LU_PITCH + 4 * s + lk],
+                                                               Us[(4 * s + lk) * LDU + 16 * ct + li], cur, 0, 0, 0);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) bstore(Ar, at(t, r), cur[r]);
+                cur = nx;
+                t = tn;
             }
             __syncthreads();
         }
-        for (int idx = tid; idx < rows * kb; idx += NT) {
-            const int c = idx / rows, r = idx - c * rows;
-            A[(size_t)(k0 + r) + ld * (size_t)(k0 + c)] = P[r + rows * c];
-        }
-        // this panel's interchanges on the columns left and right of it
-        for (int col = tid; col < n; col += NT) {
-            if (col >= k0 && col < k0 + kb) continue;
-            double* cp = A + ld * (size_t)col;
-            for (int c = 0; c < kb; ++c) {
-                const int p = ipiv[k0 + c];
-                if (p != k0 + c) { const double a = cp[k0 + c]; cp[k0 + c] = cp[p]; cp[p] = a; }
-            }
-        }
-        __syncthreads();
-        // U12 = L11^{-1} A12 and A22 -= L21 U12, one wavefront per column
-        for (int col = k0 + kb + wave; col < n; col += NT / 64) {
-            double* cp = A + ld * (size_t)col;
-            double u = (lane < kb) ? cp[k0 + lane] : 0.0;
+    }
+    // rows into the order of the pivots, a wavefront per column
+    for (int col = wv; col < n; col += W) {
+        double v[(LU_MAXN + 63) / 64];
+        double* cp = A + (size_t)n * col;
 #pragma unroll
-            for (int j = 0; j < LU_NB - 1; ++j) {
-                if (j < kb - 1) {
-                    const double uj = __shfl(u, j);
-                    if (lane > j && lane < kb) u = fma(-P[lane + rows * j], uj, u);
+        for (int q = 0; q < (LU_MAXN + 63) / 64; ++q) {
+            const int i = lane + 64 * q;
+            if (64 * q < n) v[q] = i < n ? gload(cp + prow[i]) : 0.0;
+        }
+#pragma unroll
+        for (int q = 0; q < (LU_MAXN + 63) / 64; ++q) {
+            const int i = lane + 64 * q;
+            if (64 * q < n && i < n) gstore(cp + i, v[q]);
+        }
+    }
+    for (int i = tid; i < n; i += T) perm[i] = prow[i];
+}
+
+// k_lu for n <= 64 RQ (LU_SMALL_MAXN at most): the panel is factored by one wavefront (RQ rows per
+// lane: no barrier and no LDS in the chain of columns), which first brings the
+// panel's columns up to date and then factors it while the other wavefronts
+// update the columns behind it (one barrier per panel).  A column tile (16
+// columns) is one wavefront's work: its rows of U by the unit triangle, one
+// column at a time through the matrix cores (the products with the zeroed
+// entries add nothing), then all its 16-row tiles.
+constexpr int LU_SMALL_MAXN = 320;
+template <int RQ, int W>
+__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W / 4))) void k_lu_small(
+    double* __restrict__ A_all, int* __restrict__ perm_all, const int n, const size_t stride)
+{
+    constexpr int NB = LU_NB, P = LU_PITCH, MT = 4 * RQ;   // row tiles, HT of them in registers at a time
+    constexpr int HT = RQ <= 3 ? MT : MT / 2;
+    extern __shared__ double sm[];
+    const int n16 = lu_n16(n), nrt = n16 >> 4;
+    double* const Lb = sm;                               // 2 x [row][16], pitch 17: multipliers of a panel
+    double* const Tb = Lb + 2 * (size_t)n16 * P;         // 2 x [16][16], pitch 17: its unit lower triangle
+    int* const prow = (int*)(Tb + 2 * NB * P);           // row of pivot k
+    int* const tmask = prow + n16;                       // 2 x per 16-row tile: rows not yet done
+    double* A = A_all + (size_t)blockIdx.x * stride;
+    int* perm = perm_all + (size_t)blockIdx.x * n;
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int li = lane & 15, lk = lane >> 4;
+    const BRes Ar = bres(A, sizeof(double) * (size_t)n * n);
+    constexpr int OOB = 0x40000000;
+    int pos[RQ];          // wavefront 0: position of its rows under dgetf2's interchanges
+    bool act[RQ];         // not a pivot row yet
+#pragma unroll
+    for (int q = 0; q < RQ; ++q) {
+        pos[q] = lane + 64 * q;
+        act[q] = pos[q] < n;
+    }
+    for (int i = tid; i < 2 * n16 * P; i += 64 * W) Lb[i] = 0.0;   // rows past n stay zero
+    __syncthreads();
+
+    // the panel of columns k0.. in a (wavefront 0): factored, its multipliers
+    // (zero for rows that are done), triangle and row masks to the buffers of
+    // parity b.  A column's chain is the largest |a| over the wavefront, the
+    // pivot's reciprocal and the next column's update; the other updates are
+    // left between the next column's candidates and their use.
+    auto panel = [&](double (&a)[RQ][NB], const int k0, const int b) {
+        const int kb = min(NB, n - k0);
+        double m[RQ], vm;
+        // candidates of column c: |a|, a NaN below every number, done rows below all
+        auto candidates = [&](auto CC) {
+            constexpr int c = decltype(CC)::value;
+            double v = -1.0;
+#pragma unroll
+            for (int q = 0; q < RQ; ++q) {
+                const double x = vmax(fabs(a[q][c]), -0.5);
+                m[q] = act[q] ? x : -1.0;
+                v = q == 0 ? m[0] : vmax(v, m[q]);
+            }
+            vm = wave_max(v);
+        };
+        candidates(std::integral_constant<int, 0>{});
+        auto column = [&](auto CC) {
+            constexpr int c = decltype(CC)::value;
+            if (c >= kb) return;
+            const int k = k0 + c;
+            // the pivot: row slot qb of lane best, the first position among equals
+            unsigned long long M[RQ];
+            int qb = 0, best = 0, cnt = 0;
+#pragma unroll
+            for (int q = RQ - 1; q >= 0; --q) {
+                M[q] = __ballot(m[q] == vm);
+                cnt += __popcll(M[q]);
+                if (M[q]) { qb = q; best = __ffsll((long long)M[q]) - 1; }
+            }
+            if (cnt > 1) {
+                int pb = 0x7fffffff;
+#pragma unroll
+                for (int q = 0; q < RQ; ++q)
+                    for (unsigned long long t = M[q]; t; t &= t - 1) {
+                        const int l = __ffsll((long long)t) - 1, pl = __builtin_amdgcn_readlane(pos[q], l);
+                        if (pl < pb) { pb = pl; best = l; qb = q; }
+                    }
+            }
+            double u[NB];
+            int pp = 0;
+#pragma unroll
+            for (int q = 0; q < RQ; ++q) {
+                if (q == qb) {
+                    pp = __builtin_amdgcn_readlane(pos[q], best);
+#pragma unroll
+                    for (int j = c; j < NB; ++j) u[j] = rdl(a[q][j], best);
                 }
             }
-            if (lane < kb) cp[k0 + lane] = u;
-            double ub[LU_NB];
+            const double piv = u[c], rcp = 1.0 / piv;
+            double l[RQ];
 #pragma unroll
-            for (int j = 0; j < LU_NB; ++j) ub[j] = __shfl(u, j);
-            for (int r = k0 + kb + lane; r < n; r += 64) {
-                double a = cp[r];
+            for (int q = 0; q < RQ; ++q) l[q] = a[q][c] * rcp;
+            if (!(fabs(piv) >= DBL_MIN)) {       // (uniform) subnormal, zero or NaN
 #pragma unroll
-                for (int j = 0; j < LU_NB; ++j)
-                    if (j < kb) a = fma(-P[(r - k0) + rows * j], ub[j], a);
-                cp[r] = a;
+                for (int q = 0; q < RQ; ++q) l[q] = piv == 0.0 ? a[q][c] : a[q][c] / piv;
             }
+#pragma unroll
+            for (int q = 0; q < RQ; ++q) {
+                const bool is = pos[q] == pp;          // the pivot row, and the row it displaces
+                pos[q] = is ? k : (pos[q] == k ? pp : pos[q]);
+                act[q] = act[q] && !is;
+                a[q][c] = act[q] ? l[q] : a[q][c];
+                l[q] = act[q] ? l[q] : 0.0;
+                if constexpr (c + 1 < NB) a[q][c + 1] = fma(-l[q], u[c + 1], a[q][c + 1]);
+            }
+            if constexpr (c + 1 < NB) candidates(std::integral_constant<int, c + 1>{});
+#pragma unroll
+            for (int q = 0; q < RQ; ++q)
+#pragma unroll
+                for (int j = c + 2; j < NB; ++j) a[q][j] = fma(-l[q], u[j], a[q][j]);
+        };
+        column(std::integral_constant<int, 0>{});
+        column(std::integral_constant<int, 1>{});
+        column(std::integral_constant<int, 2>{});
+        column(std::integral_constant<int, 3>{});
+        column(std::integral_constant<int, 4>{});
+        column(std::integral_constant<int, 5>{});
+        column(std::integral_constant<int, 6>{});
+        column(std::integral_constant<int, 7>{});
+        column(std::integral_constant<int, 8>{});
+        column(std::integral_constant<int, 9>{});
+        column(std::integral_constant<int, 10>{});
+        column(std::integral_constant<int, 11>{});
+        column(std::integral_constant<int, 12>{});
+        column(std::integral_constant<int, 13>{});
+        column(std::integral_constant<int, 14>{});
+        column(std::integral_constant<int, 15>{});
+        double* const Lp = Lb + (size_t)b * n16 * P;
+        double* const T11 = Tb + b * NB * P;
+#pragma unroll
+        for (int q = 0; q < RQ; ++q) {
+            const int r = lane + 64 * q;
+            const unsigned long long mk_ = __ballot(act[q]);
+            if (lane < 4 && 4 * q + lane < nrt) tmask[b * nrt + 4 * q + lane] = (int)((mk_ >> (16 * lane)) & 0xffff);
+            if (!act[q] && pos[q] >= k0 && pos[q] < k0 + kb) {
+                prow[pos[q]] = r;
+#pragma unroll
+                for (int c = 0; c < NB; ++c) T11[(pos[q] - k0) * P + c] = a[q][c];
+            }
+            if (r < n16) {
+#pragma unroll
+                for (int c = 0; c < NB; ++c) Lp[r * P + c] = act[q] ? a[q][c] : 0.0;
+            }
+        }
+    };
+    // the panel of parity b to memory, by the wavefronts w0.. of nw: a column
+    // at a time, the rows left from the multipliers, its pivot rows from the
+    // triangle
+    auto store_panel = [&](const int k0, const int b, const int w, const int nw) {
+        const double* const Lp = Lb + (size_t)b * n16 * P;
+        const double* const T11 = Tb + b * NB * P;
+        const int kb = min(NB, n - k0);
+        for (int c = w; c < kb; c += nw) {
+            double* cp = A + (size_t)n * (k0 + c);
+            for (int r = lane; r < n; r += 64)
+                if ((tmask[b * nrt + (r >> 4)] >> (r & 15)) & 1) gstore(cp + r, Lp[r * P + c]);
+            if (lane < kb) gstore(cp + prow[k0 + lane], T11[lane * P + c]);
+        }
+    };
+    // columns j0 .. j0 + 15 brought up to date with the panel k0 of parity b
+    // (wavefront-wide); to(t, C): the finished 16-row tile t
+    auto update = [&](const int k0, const int b, const int j0, auto to) {
+        const double* const Lp = Lb + (size_t)b * n16 * P;
+        const double* const T11 = Tb + b * NB * P;
+        const int col = j0 + li, co = col < n ? 8 * n * col : OOB;
+        dbl4 Y, C[HT];
+        auto fetch = [&](int t0) {
+#pragma unroll
+            for (int t = 0; t < HT; ++t)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int row = 16 * (t0 + t) + 4 * r + lk;
+                    C[t][r] = bload(Ar, row < n ? 8 * row + co : OOB);
+                }
+        };
+#pragma unroll
+        for (int r = 0; r < 4; ++r) Y[r] = bload(Ar, 8 * prow[k0 + 4 * r + lk] + co);
+        fetch(0);
+        // Y <- T11^{-1} Y: row 4 r + lk of column li in register r, which is
+        // also the layout of the product's second operand
+#pragma unroll
+        for (int j = 0; j < NB - 1; ++j) {
+            const double x = T11[li * P + j];
+            Y = __builtin_amdgcn_mfma_f64_16x16x4f64(lk == (j & 3) && li > j ? -x : 0.0, Y[j >> 2], Y, 0, 0, 0);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) bstore(Ar, 8 * prow[k0 + 4 * r + lk] + co, Y[r]);
+#pragma unroll
+        for (int t0 = 0; t0 < MT; t0 += HT) {
+            if (t0 > 0) {
+                if (t0 >= nrt) break;
+                fetch(t0);
+            }
+#pragma unroll
+            for (int t = 0; t < HT; ++t) {
+                if (t0 + t >= nrt) break;
+                const int m = __builtin_amdgcn_readfirstlane(tmask[b * nrt + t0 + t]);
+                if (m == 0) continue;
+#pragma unroll
+                for (int s = 0; s < NB / 4; ++s)
+                    C[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(-Lp[(16 * (t0 + t) + li) * P + 4 * s + lk], Y[s], C[t], 0, 0, 0);
+                to(t0 + t, m, co, C[t]);
+            }
+        }
+    };
+    {
+        if (wv == 0) {
+            double a[RQ][NB];
+#pragma unroll
+            for (int q = 0; q < RQ; ++q)
+#pragma unroll
+                for (int c = 0; c < NB; ++c) a[q][c] = bload(Ar, act[q] ? 8 * (lane + 64 * q + n * min(c, n)) : OOB);
+            panel(a, 0, 0);
         }
         __syncthreads();
     }
-    // net permutation of the interchanges: perm[i] = original row of row i
-    __shared__ int pidx[LU_MAXN];
-    for (int i = tid; i < n; i += NT) pidx[i] = i;
+    int k0 = 0, b = 0;
+    for (; k0 + NB < n; k0 += NB, b ^= 1) {
+        if (wv == 0) {
+            // the next panel: its columns through the other buffer into rows, then factored
+            double* const Ln = Lb + (size_t)(b ^ 1) * n16 * P;
+            update(k0, b, k0 + NB, [&](int t, int, int, const dbl4& C) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) Ln[(16 * t + 4 * r + lk) * P + li] = C[r];
+            });
+            double a[RQ][NB];
+#pragma unroll
+            for (int q = 0; q < RQ; ++q)
+#pragma unroll
+                for (int c = 0; c < NB; ++c) a[q][c] = act[q] ? Ln[(lane + 64 * q) * P + c] : 0.0;
+            panel(a, k0 + NB, b ^ 1);
+        } else {
+            store_panel(k0, b, wv - 1, W - 1);
+            for (int j0 = k0 + NB * (1 + wv); j0 < n; j0 += NB * (W - 1))
+                update(k0, b, j0, [&](int t, int m, int co, const dbl4& C) {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        bstore(Ar, (m >> (4 * r + lk)) & 1 ? 8 * (16 * t + 4 * r + lk) + co : OOB, C[r]);
+                });
+        }
+        __syncthreads();
+    }
+    store_panel(k0, b, wv, W);
     __syncthreads();
-    if (tid == 0) {
-        for (int k = 0; k < n; ++k) {
-            const int p = ipiv[k];
-            if (p != k) { const int a = pidx[k]; pidx[k] = pidx[p]; pidx[p] = a; }
+    // rows into the order of the pivots, a wavefront per column
+    for (int col = wv; col < n; col += W) {
+        double v[RQ];
+        double* cp = A + (size_t)n * col;
+#pragma unroll
+        for (int q = 0; q < RQ; ++q) {
+            const int i = lane + 64 * q;
+            v[q] = i < n ? gload(cp + prow[i]) : 0.0;
+        }
+#pragma unroll
+        for (int q = 0; q < RQ; ++q) {
+            const int i = lane + 64 * q;
+            if (i < n) gstore(cp + i, v[q]);
         }
     }
-    __syncthreads();
-    for (int i = tid; i < n; i += NT) perm[i] = pidx[i];
+    for (int i = tid; i < n; i += 64 * W) perm[i] = prow[i];
+}
+__host__ __device__ constexpr size_t lu_small_lds(int n)
+{
+    return sizeof(double) * (2 * (size_t)lu_n16(n) + 2 * LU_NB) * LU_PITCH +
+           sizeof(int) * ((size_t)lu_n16(n) + 2 * (lu_n16(n) / 16));
 }
 
 // ------------------------------------------------------------------ inverse
@@ -3765,7 +4209,8 @@ int kernels_init()
     SETLDS4(k_rkx_init) SETLDS4(k_rkx_update) SETLDS4(k_rkx_rhs) SETLDS4(k_budget_dr) SETLDS4(k_budget)
     SETLDS4(k_spectra)
 #undef SETLDS4
-    SETLDS(k_lu) SETLDS(k_solve<0>) SETLDS(k_solve<1>) SETLDS(k_m0)
+    SETLDS((k_lu<512, 1>)) SETLDS((k_lu<512, 3>)) SETLDS((k_lu_small<1, 4>)) SETLDS((k_lu_small<2, 4>))
+    SETLDS((k_lu_small<3, 8>)) SETLDS((k_lu_small<4, 8>)) SETLDS((k_lu_small<5, 8>)) SETLDS(k_solve<0>) SETLDS(k_solve<1>) SETLDS(k_m0)
 #define SETTILE(k) SETLDS((k<4, true, false>)) SETLDS((k<8, true, false>))
 #define SETTILEPF(k) SETTILE(k) SETLDS((k<4, true, true>)) SETLDS((k<8, true, true>)) \
     SETLDS((k<4, false, true>)) SETLDS((k<8, false, true>))
@@ -4000,8 +4445,15 @@ void launch_inv(const double* LU, const int* perm, int n, size_t stride, int nma
 void launch_lu(double* A, int* perm, int n, size_t stride, int nmat, hipStream_t st)
 {
     if (nmat <= 0) return;
-    const size_t lds = sizeof(double) * (size_t)n * LU_NB;
-    hipLaunchKernelGGL(k_lu, dim3(nmat), dim3(NT), lds, st, A, perm, n, stride);
+#define LU_SMALL(RQ, W) hipLaunchKernelGGL((k_lu_small<RQ, W>), dim3(nmat), dim3(64 * (W)), lu_small_lds(n), st, A, perm, n, stride)
+    if (n <= 64) LU_SMALL(1, 4);
+    else if (n <= 128) LU_SMALL(2, 4);
+    else if (n <= 192) LU_SMALL(3, 8);
+    else if (n <= 256) LU_SMALL(4, 8);
+    else if (n <= LU_SMALL_MAXN) LU_SMALL(5, 8);
+#undef LU_SMALL
+    else if (n <= 512) hipLaunchKernelGGL((k_lu<512, 1>), dim3(nmat), dim3(512), lu_lds(n, 8), st, A, perm, n, stride);
+    else hipLaunchKernelGGL((k_lu<512, 3>), dim3(nmat), dim3(512), lu_lds(n, 8), st, A, perm, n, stride);
 }
 
 void launch_diag(const RunDesc* runs, int nrun, const Shape& sh, int record, double* out6, hipStream_t st)

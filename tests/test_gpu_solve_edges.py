@@ -44,3 +44,11 @@ def test_lu_mode_orders(fd, orc, Nr, mBC):
 @pytest.mark.parametrize("Nr", [12, 64, 65, 129])
 def test_lu_mode_orders_imexrk(fd, orc, Nr):
     check(fd, orc, Nr, 5, "ARS443", 2, "lu")
+
+
+# matrix orders N and 2N around the factorisation's panels (16 columns), its
+# rows per lane (64 each, up to 320 in one wavefront's registers) and the
+# multi-wavefront panels above (one row per thread to 512, three beyond)
+@pytest.mark.parametrize("Nr", [16, 17, 48, 80, 95, 160, 161, 256, 257])
+def test_lu_factor_orders(fd, orc, Nr):
+    check(fd, orc, Nr, 3, "CNAB2", 2, "lu")
