@@ -821,8 +821,11 @@ const ChebMats& cheb_matrices(int N)
     mul(e1, fw, g);
     ChebMats M;
     auto cvt = [&](const std::vector<ld>& v, std::vector<double>& o) {
-        o.resize(NN);
-        for (size_t t = 0; t < NN; ++t) o[t] = (double)v[t];
+        // columns padded to a multiple of 16 rows (Shape::LE)
+        const int LE = (N + 15) & ~15;
+        o.assign((size_t)LE * N, 0.0);
+        for (int j = 0; j < N; ++j)
+            for (int i = 0; i < N; ++i) o[i + (size_t)LE * j] = (double)v[i + (size_t)N * j];
     };
     cvt(e0, M.E0); cvt(e1, M.E1); cvt(e2, M.E2); cvt(fw, M.Fw); cvt(g, M.G);
     return cache.emplace(N, std::move(M)).first->second;
@@ -971,7 +974,10 @@ int shape_get(int N, int Nm, double eta, ShapeCtx** out)
     }
     const auto twm = twiddles(sh.M), twp = twiddles(sh.Np);
     const ChebMats& cm = cheb_matrices(N);
-    const size_t nb = sizeof(double2) * (twm.size() + twp.size()) + sizeof(double) * (3 * (size_t)N + 8 * (size_t)N * N);
+    sh.LE = (N + 15) & ~15;
+    const size_t mb = sizeof(double) * (size_t)sh.LE * N;
+    const size_t nb = sizeof(double2) * (twm.size() + twp.size()) + sizeof(double) * (3 * (size_t)N + 3 * (size_t)N * N) +
+                      256 + 5 * mb;
     if (hipMalloc(&C->mem, nb) != hipSuccess) { delete C; return fail(FDNS_ENOMEM, "hipMalloc shape constants"); }
     char* p = (char*)C->mem;
     auto put = [&](const void* src, size_t bytes) { void* d = p; hipMemcpy(d, src, bytes, hipMemcpyHostToDevice); p += bytes; return d; };
@@ -984,7 +990,7 @@ int shape_get(int N, int Nm, double eta, ShapeCtx** out)
     C->t = (const double*)put(t.data(), sizeof(double) * t.size());
     C->D = (const double*)put(D.data(), sizeof(double) * D.size());
     C->D2 = (const double*)put(D2.data(), sizeof(double) * D2.size());
-    const size_t mb = sizeof(double) * (size_t)N * N;
+    p = (char*)(((uintptr_t)p + 255) & ~(uintptr_t)255);
     sh.E0 = (const double*)put(cm.E0.data(), mb);
     sh.E1 = (const double*)put(cm.E1.data(), mb);
     sh.E2 = (const double*)put(cm.E2.data(), mb);
@@ -1621,6 +1627,10 @@ void imex_launches(const RunDesc* dev, int n, const Shape& sh, const SolveSched&
                    KTimer* kt, const Side* sd = nullptr)
 {
     if (first) TIMED(kt, FDNS_KC_OTHER, st, launch_imex_prep(dev, n, sh, st));
+    if (!kt && !ss.lu && mode_fused(sh, n)) {
+        launch_imex_modes(dev, n, sh, st);
+        return;
+    }
     TIMED(kt, FDNS_KC_IMEX_PRE, st, launch_imex_pre(dev, n, sh, st));
     m0_and_solve_T(dev, n, sh, ss, 0, st, kt, sd);
     TIMED(kt, FDNS_KC_IMEX_MID, st, launch_imex_mid(dev, n, sh, st));
@@ -1632,6 +1642,10 @@ void imex_launches(const RunDesc* dev, int n, const Shape& sh, const SolveSched&
 void stage_launches(const RunDesc* dev, int n, const Shape& sh, const SolveSched& ss, int s, hipStream_t st,
                     KTimer* kt, const Side* sd = nullptr)
 {
+    if (!kt && !ss.lu && mode_fused(sh, n)) {
+        launch_rk_modes(dev, n, sh, s, st);
+        return;
+    }
     TIMED(kt, FDNS_KC_RK_PRE, st, launch_rk_pre(dev, n, sh, s, st));
     m0_and_solve_T(dev, n, sh, ss, s, st, kt, sd);
     TIMED(kt, FDNS_KC_RK_MID, st, launch_rk_mid(dev, n, sh, s, st));

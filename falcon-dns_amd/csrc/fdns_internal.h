@@ -102,7 +102,10 @@ struct Shape {
     const double* rr;   // 1/r  (r_radius)
     const double* rr2;  // 1/r^2
     const double* rad;  // r
-    // the radial transforms as N x N matrices, column-major ([row + N col]):
+    // the radial transforms as N x N matrices, column-major ([row + LE col], LE =
+    // N rounded up to 16: a column starts on a cache line; the rows past N are
+    // zero), one behind the other:
+    int LE;
     const double* E0;   // chebinvtran    coefficients -> values
     const double* E1;   // chebinvtranD1  coefficients -> d/dr values
     const double* E2;   // chebinvtranD2  coefficients -> d2/dr2 values
@@ -224,6 +227,11 @@ void launch_imex_prep(const RunDesc* runs, int nrun, const Shape& sh, hipStream_
 void launch_imex_pre(const RunDesc* runs, int nrun, const Shape& sh, hipStream_t st);
 void launch_imex_mid(const RunDesc* runs, int nrun, const Shape& sh, hipStream_t st);
 void launch_imex_post(const RunDesc* runs, int nrun, const Shape& sh, hipStream_t st);
+// small launches in inverse mode: the whole mode update of an IMEX step or an
+// IMEXRK stage in one kernel, bit for bit what the tile and solve kernels give
+bool mode_fused(const Shape& sh, int nrun);
+void launch_imex_modes(const RunDesc* runs, int nrun, const Shape& sh, hipStream_t st);
+void launch_rk_modes(const RunDesc* runs, int nrun, const Shape& sh, int s, hipStream_t st);
 // ki, ke: 0-based history slot (counted back from the first step's slot) of
 // the implicit and explicit arrays to fill from the current state, or -1 for
 // every slot of the runs whose histories are not already filled

@@ -958,7 +958,21 @@ constexpr int SOLVE_NB = 8;    // column block of lu_solve
 // columns 64 Q .. 64 Q + 63 (D ahead of their use, within the slot), so a
 // caller may stage one slot's columns at a time.
 
-// forward sweep over the columns of slot Q
+// x / d by the reciprocal rcp = 1 / d (rounded): quotient, remainder,
+// correction (Markstein), which gives the correctly rounded quotient where
+// neither the reciprocal nor the remainder leaves the normal range.
+__device__ __forceinline__ double div_by(double x, double d, double rcp)
+{
+    const double q = x * rcp;
+    return fma(fma(-q, d, x), rcp, q);
+}
+
+// Whether a reciprocal may stand for the division by d (div_by).
+__device__ __forceinline__ bool rcp_safe(double d) { return fabs(d) > 0x1p-900 && fabs(d) < 0x1p900; }
+
+// forward sweep over the columns of slot Q.  A step of the chain is the
+// broadcast of x_j and one fma: the entries on and above the diagonal count as
+// zero, so that no row needs a mask.
 template <int Q, int SLOTS, int D, class Col>
 __device__ __forceinline__ void lu_wave_fwd(double (&xr)[SLOTS], Col col, const int n)
 {
@@ -968,19 +982,21 @@ __device__ __forceinline__ void lu_wave_fwd(double (&xr)[SLOTS], Col col, const 
     if (jlo >= n) return;
     double c[D][SLOTS];   // ring of prefetched columns
     auto column = [&](double (&cv)[SLOTS], int j) {
-        j = min(max(j, jlo), jhi);
+        j = min(j, jhi);
 #pragma unroll
-        for (int p = 0; p < SLOTS; ++p) cv[p] = col(p, j);
+        for (int p = Q; p < SLOTS; ++p) cv[p] = col(p, j);
     };
 #pragma unroll
     for (int d = 0; d < D; ++d) column(c[d], jlo + d);
+#pragma unroll 1
     for (int l0 = 0; l0 < 64 && jlo + l0 < n; l0 += D) {
 #pragma unroll
         for (int d = 0; d < D; ++d) {
             const int jl = l0 + d, j = jlo + jl;
             if (j < n) {
+                const double cq = lane > jl ? c[d][Q] : 0.0;   // at its use: the read is D columns old
                 const double xj = rdl(xr[Q], jl);
-                if (lane > jl) xr[Q] = fma(-xj, c[d][Q], xr[Q]);
+                xr[Q] = fma(-xj, cq, xr[Q]);
 #pragma unroll
                 for (int p = Q + 1; p < SLOTS; ++p) xr[p] = fma(-xj, c[d][p], xr[p]);
                 column(c[d], j + D);
@@ -989,7 +1005,10 @@ __device__ __forceinline__ void lu_wave_fwd(double (&xr)[SLOTS], Col col, const 
     }
 }
 
-// backward sweep over the columns of slot Q
+// backward sweep over the columns of slot Q.  Every lane divides its row by
+// its own diagonal entry at each step (three multiply-adds by a reciprocal
+// formed ahead; the divided value of lane j is broadcast), and the slot's rows
+// are divided once more at the end: the same quotients, without a mask.
 template <int Q, int SLOTS, int D, class Col>
 __device__ __forceinline__ void lu_wave_bwd(double (&xr)[SLOTS], Col col, const int n)
 {
@@ -997,33 +1016,43 @@ __device__ __forceinline__ void lu_wave_bwd(double (&xr)[SLOTS], Col col, const 
     const int qtop = (n - 1) >> 6, ltop = (n - 1) & 63;
     if (Q > qtop) return;
     const int jlo = 64 * Q, jhi = min(64 * Q + 63, n - 1);
-    double c[D][SLOTS];
-    auto column = [&](double (&cv)[SLOTS], int j) {
-        j = min(max(j, jlo), jhi);
-#pragma unroll
-        for (int p = 0; p < SLOTS; ++p) cv[p] = col(p, j);
-    };
-    // column j is step n-1-j of the sweep and sits in ring slot (n-1-j) mod D:
-    // the slot's first group starts `phase` entries in, so ring slots
-    // d < phase first serve the second group
     const int jtop = (Q == qtop) ? ltop : 63;
-    const int phase = (n - 1 - (64 * Q + jtop)) % D;
+    const bool row = lane <= jtop;
+    double dg = col(Q, jlo + min(lane, jtop));
+    if (!row) dg = 1.0;
+    const double rcp = 1.0 / dg;
+    auto sweep = [&](auto div) {
+        double c[D][SLOTS];
+        auto column = [&](double (&cv)[SLOTS], int j) {
+            j = min(max(j, jlo), jhi);
 #pragma unroll
-    for (int d = 0; d < D; ++d) column(c[d], jlo + jtop + phase - d - (d < phase ? D : 0));
-    for (int jh = jtop + phase; jh >= 0; jh -= D) {
+            for (int p = 0; p <= Q; ++p) cv[p] = col(p, j);
+        };
+        // column j is step n-1-j of the sweep and sits in ring slot (n-1-j) mod D:
+        // the slot's first group starts `phase` entries in, so ring slots
+        // d < phase first serve the second group
+        const int phase = (n - 1 - (64 * Q + jtop)) % D;
 #pragma unroll
-        for (int d = 0; d < D; ++d) {
-            const int jl = jh - d, j = jlo + jl;
-            if (jl >= 0 && jl <= jtop) {
-                if (lane == jl) xr[Q] = xr[Q] / c[d][Q];   // x_j / U_jj
-                const double xj = rdl(xr[Q], jl);
-                if (lane < jl) xr[Q] = fma(-xj, c[d][Q], xr[Q]);
+        for (int d = 0; d < D; ++d) column(c[d], jlo + jtop + phase - d - (d < phase ? D : 0));
+#pragma unroll 1
+        for (int jh = jtop + phase; jh >= 0; jh -= D) {
 #pragma unroll
-                for (int p = 0; p < Q; ++p) xr[p] = fma(-xj, c[d][p], xr[p]);
-                column(c[d], j - D);
+            for (int d = 0; d < D; ++d) {
+                const int jl = jh - d, j = jlo + jl;
+                if (jl >= 0 && jl <= jtop) {
+                    const double cq = lane < jl ? c[d][Q] : 0.0;
+                    const double xj = rdl(div(xr[Q]), jl);
+                    xr[Q] = fma(-xj, cq, xr[Q]);
+#pragma unroll
+                    for (int p = 0; p < Q; ++p) xr[p] = fma(-xj, c[d][p], xr[p]);
+                    column(c[d], j - D);
+                }
             }
         }
-    }
+        xr[Q] = div(xr[Q]);
+    };
+    if (__any(!rcp_safe(dg))) sweep([&](double x) { return x / dg; });
+    else sweep([&](double x) { return div_by(x, dg, rcp); });
 }
 
 // The whole solve with every column readable by col.
@@ -1082,15 +1111,6 @@ __device__ __forceinline__ void lds_barrier()
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
-// x / d by the reciprocal rcp = 1 / d (rounded): quotient, remainder,
-// correction (Markstein), which gives the correctly rounded quotient where
-// neither the reciprocal nor the remainder leaves the normal range.
-__device__ __forceinline__ double div_by(double x, double d, double rcp)
-{
-    const double q = x * rcp;
-    return fma(fma(-q, d, x), rcp, q);
 }
 
 // The 8 x 8 diagonal block of a sweep on a quad of lanes: lane l of the quad
@@ -1157,8 +1177,7 @@ __device__ __forceinline__ void lux_diag(double2& x0, double2& x1, const double 
             x1 = mk(div(x1.x, d1, r1), div(x1.y, d1, r1));
         };
         // a diagonal out of the range where the reciprocal is safe: divide
-        const auto safe = [](double d) { return fabs(d) > 0x1p-900 && fabs(d) < 0x1p900; };
-        if (__any(!(safe(d0) && safe(d1)))) sweep([](double x, double d, double) { return x / d; });
+        if (__any(!(rcp_safe(d0) && rcp_safe(d1)))) sweep([](double x, double d, double) { return x / d; });
         else sweep([](double x, double d, double r) { return div_by(x, d, r); });
     }
 }
@@ -2303,6 +2322,17 @@ __global__ __launch_bounds__(NT) void k_asm_LAP(double* __restrict__ A, const do
     }
 }
 
+// The mode updates below exist in two forms, the column tiles and the whole
+// mode updates, whose results must not differ: every multiplication and
+// addition outside the matrix products rounds by itself.
+#pragma clang fp contract(off)
+__device__ __forceinline__ double2 tadd(double2 a, double2 b) { return mk(a.x + b.x, a.y + b.y); }
+__device__ __forceinline__ double2 tsub(double2 a, double2 b) { return mk(a.x - b.x, a.y - b.y); }
+__device__ __forceinline__ double2 tsc(double s, double2 a) { return mk(s * a.x, s * a.y); }
+__device__ __forceinline__ double2 tneg(double2 a) { return mk(-a.x, -a.y); }
+// i*m*(1/r)*z, (ii*m*r_radius)*z of the reference (rhs_create.F90:99)
+__device__ __forceinline__ double2 timr(double m, double r, double2 z) { return mk(-((m * r) * z.y), (m * r) * z.x); }
+
 // ------------------------------------------------------------------ column tiles
 // The per-mode radial work of a step (Nm_maxLOOP, fourierloop.F90:108-230, and
 // Get_stage_var, fourierloop_imexrk.F90:169-393) as dense products over
@@ -2331,7 +2361,7 @@ struct ColIn {
 };
 
 // acc[2q + t] += Op_q X_{b(q)} for the P0 + P1 + P2 operators in ops (N x N,
-// column-major), the first P0 applied to block x0, the next P1 to x1, the last
+// column-major, leading dimension LE), the first P0 applied to block x0, the next P1 to x1, the last
 // P2 to x2 (t = 0 real, 1 imaginary parts).  A operand rows
 // arow = 16 st + li.  KC k-steps of every operand are loaded ahead of the
 // products.  Rows k >= N lie past the end of every resource and load as zero;
@@ -2339,15 +2369,15 @@ struct ColIn {
 // discarded.  Each output is the sum over k in ascending steps of four,
 // independent of the other columns.
 template <int P0, int P1, int P2, int KCMAX = 4>
-__device__ __forceinline__ void col_pass(const BRes* ops, const int N, const int arow, const ColIn x0, const ColIn x1,
-                                         const ColIn x2, dbl4* acc)
+__device__ __forceinline__ void col_pass(const BRes* ops, const int N, const int LE, const int arow, const ColIn x0,
+                                         const ColIn x1, const ColIn x2, dbl4* acc)
 {
     constexpr int NP = P0 + P1 + P2;
     constexpr int NX = (P0 > 0) + (P1 > 0) + (P2 > 0);
     constexpr int KC = (NP + 2 * NX <= 6 && KCMAX >= 4) ? 4 : 2;
     const int lk = (threadIdx.x & 63) >> 4;
     const int nk = (N + 3) >> 2;
-    const int ao = 8 * (arow + N * lk), astep = 32 * N;         // bytes
+    const int ao = 8 * (arow + LE * lk), astep = 32 * LE;       // bytes
     const BRes xs[3] = {x0.r, x1.r, x2.r};
     const int bo[3] = {x0.o + x0.st * lk, x1.o + x1.st * lk, x2.o + x2.st * lk};
     const int bstep[3] = {4 * x0.st, 4 * x1.st, 4 * x2.st};
@@ -2432,7 +2462,7 @@ __device__ __forceinline__ void stage_cols(double2* bs, const int N, const int K
 // col_pass with the B operands from the staged blocks (stage_cols): the same
 // products, each output summed over k in the same ascending steps of four.
 template <int P0, int P1, int P2, int KCMAX = 4>
-__device__ __forceinline__ void col_pass_lds(const BRes* ops, const int N, const int K4, const int arow,
+__device__ __forceinline__ void col_pass_lds(const BRes* ops, const int N, const int LE, const int K4, const int arow,
                                              const double2* bs, dbl4* acc)
 {
     constexpr int NP = P0 + P1 + P2;
@@ -2440,7 +2470,7 @@ __device__ __forceinline__ void col_pass_lds(const BRes* ops, const int N, const
     constexpr int KC = (NP <= 3 && KCMAX >= 4) ? 4 : 2;
     const int lane = threadIdx.x & 63, lk = lane >> 4, li = lane & 15;
     const int nk = (N + 3) >> 2;
-    const int ao = 8 * (arow + N * lk), astep = 32 * N;
+    const int ao = 8 * (arow + LE * lk), astep = 32 * LE;
     const int bo = lk * STG_PITCH + li, bstep = 4 * STG_PITCH, bslot = K4 * STG_PITCH;
     double a0[KC][NP], a1[KC][NP];
     double2 b0[KC][NX], b1[KC][NX];
@@ -2544,7 +2574,7 @@ __host__ __device__ inline int tile_split(bool allowed, int tiles) { return (all
     auto fres = [&](const double2* f, int nslot = 1) { return bres(f, fb * (size_t)nslot); };         \
     const int xo = 16 * m, xst = 16 * Nm1;   /* this lane's column, row stride (bytes) */              \
     const int sst = (int)fb;                 /* bytes between history / stage slots */                 \
-    const size_t ob = sizeof(double) * (size_t)N * N;                                                  \
+    const size_t ob = sizeof(double) * (size_t)sh.LE * N;                                              \
     const BRes E0 = bres(sh.E0, ob), E1 = bres(sh.E1, ob), E2 = bres(sh.E2, ob), G = bres(sh.G, ob);   \
     /* right-hand sides (sx) and solutions (sy), mode-major: rows 0..2N-1 of mode m at +2N m */        \
     const BRes syR = fres((const double2*)R.sy, 2);                                                    \
@@ -2565,8 +2595,8 @@ __host__ __device__ inline int tile_split(bool allowed, int tiles) { return (all
 // KC: at most KC k-steps of operands loaded ahead (4 or 2; fewer registers)
 #define COL_PASS_KC(KC, OPS, P0, P1, P2, X0, X1, X2)                            \
     do {                                                                       \
-        if (STG) col_pass_lds<P0, P1, P2, KC>(OPS, N, K4, arow, stg_, acc);    \
-        else col_pass<P0, P1, P2, KC>(OPS, N, arow, X0, X1, X2, acc);          \
+        if (STG) col_pass_lds<P0, P1, P2, KC>(OPS, N, sh.LE, K4, arow, stg_, acc); \
+        else col_pass<P0, P1, P2, KC>(OPS, N, sh.LE, arow, X0, X1, X2, acc);   \
     } while (0)
 
 // this lane's rows of strip st: index, validity, field byte offset; then
@@ -2653,27 +2683,27 @@ __global__ __launch_bounds__(64 * TW) __attribute__((amdgpu_waves_per_eu(2))) vo
         UNROLL for (int r = 0; r < 4; ++r) {
             Tn[r] = EPV(0, r, rT, fo[r]);
             const double2 upT = EPV(1, r, rUp, fo[r]), urT = EPV(2, r, rUr, fo[r]);
-            NT_[r] = cadd(cadd(cimr(mm, rri[r], upT), ACC(acc, 2, r)), csc(rri[r], urT));
+            NT_[r] = tadd(tadd(timr(mm, rri[r], upT), ACC(acc, 2, r)), tsc(rri[r], urT));
         }
         if (cn) {
             const double c = ((1.0 - R.wi[0]) * dt) * (1.0 / Pr);
             UNROLL for (int r = 0; r < 4; ++r) {
-                const double2 lap = csub(cadd(csc(rri[r], ACC(acc, 0, r)), ACC(acc, 1, r)), csc((mm * mm) * rr2i[r], Tn[r]));
-                r0[r] = cadd(Tn[r], csc(c, lap));
+                const double2 lap = tsub(tadd(tsc(rri[r], ACC(acc, 0, r)), ACC(acc, 1, r)), tsc((mm * mm) * rr2i[r], Tn[r]));
+                r0[r] = tadd(Tn[r], tsc(c, lap));
             }
         } else {
-            UNROLL for (int r = 0; r < 4; ++r) r0[r] = csc(R.wi[0], Tn[r]);
+            UNROLL for (int r = 0; r < 4; ++r) r0[r] = tsc(R.wi[0], Tn[r]);
             slot_sum<MAXH - 1>(1, ni, [&](int o, int r) { return bload2(rHi, slot(o) + fo[r]); },
                                [&](int o, const double2 (&x)[4]) {
                                    const double w = R.wi[o];
-                                   UNROLL for (int r = 0; r < 4; ++r) r0[r] = cadd(r0[r], csc(w, x[r]));
+                                   UNROLL for (int r = 0; r < 4; ++r) r0[r] = tadd(r0[r], tsc(w, x[r]));
                                });
         }
-        UNROLL for (int r = 0; r < 4; ++r) r0[r] = csub(r0[r], csc(dt, csc(R.we[0], NT_[r])));
+        UNROLL for (int r = 0; r < 4; ++r) r0[r] = tsub(r0[r], tsc(dt, tsc(R.we[0], NT_[r])));
         slot_sum<MAXH - 1>(1, ne, [&](int o, int r) { return bload2(rHe, slot(o) + fo[r]); },
                            [&](int o, const double2 (&x)[4]) {
                                const double w = R.we[o];
-                               UNROLL for (int r = 0; r < 4; ++r) r0[r] = csub(r0[r], csc(dt, csc(w, x[r])));
+                               UNROLL for (int r = 0; r < 4; ++r) r0[r] = tsub(r0[r], tsc(dt, tsc(w, x[r])));
                            });
         UNROLL for (int r = 0; r < 4; ++r) {
             if (!vr[r]) continue;
@@ -2742,7 +2772,7 @@ __global__ __launch_bounds__(64 * TW) __attribute__((amdgpu_waves_per_eu(2))) vo
             UNROLL for (int r = 0; r < 4; ++r) {
                 ub[r] = bload2(rUb, fo[r]);
                 uw[r] = bload(rUw, 8 * ir[r]);
-                const double2 ud = cadd(csub(ACC(acc, 2, r), csc(rr2i[r], ub[r])), csc(rri[r], ACC(acc, 1, r)));
+                const double2 ud = tadd(tsub(ACC(acc, 2, r), tsc(rr2i[r], ub[r])), tsc(rri[r], ACC(acc, 1, r)));
                 v[r] = cn ? ub[r].x + ((1.0 - R.wi[0]) * dt) * ud.x : R.wi[0] * ub[r].x;
             }
             if (!cn)
@@ -2775,37 +2805,37 @@ __global__ __launch_bounds__(64 * TW) __attribute__((amdgpu_waves_per_eu(2))) vo
         UNROLL for (int r = 0; r < 4; ++r) {
             Wn[r] = EPV(1, r, rWn, fo[r]);
             const double2 upW = EPV(2, r, rUp, fo[r]), urW = EPV(3, r, rUr, fo[r]);
-            NW[r] = cadd(cadd(cimr(mm, rri[r], upW), ACC(acc, 3, r)), csc(rri[r], urW));
+            NW[r] = tadd(tadd(timr(mm, rri[r], upW), ACC(acc, 3, r)), tsc(rri[r], urW));
         }
         if (cn) {
             UNROLL for (int r = 0; r < 4; ++r) {
-                const double2 lap = csub(cadd(csc(rri[r], ACC(acc, 1, r)), ACC(acc, 2, r)), csc((mm * mm) * rr2i[r], Wn[r]));
-                const double2 b1 = cimr(mm, rri[r], ACC(acc, 0, r));
-                const double2 b2 = cimr(mm, rri[r], bload2(rHT, slot(0) + fo[r]));
-                r2[r] = csub(cadd(Wn[r], csc((1.0 - R.wi[0]) * dt, lap)), csc((raPr * dt) * 0.5, cadd(b1, b2)));
-                r2[r] = csub(r2[r], csc(dt, csc(R.we[0], NW[r])));
+                const double2 lap = tsub(tadd(tsc(rri[r], ACC(acc, 1, r)), ACC(acc, 2, r)), tsc((mm * mm) * rr2i[r], Wn[r]));
+                const double2 b1 = timr(mm, rri[r], ACC(acc, 0, r));
+                const double2 b2 = timr(mm, rri[r], bload2(rHT, slot(0) + fo[r]));
+                r2[r] = tsub(tadd(Wn[r], tsc((1.0 - R.wi[0]) * dt, lap)), tsc((raPr * dt) * 0.5, tadd(b1, b2)));
+                r2[r] = tsub(r2[r], tsc(dt, tsc(R.we[0], NW[r])));
             }
             slot_sum<MAXH - 1>(1, ne, [&](int o, int r) { return bload2(rHe, slot(o) + fo[r]); },
                                [&](int o, const double2 (&x)[4]) {
                                    const double w = R.we[o];
-                                   UNROLL for (int r = 0; r < 4; ++r) r2[r] = csub(r2[r], csc(dt, csc(w, x[r])));
+                                   UNROLL for (int r = 0; r < 4; ++r) r2[r] = tsub(r2[r], tsc(dt, tsc(w, x[r])));
                                });
         } else {
-            UNROLL for (int r = 0; r < 4; ++r) r2[r] = csc(R.wi[0], Wn[r]);
+            UNROLL for (int r = 0; r < 4; ++r) r2[r] = tsc(R.wi[0], Wn[r]);
             slot_sum<MAXH - 1>(1, ni, [&](int o, int r) { return bload2(rHi, slot(o) + fo[r]); },
                                [&](int o, const double2 (&x)[4]) {
                                    const double w = R.wi[o];
-                                   UNROLL for (int r = 0; r < 4; ++r) r2[r] = cadd(r2[r], csc(w, x[r]));
+                                   UNROLL for (int r = 0; r < 4; ++r) r2[r] = tadd(r2[r], tsc(w, x[r]));
                                });
-            UNROLL for (int r = 0; r < 4; ++r) r2[r] = csub(r2[r], csc(dt, csc(R.we[0], NW[r])));
+            UNROLL for (int r = 0; r < 4; ++r) r2[r] = tsub(r2[r], tsc(dt, tsc(R.we[0], NW[r])));
             slot_sum<MAXH - 1>(1, ne, [&](int o, int r) { return bload2(rHe, slot(o) + fo[r]); },
                                [&](int o, const double2 (&x)[4]) {
                                    const double w = R.we[o];
-                                   UNROLL for (int r = 0; r < 4; ++r) r2[r] = csub(r2[r], csc(dt, csc(w, x[r])));
+                                   UNROLL for (int r = 0; r < 4; ++r) r2[r] = tsub(r2[r], tsc(dt, tsc(w, x[r])));
                                });
             UNROLL for (int r = 0; r < 4; ++r) {
-                const double2 bt = csc(-raPr, cimr(mm, rri[r], ACC(acc, 0, r)));
-                r2[r] = cadd(r2[r], csc(dt * R.wl, bt));
+                const double2 bt = tsc(-raPr, timr(mm, rri[r], ACC(acc, 0, r)));
+                r2[r] = tadd(r2[r], tsc(dt * R.wl, bt));
             }
         }
         UNROLL for (int r = 0; r < 4; ++r) {
@@ -2856,14 +2886,14 @@ __global__ __launch_bounds__(64 * TW) __attribute__((amdgpu_waves_per_eu(2))) vo
                 const double2 u = ACC(acc, 0, r);
                 upFR_[e] = u;
                 urFR_[e] = mk(0.0, 0.0);
-                omgFR_[e] = cadd(csc(rri[r], u), ACC(acc, 1, r));
+                omgFR_[e] = tadd(tsc(rri[r], u), ACC(acc, 1, r));
                 continue;
             }
             omgFR_[e] = ACC(acc, 0, r);
             const double2 ps = ACC(acc, 2, r);
             psi_[e] = ps;
-            upFR_[e] = cneg(ACC(acc, 3, r));
-            urFR_[e] = cimr(mm, rri[r], ps);
+            upFR_[e] = tneg(ACC(acc, 3, r));
+            urFR_[e] = timr(mm, rri[r], ps);
         }
     }
 }
@@ -2922,28 +2952,28 @@ __global__ __launch_bounds__(64 * TW) __attribute__((amdgpu_waves_per_eu(3))) vo
         double2 faT[4], faW[4], Fd[4], Fa[4];
         if (fa_prev) {
             UNROLL for (int r = 0; r < 4; ++r) {
-                faT[r] = cneg(cadd(cadd(cimr(mm, rri[r], EPV(1, r, rUpT, fo[r])), ACC(acc, 0, r)),
-                                   csc(rri[r], EPV(2, r, rUrT, fo[r]))));
+                faT[r] = tneg(tadd(tadd(timr(mm, rri[r], EPV(1, r, rUpT, fo[r])), ACC(acc, 0, r)),
+                                   tsc(rri[r], EPV(2, r, rUrT, fo[r]))));
                 if (m == 0) faW[r] = mk(-bload(rUw, 8 * ir[r]), 0.0);
-                else faW[r] = cneg(cadd(cadd(cimr(mm, rri[r], EPV(3, r, rUpW, fo[r])), ACC(acc, 1, r)),
-                                        csc(rri[r], EPV(4, r, rUrW, fo[r]))));
+                else faW[r] = tneg(tadd(tadd(timr(mm, rri[r], EPV(3, r, rUpW, fo[r])), ACC(acc, 1, r)),
+                                        tsc(rri[r], EPV(4, r, rUrW, fo[r]))));
             }
         }
         UNROLL for (int r = 0; r < 4; ++r) { Fd[r] = mk(0.0, 0.0); Fa[r] = mk(0.0, 0.0); }
         slot_sum<2>(0, s, [&](int k, int r) { return bload2(rFdT, k * sst + fo[r]); },
                     [&](int k, const double2 (&x)[4]) {
                         const double w = aD[k];
-                        UNROLL for (int r = 0; r < 4; ++r) Fd[r] = cadd(Fd[r], csc(w, x[r]));
+                        UNROLL for (int r = 0; r < 4; ++r) Fd[r] = tadd(Fd[r], tsc(w, x[r]));
                     });
         // the terms of stage s - 1 are the ones just formed when fa_prev
         slot_sum<2>(0, fa_prev ? s - 1 : s, [&](int k, int r) { return bload2(rFaT, k * sst + fo[r]); },
                     [&](int k, const double2 (&x)[4]) {
                         const double w = aA[k];
-                        UNROLL for (int r = 0; r < 4; ++r) Fa[r] = cadd(Fa[r], csc(w, x[r]));
+                        UNROLL for (int r = 0; r < 4; ++r) Fa[r] = tadd(Fa[r], tsc(w, x[r]));
                     });
-        if (fa_prev) UNROLL for (int r = 0; r < 4; ++r) Fa[r] = cadd(Fa[r], csc(aA[s - 1], faT[r]));
+        if (fa_prev) UNROLL for (int r = 0; r < 4; ++r) Fa[r] = tadd(Fa[r], tsc(aA[s - 1], faT[r]));
         double2 v[4];
-        UNROLL for (int r = 0; r < 4; ++r) v[r] = cadd(EPV(0, r, rTs, fo[r]), csc(dt, cadd(Fd[r], Fa[r])));
+        UNROLL for (int r = 0; r < 4; ++r) v[r] = tadd(EPV(0, r, rTs, fo[r]), tsc(dt, tadd(Fd[r], Fa[r])));
         UNROLL for (int r = 0; r < 4; ++r) {
             if (!vr[r]) continue;
             const int i = ir[r];
@@ -3007,17 +3037,17 @@ __global__ __launch_bounds__(64 * TW) __attribute__((amdgpu_waves_per_eu(2))) vo
         UNROLL for (int r = 0; r < 4; ++r) {
             y0[r] = (m == 0) ? bload2(rUb, 16 * ir[r]) : EPV(0, r, rWs, fo[r]);
             Fd[r] = mk(0.0, 0.0); Fa[r] = mk(0.0, 0.0); Fb[r] = mk(0.0, 0.0);
-            bu[r] = csc(-raPr, cimr(mm, rri[r], ACC(acc, 0, r)));   // buoyancy of this stage
+            bu[r] = tsc(-raPr, timr(mm, rri[r], ACC(acc, 0, r)));   // buoyancy of this stage
         }
         slot_sum<2>(0, s, [&](int k, int r) { return bload2(rFdW, k * sst + fo[r]); },
                     [&](int k, const double2 (&x)[4]) {
                         const double w = aD[k];
-                        UNROLL for (int r = 0; r < 4; ++r) Fd[r] = cadd(Fd[r], csc(w, x[r]));
+                        UNROLL for (int r = 0; r < 4; ++r) Fd[r] = tadd(Fd[r], tsc(w, x[r]));
                     });
         slot_sum<2>(0, s, [&](int k, int r) { return bload2(rFaW, k * sst + fo[r]); },
                     [&](int k, const double2 (&x)[4]) {
                         const double w = aA[k];
-                        UNROLL for (int r = 0; r < 4; ++r) Fa[r] = cadd(Fa[r], csc(w, x[r]));
+                        UNROLL for (int r = 0; r < 4; ++r) Fa[r] = tadd(Fa[r], tsc(w, x[r]));
                     });
         if (m > 0) {
             // the buoyancy terms: weights aD (implicit buoyancy) or aA
@@ -3025,9 +3055,9 @@ __global__ __launch_bounds__(64 * TW) __attribute__((amdgpu_waves_per_eu(2))) vo
             slot_sum<2>(0, s, [&](int k, int r) { return bload2(rFb, k * sst + fo[r]); },
                         [&](int k, const double2 (&x)[4]) {
                             const double w = wb[k];
-                            UNROLL for (int r = 0; r < 4; ++r) Fb[r] = cadd(Fb[r], csc(w, x[r]));
+                            UNROLL for (int r = 0; r < 4; ++r) Fb[r] = tadd(Fb[r], tsc(w, x[r]));
                         });
-            if (bimp) UNROLL for (int r = 0; r < 4; ++r) Fb[r] = cadd(Fb[r], csc(aD[s], bu[r]));
+            if (bimp) UNROLL for (int r = 0; r < 4; ++r) Fb[r] = tadd(Fb[r], tsc(aD[s], bu[r]));
         }
         double2 xc[4];
         if (last && m == 0) UNROLL for (int r = 0; r < 4; ++r) xc[r] = bload2(syR, sxo + 16 * ir[r]);
@@ -3038,8 +3068,8 @@ __global__ __launch_bounds__(64 * TW) __attribute__((amdgpu_waves_per_eu(2))) vo
             const double2 T1 = ACC(acc, 0, r);
             tFR_[e] = T1;
             if (fd) {
-                const double2 lap = csub(cadd(csc(rri[r], ACC(acc, 1, r)), ACC(acc, 2, r)), csc((mm * mm) * rr2i[r], T1));
-                FdT_[(size_t)fslot * S + e] = csc(1.0 / Pr, lap);
+                const double2 lap = tsub(tadd(tsc(rri[r], ACC(acc, 1, r)), ACC(acc, 2, r)), tsc((mm * mm) * rr2i[r], T1));
+                FdT_[(size_t)fslot * S + e] = tsc(1.0 / Pr, lap);
             }
             if (last) {   // Assembly_stage_SA: the stage value is the new state
                 tspec_[e] = T1;
@@ -3049,12 +3079,12 @@ __global__ __launch_bounds__(64 * TW) __attribute__((amdgpu_waves_per_eu(2))) vo
             }
             if (m == 0) {
                 // mean flow stage (fourierloop_imexrk.F90:233-273)
-                const double2 v = cadd(y0[r], csc(dt, cadd(Fd[r], Fa[r])));
+                const double2 v = tadd(y0[r], tsc(dt, tadd(Fd[r], Fa[r])));
                 sx_[sxe + N + i] = mk((i == 0 || i == N - 1) ? 0.0 : v.x, 0.0);
                 continue;
             }
             // vorticity stage (fourierloop_imexrk.F90:276-388)
-            const double2 v = cadd(y0[r], csc(dt, cadd(cadd(Fd[r], Fa[r]), Fb[r])));
+            const double2 v = tadd(y0[r], tsc(dt, tadd(tadd(Fd[r], Fa[r]), Fb[r])));
             sx_[sxe + N + i] = csel(i == 0 || i == N - 1, mk(0.0, 0.0), v);
             // this stage's buoyancy; after the last stage it is the buoyancy of
             // the next step's start state (slot 0, read above by this lane)
@@ -3102,10 +3132,10 @@ __global__ __launch_bounds__(64 * TW) __attribute__((amdgpu_waves_per_eu(2))) vo
                 upFR_[e] = V1;
                 if (fd) {
                     // rhs_construct_uphibar_d (rhs_create_imexrk.F90:162-191)
-                    const double2 v = cadd(csub(ACC(acc, 2, r), csc(rr2i[r], V1)), csc(rri[r], ACC(acc, 1, r)));
+                    const double2 v = tadd(tsub(ACC(acc, 2, r), tsc(rr2i[r], V1)), tsc(rri[r], ACC(acc, 1, r)));
                     FdW_[(size_t)fslot * S + e] = mk(v.x, 0.0);
                 }
-                const double2 om = cadd(csc(rri[r], V1), ACC(acc, 1, r));
+                const double2 om = tadd(tsc(rri[r], V1), ACC(acc, 1, r));
                 urFR_[e] = mk(0.0, 0.0);
                 omgFR_[e] = om;
                 if (last) {
@@ -3118,15 +3148,558 @@ __global__ __launch_bounds__(64 * TW) __attribute__((amdgpu_waves_per_eu(2))) vo
             const double2 ps = qp == 3 ? ACC(acc, 3, r) : ACC(acc, 2, r);
             const double2 dps = qp == 3 ? ACC(acc, 4, r) : ACC(acc, 3, r);
             psi_[e] = ps;
-            upFR_[e] = cneg(dps);
-            urFR_[e] = cimr(mm, rri[r], ps);
+            upFR_[e] = tneg(dps);
+            urFR_[e] = timr(mm, rri[r], ps);
             if (fd)   // rhs_construct_vort_d (rhs_create_imexrk.F90:244-289)
                 FdW_[(size_t)fslot * S + e] =
-                    csub(cadd(csc(rri[r], ACC(acc, 1, r)), ACC(acc, 2, r)), csc((mm * mm) * rr2i[r], V1));
+                    tsub(tadd(tsc(rri[r], ACC(acc, 1, r)), ACC(acc, 2, r)), tsc((mm * mm) * rr2i[r], V1));
             if (last) wspec_[e] = V1;
         }
     }
 }
+
+// ------------------------------------------------------------------ whole mode updates
+// Everything a step (or an IMEXRK stage) does between two nonlinear passes is
+// independent from mode to mode.  In a small launch -- one run, a few runs --
+// the five kernels of the column-tile form (right-hand sides, temperature
+// solves, the second right-hand sides, vorticity solves, new fields) are each
+// bound by their launch and their chain of dependent loads on a few workgroups
+// (65 x 128: 9 tiles), so here one workgroup takes one mode of one run through
+// all five, with the vectors between them in LDS.
+//
+// A phase is a list of matrix products, dealt to the wavefronts by 32-row
+// blocks (fu_rows), with the results in LDS, a barrier, and one (row, column)
+// per thread for the reference's operations on them.  A product takes four
+// columns: the real and imaginary parts of two vectors that meet the same
+// operator -- the coefficients of temperature and vorticity, the two fluxes,
+// vorticity and streamfunction -- so that a step reads 6 N^2 entries of the
+// shared operators and 3 N^2 of the mode's own.  The products are
+// v_mfma_f64_4x4x4f64: its four blocks are 16 rows, and lane l holds
+// A(l % 16, l / 16), X(l / 16, l % 4) and the output of row 4 ((l / 4) % 4) +
+// l / 16, column l % 4.  Its outputs are the same ascending fma chains as the
+// 16 x 16 x 4 form's and the operations are the column tiles' on one part at a
+// time (no contraction in either), so the results are bit for bit theirs.
+//
+// In a launch of few modes a workgroup has one; above one mode per CU it has
+// two (P), which share the loads of the shared operators.
+//
+// What bounds it: the operators through the CU's L1 (about 24 cycles per 1 KiB
+// load of four columns' 32 rows, 16 where the columns start on a cache line:
+// the leading dimension LE), the latency of the few loads of a phase, and for
+// m = 0 the sweeps of its temperature, solved in dgetrs' order.  Measured, one
+// run's CNAB2 step (nonlinear pass included), tiles -> here: 33 x 16 46 -> 27
+// us, 65 x 128 70 -> 35, 97 x 256 105 -> 53, 129 x 128 150 -> 53; ARS443:
+// 169 -> 85, 237 -> 119, 382 -> 191, 527 -> 189.
+constexpr int FU_MAXN = 130;        // the m = 0 factor and six vectors within 160 KiB
+constexpr int FU_MAXW = 12;         // wavefronts per workgroup (three per SIMD)
+constexpr int FU_VEC = 8;           // LDS vectors, [row][4]
+constexpr int FU_ZVEC = 6;          // m = 0: vectors before its staged factor
+__host__ __device__ inline int fu_k4(int N) { return 4 * ((N + 3) >> 2); }
+// workgroups per run, of P modes each: m = 0, then the others
+__host__ __device__ inline int fu_groups(int Nm1, int P) { return 1 + (Nm1 - 1 + P - 1) / P; }
+// A thread per (row, column); in a launch of at most one workgroup per CU a
+// wavefront for most 32-row blocks of a phase.
+inline int fu_waves(int N, bool alone)
+{
+    const int w = (4 * N + 63) / 64;
+    return w < 4 ? 4 : (!alone ? w : (N <= 64 ? 8 : FU_MAXW));
+}
+inline size_t fu_lds(int N, int P, bool staged)
+{
+    const size_t vec = 4 * (size_t)fu_k4(N), all = P * FU_VEC * vec, m0 = FU_ZVEC * vec + (size_t)N * N + 192;
+    return sizeof(double) * (staged && m0 > all ? m0 : all);
+}
+
+// Rows 32 rb .. 32 rb + 31 of A x (A column-major with leading dimension ld,
+// rows x ncols) for P vectors x, vs doubles apart in LDS ([k][4], finite from
+// ncols to the next multiple of four): rows below split to ya, the others to
+// yb ([row][4]), of the columns in mask.  A lane loads two adjacent rows (16 B:
+// half the load instructions), which feed two products.
+template <int P>
+__device__ __forceinline__ void fu_rows(const double* A, const int ld, const int rows, const int ncols, const int rb,
+                                        const double* x, double* ya, double* yb, const int split, const int mask,
+                                        const int vs)
+{
+    constexpr int KC = 8;
+    const int lane = threadIdx.x & 63, lk = lane >> 4;
+    const int nk = (ncols + 3) >> 2;
+    const BRes Ar = bres(A, sizeof(double) * (size_t)ld * ncols);
+    const int ao = 8 * (32 * rb + 2 * (lane & 15) + ld * lk), astep = 32 * ld;
+    const LDS_AS double* xl = (const LDS_AS double*)x + 4 * lk + (lane & 3);
+    double2 a0[KC], a1[KC];
+    double y0[P], y1[P];
+    UNROLL for (int j = 0; j < P; ++j) y0[j] = y1[j] = 0.0;
+    auto load = [&](double2 (&a)[KC], int k0) {
+#pragma unroll
+        for (int c = 0; c < KC; ++c) a[c] = bload2(Ar, ao + astep * (k0 + c));
+    };
+    auto mac = [&](const double2 (&a)[KC], int k0) {
+#pragma unroll
+        for (int c = 0; c < KC; ++c) {
+            if (k0 + c < nk) {
+#pragma unroll
+                for (int j = 0; j < P; ++j) {
+                    const double b = xl[16 * (k0 + c) + j * vs];
+                    y0[j] = __builtin_amdgcn_mfma_f64_4x4x4f64(a[c].x, b, y0[j], 0, 0, 0);
+                    y1[j] = __builtin_amdgcn_mfma_f64_4x4x4f64(a[c].y, b, y1[j], 0, 0, 0);
+                }
+            }
+        }
+    };
+    load(a0, 0);
+    for (int k0 = 0; k0 < nk; k0 += 2 * KC) {
+        load(a1, k0 + KC);
+        mac(a0, k0);
+        load(a0, k0 + 2 * KC);
+        mac(a1, k0 + KC);
+    }
+    const int r = 32 * rb + 8 * ((lane >> 2) & 3) + 2 * (lane >> 4), col = lane & 3;
+    if ((mask >> col) & 1) {
+#pragma unroll
+        for (int j = 0; j < P; ++j) {
+            if (r < rows) (r < split ? ya + 4 * r : yb + 4 * (r - split))[col + j * vs] = y0[j];
+            if (r + 1 < rows) (r + 1 < split ? ya + 4 * (r + 1) : yb + 4 * (r + 1 - split))[col + j * vs] = y1[j];
+        }
+    }
+}
+
+// The other part (real <-> imaginary) of this lane's complex value.
+__device__ __forceinline__ double other_part(double v)
+{
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)(b & 0xffffffffll), 0xB1, 0xf, 0xf, true);   // quad_perm 1, 0, 3, 2
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), 0xB1, 0xf, 0xf, true);
+    return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned int)lo);
+}
+
+// The m = 0 temperature system in dgetrs' order (lu_wave_fwd / lu_wave_bwd,
+// wavefront 0 the real, wavefront 1 the imaginary part): right-hand side
+// x[4 i + part], solution to y.  The factor is staged in LDS from the kernel's
+// start in launches of one workgroup per CU, else read from memory.
+__device__ __forceinline__ void fu_m0_stage(const RunDesc& R, const int N, double* stg)
+{
+    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const BRes fr = bres(R.Ti, sizeof(double) * (size_t)N * N);
+    for (int c = wv; 128 * c < N * N; c += (int)blockDim.x / 64) lds_dma(fr, (double2*)(stg + 128 * c), 16 * (64 * c + lane));
+}
+template <int SLOTS, class Col>
+__device__ __forceinline__ void fu_m0(const RunDesc& R, const int N, const double* x, double* y, Col col)
+{
+    const int lane = threadIdx.x & 63, im = (threadIdx.x >> 6) & 1;
+    double v[SLOTS];
+#pragma unroll
+    for (int q = 0; q < SLOTS; ++q) {
+        const int r = lane + 64 * q;
+        v[q] = r < N ? ((const LDS_AS double*)x)[4 * gload(R.pT + r) + im] : 0.0;
+    }
+    lu_solve_wave<SLOTS, 8>(v, col, N);
+#pragma unroll
+    for (int q = 0; q < SLOTS; ++q) {
+        const int r = lane + 64 * q;
+        if (r < N) y[4 * r + im] = v[q];
+    }
+}
+
+// Set-up shared by the two kernels.  The workgroup's modes m0 .. m0 + nmo - 1
+// (m = 0 by itself); this thread's element of each: row i, vector v (0
+// temperature, 1 vorticity or mean flow), part (0 real, 1 imaginary).  EACH
+// goes over the modes; a missing second one repeats the first and stores
+// nothing (in).
+#define EACH _Pragma("unroll") for (int j = 0; j < P; ++j)
+#define FU_SETUP                                                                                        \
+    const int N = sh.N, Nm1 = sh.Nm1, npr = fu_groups(Nm1, P);                                          \
+    int w;                                                                                              \
+    if (!map_work(nrun * npr, w)) return;                                                               \
+    const int ri = w / npr, pr = w - ri * npr;                                                          \
+    const RunDesc& R = runs[ri];                                                                        \
+    const int tid = threadIdx.x, T = blockDim.x, NW = T >> 6, col = tid & 3;                            \
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);                                            \
+    const bool zero = pr == 0;                                                                          \
+    const int m0 = zero ? 0 : P * (pr - 1) + 1, nmo = zero || m0 + 1 >= Nm1 ? 1 : P;                    \
+    const int v = (tid >> 1) & 1, part = tid & 1, i = tid >> 2;                                         \
+    const bool wall = i == 0 || i == N - 1;                                                             \
+    const double sg = part ? 1.0 : -1.0;                                                                \
+    const size_t S = (size_t)Nm1 * N;                                                                   \
+    const int K4 = fu_k4(N), nrb = (N + 31) >> 5, VS = FU_VEC * 4 * K4;                                 \
+    bool in[P];                                                                                         \
+    double mm[P];                                                                                       \
+    size_t e_[P];   /* this thread's place in a field */                                                \
+    EACH {                                                                                              \
+        const int m = j < nmo ? m0 + j : m0;                                                            \
+        in[j] = i < N && j < nmo;                                                                       \
+        mm[j] = (double)m;                                                                              \
+        e_[j] = m + (size_t)Nm1 * (i < N ? i : 0);                                                      \
+    }                                                                                                   \
+    extern __shared__ double2 stg_[];                                                                   \
+    auto V = [&](int k, int j = 0) { return (double*)stg_ + k * 4 * K4 + j * VS; };                     \
+    /* the modes' columns of fields a and b into vector k */                                            \
+    auto fill = [&](int k, const double2* a, const double2* b) {                                        \
+        for (int j = 0; j < nmo; ++j) for (int e = tid; e < 2 * K4; e += T) {                           \
+            const int r = e >> 1;                                                                       \
+            const double2 z = r < N ? gload((e & 1 ? b : a) + m0 + j + (size_t)Nm1 * r) : mk(0.0, 0.0); \
+            lstore((double2*)(V(k, j) + 2 * e), z);                                                     \
+        }                                                                                               \
+    };                                                                                                  \
+    /* rows N.. of a vector stay zero */                                                                \
+    auto pad = [&](int k) {                                                                             \
+        if (tid < 4 * (K4 - N)) for (int j = 0; j < nmo; ++j) V(k, j)[4 * N + tid] = 0.0;               \
+    };                                                                                                  \
+    /* nq products, hexadecimal digits from the lowest: operator (0 E0, 1 E1, 2 E2, 4 G: as they lie in */ \
+    /* memory), vector, result */                                                                       \
+    auto products = [&](int nq, unsigned ops, unsigned xs, unsigned ys) {                               \
+        for (int t = wv; t < nq * nrb; t += NW) {                                                       \
+            const int q = t % nq, d = 4 * q;                                                            \
+            const double* const A = sh.E0 + (size_t)sh.LE * N * ((ops >> d) & 15);                      \
+            const double* const x = V((int)(xs >> d) & 15);                                             \
+            double* const y = V((int)(ys >> d) & 15);                                                   \
+            if (P == 1 || nmo == 1) fu_rows<1>(A, sh.LE, N, N, t / nq, x, y, y, N, 15, 0);              \
+            else fu_rows<P>(A, sh.LE, N, N, t / nq, x, y, y, N, 15, VS);                                \
+        }                                                                                               \
+    };                                                                                                  \
+    /* this thread's element of a vector, and of a field */                                             \
+    auto at = [&](int k, int j) { return in[j] ? V(k, j)[4 * i + col] : 0.0; };                         \
+    auto get = [&](const double2* f, int j, size_t slot = 0) { return gload((const double*)(f + slot * S + e_[j]) + part); }; \
+    auto put = [&](double2* f, int j, size_t slot, double z) { gstore((double*)(f + slot * S + e_[j]) + part, z); }; \
+    const double rri = gload(sh.rr + (i < N ? i : 0)), rr2i = gload(sh.rr2 + (i < N ? i : 0));          \
+    /* i m / r z from the other part of z */                                                            \
+    auto imr = [&](int j, double zo) { return sg * ((mm[j] * rri) * zo); }
+
+// LDS vectors: coefficients (temperature, vorticity); fluxes, then the
+// temperature's solution (m = 0: with the mean flow's); right-hand sides;
+// three products; the temperature's values; (vorticity, streamfunction).
+enum FuVec : int { FV_C = 0, FV_Y = 1, FV_R = 2, FV_P1 = 3, FV_P2 = 4, FV_P3 = 5, FV_T = 6, FV_W = 7 };
+
+// The temperature solves (m >= 1): FV_R's first vector -> FV_Y's.
+#define FU_SOLVE_T                                                                                      \
+    do {                                                                                                \
+        for (int t = wv; t < nmo * nrb; t += NW) {                                                      \
+            const int j = t >= nrb;                                                                     \
+            fu_rows<1>(R.Ti + (size_t)(m0 + j) * N * N, N, N, N, t - j * nrb, V(FV_R, j), V(FV_Y, j), V(FV_Y, j), N, 3, 0); \
+        }                                                                                               \
+        __syncthreads();                                                                                \
+    } while (0)
+
+// The vorticity-streamfunction solves (m >= 1) of FV_R's first vector, interior
+// row i at i - 1, zeros behind them -> FV_W.
+#define FU_SOLVE_F                                                                                      \
+    do {                                                                                                \
+        if (tid < 4 * (K4 - N + 2)) for (int j = 0; j < nmo; ++j) V(FV_R, j)[4 * (N - 2) + tid] = 0.0;  \
+        pad(FV_W);                                                                                      \
+        __syncthreads();                                                                                \
+        const int nfb = (2 * N + 31) >> 5;                                                              \
+        for (int t = wv; t < nmo * nfb; t += NW) {                                                      \
+            const int j = t >= nfb;                                                                     \
+            fu_rows<1>(R.Fi + (size_t)(m0 + j - 1) * 2 * N * (N - 2), 2 * N, 2 * N, N - 2, t - j * nfb, V(FV_R, j), \
+                       V(FV_W, j) + 2, V(FV_W, j), N, 3, 0);                                            \
+        }                                                                                               \
+        __syncthreads();                                                                                \
+    } while (0)
+
+// m = 0: the temperature's sweeps on wavefronts 0 and 1 beside the mean flow's
+// solve (FV_R's second vector) on the others -> FV_Y.
+#define FU_ZERO                                                                                         \
+    do {                                                                                                \
+        if (staged) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                                    \
+        __syncthreads();                                                                                \
+        if (wv < 2) {                                                                                   \
+            const int lane = tid & 63;                                                                  \
+            if (staged) {                                                                               \
+                const LDS_AS double* fl = (const LDS_AS double*)V(FU_ZVEC);                             \
+                auto cl = [fl, lane, N](int p, int q) { return fl[lane + 64 * p + N * q]; };            \
+                if (N <= 64) fu_m0<1>(R, N, V(FV_R), V(FV_Y), cl);                                      \
+                else if (N <= 128) fu_m0<2>(R, N, V(FV_R), V(FV_Y), cl);                                \
+                else fu_m0<3>(R, N, V(FV_R), V(FV_Y), cl);                                              \
+            } else {                                                                                    \
+                const BRes fr = bres(R.Ti, sizeof(double) * (size_t)N * N);                             \
+                auto cg = [fr, lane, N](int p, int q) { return bload(fr, 8 * (lane + 64 * p + N * q)); }; \
+                if (N <= 128) fu_m0<2>(R, N, V(FV_R), V(FV_Y), cg);                                     \
+                else fu_m0<3>(R, N, V(FV_R), V(FV_Y), cg);                                              \
+            }                                                                                           \
+        } else {                                                                                        \
+            for (int t = wv - 2; t < nrb; t += NW - 2) fu_rows<1>(R.Ui, N, N, N, t, V(FV_R), V(FV_Y), V(FV_Y), N, 12, 0); \
+        }                                                                                               \
+        __syncthreads();                                                                                \
+    } while (0)
+
+// One IMEX step of the workgroup's modes: k_imex_pre, the temperature solve,
+// k_imex_mid, the vorticity solve, k_imex_post.
+template <int P>
+__global__ __launch_bounds__(64 * FU_MAXW) void k_imex_modes(const RunDesc* __restrict__ runs, const Shape sh,
+                                                             const int nrun, const int staged)
+{
+    FU_SETUP;
+    const int L = R.L;
+    const int head = (R.head + 1) % L;
+    auto slot = [&](int o) { return (size_t)((head - o + L) % L); };
+    const double dt = R.dt, Pr = R.Pr, raPr = R.Ra / Pr;
+    const bool cn = (R.imp == IMP_CN);
+    const int ni = cn ? 1 : R.n_imp, ne = R.n_exp;
+    double2 *const tFR = R.tFR, *const omgFR = R.omgFR, *const upFR = R.upFR, *const urFR = R.urFR, *const psi = R.psi;
+    double2 *const tspec = R.tspec, *const wspec = R.wspec, *const TFC = R.TFC;
+    // the histories of this thread's equation; the mean flow's are vectors of N
+    const bool ub = zero && v == 1;
+    double2 *const hi = ub ? (double2*)R.hiU : (v ? (double2*)R.hiW : (double2*)R.hiT);
+    double2 *const he = ub ? (double2*)R.heU : (v ? (double2*)R.heW : (double2*)R.heT);
+    const size_t hs = ub ? (size_t)N : S;
+    auto hp = [&](int j) { return ub ? (size_t)(i < N ? i : 0) : e_[j]; };
+    auto hget = [&](const double2* f, int o, int j) { return gload((const double*)(f + slot(o) * hs + hp(j)) + part); };
+    auto hput = [&](double2* f, int j, double z) { gstore((double*)(f + slot(0) * hs + hp(j)) + part, z); };
+    if (zero && staged) fu_m0_stage(R, N, V(FU_ZVEC));
+    fill(FV_C, tspec, wspec);
+    fill(FV_Y, R.urT, R.urW);
+    pad(FV_R);
+    // this thread's inputs: temperature, vorticity or mean flow; u_phi's product (its other part)
+    double x[P], up[P], h[P][MAXH], e[P][MAXH];
+    const double uw = gload((const double*)R.urw + (i < N ? i : 0));
+    EACH {
+        x[j] = get(v ? (zero ? upFR : omgFR) : tFR, j);
+        up[j] = other_part(get(v ? R.upW : R.upT, j));
+        UNROLL for (int o = 1; o < MAXH; ++o) {
+            if (o < ni) h[j][o] = hget(hi, o, j);
+            if (o < ne) e[j][o] = hget(he, o, j);
+        }
+    }
+    // sums over the histories, z the implicit part's first term, n0 the explicit one's
+    auto history = [&](int j, double z, double n0) {
+        UNROLL for (int o = 1; o < MAXH; ++o)
+            if (o < ni) z = z + R.wi[o] * h[j][o];
+        z = z - dt * (R.we[0] * n0);
+        UNROLL for (int o = 1; o < MAXH; ++o)
+            if (o < ne) z = z - dt * (R.we[o] * e[j][o]);
+        return z;
+    };
+    __syncthreads();
+    double ur[P], d1[P], d2[P], nl[P];
+    EACH ur[j] = at(FV_Y, j);
+    products(3, 0x421, 0x100, 0x543);   // d/dr, d2/dr2 of both coefficient vectors; both flux derivatives
+    __syncthreads();
+    // ---- rhs_construct_temp; for m = 0 rhs_construct_uphi_bar
+    EACH {
+        d1[j] = at(FV_P1, j), d2[j] = at(FV_P2, j);
+        // the explicit term: advection, or <u_r omega> for the mean flow
+        nl[j] = ub ? (part ? 0.0 : uw) : (imr(j, up[j]) + at(FV_P3, j)) + rri * ur[j];
+        if (in[j]) {
+            hput(hi, j, x[j]);
+            hput(he, j, nl[j]);
+        }
+        if (v == 0 || zero) {
+            double r;
+            if (cn) {
+                // (1 - w) dt, and 1 / Pr for the temperature
+                const double c = v ? (1.0 - R.wi[0]) * dt : ((1.0 - R.wi[0]) * dt) * (1.0 / Pr);
+                const double lap = v ? (d2[j] - rr2i * x[j]) + rri * d1[j]
+                                     : (rri * d1[j] + d2[j]) - ((mm[j] * mm[j]) * rr2i) * x[j];
+                r = x[j] + c * lap;
+            } else {
+                r = R.wi[0] * x[j];
+            }
+            r = history(j, r, nl[j]);
+            if (wall) r = i == 0 && zero && col == 0 ? 1.0 : 0.0;
+            if (ub && part) r = 0.0;
+            if (in[j]) V(FV_R, j)[4 * i + col] = r;
+        }
+    }
+    if (zero) {
+        FU_ZERO;
+        products(2, 0x10, 0x11, 0x43);
+        __syncthreads();
+        if (in[0]) {
+            const double c = at(FV_Y, 0), z = at(FV_P1, 0);
+            put(v ? wspec : tspec, 0, 0, c);   // upFC(1,:); the temperature's coefficients
+            put(v ? upFR : tFR, 0, 0, z);
+            if (v) {
+                put(urFR, 0, 0, 0.0);
+                put(omgFR, 0, 0, rri * z + at(FV_P2, 0));
+            } else {
+                gstore((double*)(TFC + i) + part, c);
+            }
+        }
+        return;
+    }
+    __syncthreads();
+    FU_SOLVE_T;
+    // ---- the new temperature; rhs_construct_vort
+    products(1, 0x0, 0x1, 0x6);
+    __syncthreads();
+    EACH {
+        // the new and the old temperature's other part, for the vorticity threads
+        const double To = in[j] ? V(FV_T, j)[4 * i + (part ^ 1)] : 0.0;
+        const int lane = tid & 63;
+        const double xo = __shfl(x[j], (lane & ~3) | (part ^ 1));
+        if (v == 0) {
+            if (in[j]) {
+                put(tspec, j, 0, at(FV_Y, j));
+                put(tFR, j, 0, at(FV_T, j));
+            }
+        } else {
+            const double bT = imr(j, To);
+            double r;
+            if (cn) {
+                const double lap = (rri * d1[j] + d2[j]) - ((mm[j] * mm[j]) * rr2i) * x[j];
+                r = (x[j] + ((1.0 - R.wi[0]) * dt) * lap) - ((raPr * dt) * 0.5) * (bT + imr(j, xo));
+            } else {
+                r = R.wi[0] * x[j];
+            }
+            r = history(j, r, nl[j]);
+            if (!cn) r = r + (dt * R.wl) * ((-raPr) * bT);
+            if (in[j] && !wall) V(FV_R, j)[4 * (i - 1) + part] = r;
+        }
+    }
+    FU_SOLVE_F;
+    // ---- the new fields
+    products(2, 0x10, 0x77, 0x43);
+    __syncthreads();
+    EACH {
+        const double z = at(FV_P1, j), zo = other_part(z);
+        if (in[j]) {
+            if (v == 0) {
+                put(wspec, j, 0, at(FV_W, j));
+                put(omgFR, j, 0, z);
+            } else {
+                put(psi, j, 0, z);
+                put(upFR, j, 0, -at(FV_P2, j));
+                put(urFR, j, 0, imr(j, zo));
+            }
+        }
+    }
+}
+
+// One IMEXRK stage (1 <= s < S) of the workgroup's modes: k_rk_pre, the
+// temperature solve, k_rk_mid, the vorticity solve, k_rk_post.
+template <int P>
+__global__ __launch_bounds__(64 * FU_MAXW) void k_rk_modes(const RunDesc* __restrict__ runs, const Shape sh,
+                                                           const int nrun, const int staged, const int s)
+{
+    FU_SETUP;
+    const bool last = (s == R.S - 1) && R.sa != 0;
+    const double dt = R.dt, Pr = R.Pr, raPr = R.Ra / R.Pr;
+    const double* aD = R.aD + s * MAXS;
+    const double* aA = R.aA + s * MAXS;
+    const bool fa_prev = R.fa_col[s - 1] != 0;
+    const int fslot = last ? 0 : s;
+    const bool fd = R.need_fd[fslot] != 0, bimp = R.buo_imp != 0;
+    const bool ub = zero && v == 1;
+    double2 *const tFR = R.tFR, *const omgFR = R.omgFR, *const upFR = R.upFR, *const urFR = R.urFR, *const psi = R.psi;
+    double2 *const tspec = R.tspec, *const wspec = R.wspec, *const TFC = R.TFC, *const ubar = R.ubar;
+    double2 *const FaX = v ? (double2*)R.FaW : (double2*)R.FaT, *const FdX = v ? (double2*)R.FdW : (double2*)R.FdT;
+    double2 *const FdT = R.FdT, *const FdW = R.FdW, *const Fb = R.Fb;
+    if (zero && staged) fu_m0_stage(R, N, V(FU_ZVEC));
+    if (fa_prev) fill(FV_Y, R.urT, R.urW);
+    else pad(FV_Y);
+    pad(FV_R);
+    // this thread's inputs, its terms of the stages before
+    double y0[P], up[P], Fd[P], Fa[P], Fbs[P];
+    const int nfa = fa_prev ? s - 1 : s;   // explicit terms read back: all but those formed here
+    const bool buo = v == 1 && !zero;
+    const double uw = fa_prev ? gload((const double*)R.urw + (i < N ? i : 0)) : 0.0;
+    EACH {
+        y0[j] = ub ? gload((const double*)(ubar + (i < N ? i : 0)) + part) : get(v ? wspec : tspec, j);
+        up[j] = fa_prev ? other_part(get(v ? R.upW : R.upT, j)) : 0.0;
+        Fd[j] = Fa[j] = Fbs[j] = 0.0;
+        double xd[MAXS], xa[MAXS], xb[MAXS];
+        UNROLL for (int k = 0; k < MAXS - 1; ++k) {
+            if (k < s) {
+                xd[k] = get(FdX, j, (size_t)k);
+                xb[k] = buo ? get(Fb, j, (size_t)k) : 0.0;
+            }
+            if (k < nfa) xa[k] = get(FaX, j, (size_t)k);
+        }
+        UNROLL for (int k = 0; k < MAXS - 1; ++k) {
+            if (k < s) {
+                Fd[j] = Fd[j] + aD[k] * xd[k];
+                Fbs[j] = Fbs[j] + (bimp ? aD[k] : aA[k]) * xb[k];
+            }
+            if (k < nfa) Fa[j] = Fa[j] + aA[k] * xa[k];
+        }
+    }
+    __syncthreads();
+    // ---- the explicit terms of stage s - 1; the temperature stage right-hand
+    // side and, for m = 0, the mean flow's (fourierloop_imexrk.F90:233-273)
+    if (fa_prev) {
+        double ur[P];
+        EACH ur[j] = at(FV_Y, j);
+        products(1, 0x4, 0x1, 0x3);
+        __syncthreads();
+        EACH {
+            const double fa = ub ? (part ? 0.0 : -uw) : -((imr(j, up[j]) + at(FV_P1, j)) + rri * ur[j]);
+            Fa[j] = Fa[j] + aA[s - 1] * fa;
+            if (in[j]) put(FaX, j, (size_t)(s - 1), fa);
+        }
+    }
+    EACH if (in[j] && (v == 0 || zero)) {
+        double r = y0[j] + dt * (Fd[j] + Fa[j]);
+        if (wall) r = i == 0 && zero && col == 0 ? 1.0 : 0.0;
+        if (ub && part) r = 0.0;
+        V(FV_R, j)[4 * i + col] = r;
+    }
+    if (zero) {
+        FU_ZERO;
+        if (fd) products(3, 0x210, 0x111, 0x543);
+        else products(2, 0x10, 0x11, 0x43);
+        __syncthreads();
+        if (in[0]) {
+            const double z = at(FV_P1, 0), dz = at(FV_P2, 0), om = rri * z + dz;
+            put(v ? upFR : tFR, 0, 0, z);
+            if (fd) {
+                const double t = v ? (at(FV_P3, 0) - rr2i * z) + rri * dz
+                                   : (1.0 / Pr) * ((rri * dz + at(FV_P3, 0)) - ((mm[0] * mm[0]) * rr2i) * z);
+                put(FdX, 0, (size_t)fslot, ub && part ? 0.0 : t);
+            }
+            if (v) {
+                put(urFR, 0, 0, 0.0);
+                put(omgFR, 0, 0, om);
+            }
+            if (last) {
+                put(v ? wspec : tspec, 0, 0, v ? om : z);
+                gstore((double*)((v ? ubar : TFC) + i) + part, v ? z : at(FV_Y, 0));
+            }
+        }
+        return;
+    }
+    __syncthreads();
+    FU_SOLVE_T;
+    // ---- the stage temperature and its diffusion term; the vorticity stage right-hand side
+    if (fd) products(3, 0x210, 0x111, 0x543);
+    else products(1, 0x0, 0x1, 0x3);
+    __syncthreads();
+    EACH {
+        if (v == 0) {
+            if (in[j]) {
+                const double T1 = at(FV_P1, j);
+                put(tFR, j, 0, T1);
+                if (fd) put(FdT, j, (size_t)fslot, (1.0 / Pr) * ((rri * at(FV_P2, j) + at(FV_P3, j)) - ((mm[j] * mm[j]) * rr2i) * T1));
+                if (last) put(tspec, j, 0, T1);   // Assembly_stage_SA: the stage value is the new state
+            }
+        } else if (in[j]) {
+            const double bu = (-raPr) * imr(j, V(FV_P1, j)[4 * i + (part ^ 1)]);   // buoyancy of this stage
+            if (bimp) Fbs[j] = Fbs[j] + aD[s] * bu;
+            const double r = y0[j] + dt * ((Fd[j] + Fa[j]) + Fbs[j]);
+            put(Fb, j, (size_t)fslot, bu);
+            if (!wall) V(FV_R, j)[4 * (i - 1) + part] = r;
+        }
+    }
+    FU_SOLVE_F;
+    // ---- the stage vorticity, streamfunction and velocities and their diffusion terms
+    if (fd) products(3, 0x210, 0x777, 0x543);
+    else products(2, 0x10, 0x77, 0x43);
+    __syncthreads();
+    EACH {
+        const double z = at(FV_P1, j), zo = other_part(z);
+        if (in[j]) {
+            if (v == 0) {
+                put(omgFR, j, 0, z);
+                if (fd) put(FdW, j, (size_t)fslot, (rri * at(FV_P2, j) + at(FV_P3, j)) - ((mm[j] * mm[j]) * rr2i) * z);
+                if (last) put(wspec, j, 0, z);
+            } else {
+                put(psi, j, 0, z);
+                put(upFR, j, 0, -at(FV_P2, j));
+                put(urFR, j, 0, imr(j, zo));
+            }
+        }
+    }
+}
+
+#pragma clang fp contract(fast)
 
 // ------------------------------------------------------------------ matrices
 // mat_build / mat_build_IRK / mat_build_uphibar (mat_assembly.F90:68-413), one
@@ -4211,6 +4784,7 @@ int kernels_init()
 #undef SETLDS4
     SETLDS((k_lu<512, 1>)) SETLDS((k_lu<512, 3>)) SETLDS((k_lu_small<1, 4>)) SETLDS((k_lu_small<2, 4>))
     SETLDS((k_lu_small<3, 8>)) SETLDS((k_lu_small<4, 8>)) SETLDS((k_lu_small<5, 8>)) SETLDS(k_solve<0>) SETLDS(k_solve<1>) SETLDS(k_m0)
+    SETLDS(k_imex_modes<1>) SETLDS(k_imex_modes<2>) SETLDS(k_rk_modes<1>) SETLDS(k_rk_modes<2>)
 #define SETTILE(k) SETLDS((k<4, true, false>)) SETLDS((k<8, true, false>))
 #define SETTILEPF(k) SETTILE(k) SETLDS((k<4, true, true>)) SETLDS((k<8, true, true>)) \
     SETLDS((k<4, false, true>)) SETLDS((k<8, false, true>))
@@ -4298,6 +4872,50 @@ size_t tile_stage_bytes(const Shape& sh, int nx)
         else TILE_LAUNCH_TW(KERNEL, 8, NPF, ##__VA_ARGS__);                                                      \
     } while (0)
 
+
+// Whole mode updates instead of the column tiles: modes per workgroup, 0 for
+// the tiles.  Up to one mode per CU (256) a workgroup takes one: 65 x 128, 129
+// modes, 35 us a step against 39 with two.  Above that two: 97 x 256, 257
+// modes, 53 us against 64.  The tiles read the shared operators once per 16
+// modes, so they keep the launches that fill the chip several times.  The line
+// (measured, steps of the tiles / of the mode kernels):
+//   - a workgroup per CU: 1.4 - 2.4 up to 256 workgroups at every N; at 260,
+//     four runs of 65 x 128, 0.95;
+//   - N <= 64: three workgroups of four wavefronts share a CU: 1.2 at 392
+//     (49 x 96), 1.03 at 520 (64 x 128), 1.4 at 528 (17 x 64); 1.0 at 784;
+//   - one run, whose column tiles are few: 1.1 - 1.4 at 385 (65, 97, 129 x
+//     768), but 0.97 at 513 (65 x 1024).
+static int fu_modes(const Shape& sh, int nrun)
+{
+    if (sh.N > FU_MAXN) return 0;
+    if (nrun * sh.Nm1 <= 256) return 1;
+    const int G = nrun * fu_groups(sh.Nm1, 2);
+    return G <= (sh.N <= 64 ? 512 : (nrun == 1 ? 400 : 256)) ? 2 : 0;
+}
+
+bool mode_fused(const Shape& sh, int nrun) { return fu_modes(sh, nrun) != 0; }
+
+// Launch K<1> or K<2>.
+template <class K1, class K2, class... A>
+static void fu_launch(K1 k1, K2 k2, const RunDesc* runs, int nrun, const Shape& sh, hipStream_t st, A... a)
+{
+    const int P = fu_modes(sh, nrun), G = nrun * fu_groups(sh.Nm1, P);
+    const bool one = G <= 256;   // alone on its CU: more wavefronts, m = 0's factor in LDS
+    const dim3 grid(padded_grid(G)), block(64 * fu_waves(sh.N, one));
+    const size_t lds = fu_lds(sh.N, P, one);
+    if (P == 1) hipLaunchKernelGGL(k1, grid, block, lds, st, runs, sh, nrun, (int)one, a...);
+    else hipLaunchKernelGGL(k2, grid, block, lds, st, runs, sh, nrun, (int)one, a...);
+}
+
+void launch_imex_modes(const RunDesc* runs, int nrun, const Shape& sh, hipStream_t st)
+{
+    fu_launch(k_imex_modes<1>, k_imex_modes<2>, runs, nrun, sh, st);
+}
+
+void launch_rk_modes(const RunDesc* runs, int nrun, const Shape& sh, int s, hipStream_t st)
+{
+    fu_launch(k_rk_modes<1>, k_rk_modes<2>, runs, nrun, sh, st, s);
+}
 
 void launch_imex_prep(const RunDesc* runs, int nrun, const Shape& sh, hipStream_t st)
 {
