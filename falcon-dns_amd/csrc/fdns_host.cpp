@@ -1656,13 +1656,23 @@ void stage_launches(const RunDesc* dev, int n, const Shape& sh, const SolveSched
 // The launch sequence of one time step of one group of runs that share a
 // shape, a scheme structure and a solver mode.  first: this is the group's
 // first step.
-void step_launches(const RunDesc* dev, int n, const Shape& sh, const Scheme& sc, const SolveSched& ss, bool first,
+void step_launches(RunDesc* dev, int n, const Shape& sh, const Scheme& sc, const SolveSched& ss, bool first,
                    bool restart, bool record, hipStream_t st, KTimer* kt = nullptr, bool keep = false,
                    const Side* sd = nullptr)
 {
+    // The counters go on, and the temperature of the step's last pass is kept
+    // for the power budget (IMEX: with upFR_prev of the step's start), in that
+    // pass's launch; on their own where the step has none.
+    const int up = sc.kind == SK_IMEX ? 1 : 0;
+    const int with = NL_ADVANCE | (keep ? NL_KEEP | (up ? NL_KEEP_UP : 0) : 0);
+    auto nonlin = [&](bool last) { TIMED(kt, FDNS_KC_NONLIN, st, launch_nonlin(dev, n, sh, st, last ? with : 0)); };
+    auto no_pass = [&](bool keeps) {
+        if (keep && keeps) TIMED(kt, FDNS_KC_OTHER, st, launch_keep(dev, n, sh, up, st));
+        TIMED(kt, FDNS_KC_OTHER, st, launch_advance(dev, n, st));
+    };
     if (sc.kind == SK_IMEX) {
-        if (keep) TIMED(kt, FDNS_KC_OTHER, st, launch_keep(dev, n, sh, 1, st));   // tt, upFR_prev of the step's start
-        if (!first || restart) TIMED(kt, FDNS_KC_NONLIN, st, launch_nonlin(dev, n, sh, st));   // steptime.F90:202
+        if (!first || restart) nonlin(true);   // steptime.F90:202
+        else no_pass(true);
         imex_launches(dev, n, sh, ss, first ? 1 : 0, st, kt, sd);
     } else if (sc.kind == SK_RK) {
         // timeloop_rk (steptime_rk.F90:108-133): stage values from stage 2,
@@ -1670,8 +1680,8 @@ void step_launches(const RunDesc* dev, int n, const Shape& sh, const Scheme& sc,
         // the stage's right-hand sides; Assembly_stage ends the step
         for (int s = 0; s < sc.S; ++s) {
             if (s > 0) TIMED(kt, FDNS_KC_OTHER, st, launch_rkx_update(dev, n, sh, s, st));
-            if (keep && s == sc.S - 1) TIMED(kt, FDNS_KC_OTHER, st, launch_keep(dev, n, sh, 0, st));
-            if (!first || s > 0 || restart) TIMED(kt, FDNS_KC_NONLIN, st, launch_nonlin(dev, n, sh, st));
+            if (!first || s > 0 || restart) nonlin(s == sc.S - 1);
+            else if (s == sc.S - 1) no_pass(true);
             TIMED(kt, FDNS_KC_OTHER, st, launch_rkx_rhs(dev, n, sh, s, st));
         }
         TIMED(kt, FDNS_KC_OTHER, st, launch_rkx_update(dev, n, sh, sc.S, st));
@@ -1682,30 +1692,27 @@ void step_launches(const RunDesc* dev, int n, const Shape& sh, const Scheme& sc,
         // the prologue on the first step), a nonlinear pass follows the last
         // stage when its column is used, and Assembly_stage ends the step.
         if (!sc.sa && !first) TIMED(kt, FDNS_KC_OTHER, st, launch_rk_init(dev, n, sh, st));
-        // the step's passes: stage 0's, then after stage s; the temperature of
-        // the last one is kept for the power budget
+        // the step's passes: stage 0's, then after stage s
         auto pass = [&](int s) {
             return s == 0 ? ((!first || restart) && sc.nl_col[0]) : ((s < sc.S - 1 || !sc.sa) && sc.nl_col[s]);
         };
         int last = -1;
         for (int s = 0; s < sc.S; ++s)
             if (pass(s)) last = s;
-        if (keep && last == 0) TIMED(kt, FDNS_KC_OTHER, st, launch_keep(dev, n, sh, 0, st));
-        if (pass(0)) TIMED(kt, FDNS_KC_NONLIN, st, launch_nonlin(dev, n, sh, st));
+        if (last < 0) no_pass(false);
+        if (pass(0)) nonlin(last == 0);
         for (int s = 1; s < sc.S; ++s) {
             stage_launches(dev, n, sh, ss, s, st, kt, sd);
-            if (keep && last == s) TIMED(kt, FDNS_KC_OTHER, st, launch_keep(dev, n, sh, 0, st));
-            if (pass(s)) TIMED(kt, FDNS_KC_NONLIN, st, launch_nonlin(dev, n, sh, st));
+            if (pass(s)) nonlin(last == s);
         }
         if (!sc.sa) TIMED(kt, FDNS_KC_OTHER, st, launch_rk_asm(dev, n, sh, st));
     }
-    TIMED(kt, FDNS_KC_OTHER, st, launch_advance((RunDesc*)dev, n, st));
     if (record) TIMED(kt, FDNS_KC_OTHER, st, launch_diag(dev, n, sh, 1, nullptr, st));
 }
 
 // Work that precedes the first step: the restart history start-up (IMEX) or
 // the stage-0 terms of the initial state (IMEXRK).
-void prologue_launches(const RunDesc* dev, int n, const Shape& sh, const Scheme& sc, bool restart, hipStream_t st)
+void prologue_launches(RunDesc* dev, int n, const Shape& sh, const Scheme& sc, bool restart, hipStream_t st)
 {
     if (sc.kind == SK_IMEX) {
         if (restart) {
@@ -1984,8 +1991,8 @@ int vardt_steps(fdns_run* R, int nsteps)
             if ((rc = rebind_ops(R, wl, R->dta[0]))) return rc;
         if ((rc = upload_desc(R))) return rc;
         if (imex) {
-            imex_launches(R->dev, 1, sh, R->solo, first ? 1 : 0, R->st, nullptr);
             launch_advance(R->dev, 1, R->st);
+            imex_launches(R->dev, 1, sh, R->solo, first ? 1 : 0, R->st, nullptr);
             if (rec) launch_diag(R->dev, 1, sh, 1, nullptr, R->st);
         } else {
             step_launches(R->dev, 1, sh, R->sc, R->solo, first, restart, rec, R->st, nullptr, R->h.keep != 0);

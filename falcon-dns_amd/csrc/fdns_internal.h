@@ -175,7 +175,7 @@ struct RunDesc {
     // physics and scheme
     double Ra, Pr, dt;
     int kind, imp, n_imp, n_exp, L;  // L = history ring length
-    int head;                         // slot written by the previous IMEX step
+    int head;                         // newest slot: that of the IMEX step under way or, between steps, the last one's
     int hist_ready;                   // IMEX restart: histories already filled
                                       // from checkpoint states (no constant fill)
     int buo_imp;
@@ -220,7 +220,12 @@ struct SolvePlan {
 };
 
 // ---- kernel launchers (fdns_kernels.hip) ----
-void launch_nonlin(const RunDesc* runs, int nrun, const Shape& sh, hipStream_t st);
+// With the pass, in one launch: the runs' step counter, time and (IMEX) head
+// go on by one step (NL_ADVANCE; the IMEX kernels after it take the new head),
+// runs that record keep the pass's temperature (NL_KEEP) and the mean flow at
+// its start (NL_KEEP_UP), as launch_advance and launch_keep do by themselves.
+enum NlFlags : int { NL_ADVANCE = 1, NL_KEEP = 2, NL_KEEP_UP = 4 };
+void launch_nonlin(RunDesc* runs, int nrun, const Shape& sh, hipStream_t st, int flags = 0);
 void launch_forfft(const double* x, double2* f, const Shape& sh, hipStream_t st);
 void launch_copy(const double* a, double* b, size_t n16, hipStream_t st);
 void launch_imex_prep(const RunDesc* runs, int nrun, const Shape& sh, hipStream_t st);
