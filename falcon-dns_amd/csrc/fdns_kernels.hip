@@ -4500,15 +4500,91 @@ __global__ __launch_bounds__(64) void k_inv(const double* __restrict__ LU, const
 }
 
 // ------------------------------------------------------------------ diagnostics
+// The sums over the modes of every level, one wavefront per (run, level): they
+// are nearly all of the diagnostics' bytes, and a wavefront that went over the
+// modes of its levels by itself took 290 (k_diag) and 340 us (k_budget) at
+// 129 x 256, bound by one chain of loads; these take 4.5, and the kernels that
+// integrate the sums 17 and 15.  |z^2| is x^2 + y^2.
+__device__ __forceinline__ double wave_total(double v)
+{
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) v = v + __shfl_xor(v, d);
+    return v;
+}
+
+constexpr int LV_WAVES = 4;   // levels per workgroup
+
+// sy[j] = (sum_m |ur_m^2|, sum_m |up_m^2|) of level j
+__global__ __launch_bounds__(64 * LV_WAVES) void k_level_ke(const RunDesc* __restrict__ runs, const int Nm1, const int N)
+{
+    const RunDesc& R = runs[blockIdx.y];
+    const int lane = threadIdx.x & 63, j = blockIdx.x * LV_WAVES + (threadIdx.x >> 6);
+    if (j >= N) return;
+    const double2 *ur = R.urFR, *up = R.upFR;
+    double a = 0.0, b = 0.0;
+#pragma unroll 4
+    for (int q = lane; q < Nm1; q += 64) {
+        const double2 zr = gload(ur + q + (size_t)Nm1 * j), zp = gload(up + q + (size_t)Nm1 * j);
+        a = a + (zr.x * zr.x + zr.y * zr.y);
+        b = b + (zp.x * zp.x + zp.y * zp.y);
+    }
+    a = wave_total(a);
+    b = wave_total(b);
+    if (lane == 0) gstore((double2*)R.sy + j, mk(a, b));
+}
+
+// The budget's sums of level j (k_budget): sy[S + Nm1 j + 1] = (<u_r tt>,
+// <omega^2>), the Reynolds-stress column of the output, and at the walls
+// sum_m |up_m^2| in out[0], out[1].  sy holds k_budget_dr's derivatives.
+__global__ __launch_bounds__(64 * LV_WAVES) void k_level_budget(const RunDesc* __restrict__ runs, const double* __restrict__ rr,
+                                                                const int Nm1, const int N, double* __restrict__ out)
+{
+    const RunDesc& R = runs[blockIdx.y];
+    const int lane = threadIdx.x & 63, j = blockIdx.x * LV_WAVES + (threadIdx.x >> 6);
+    if (j >= N) return;
+    const size_t S = (size_t)Nm1 * N, at = (size_t)Nm1 * j;
+    const double2 *urF = R.urFR, *upF = R.upFR, *omF = R.omgFR, *tpF = R.tpass, *duF = R.sy;
+    double ut = 0.0, w2 = 0.0, up2 = 0.0, su = 0.0, sd = 0.0;
+#pragma unroll 2
+    for (int q = lane; q < Nm1; q += 64) {
+        const double2 ur = gload(urF + at + q), up = gload(upF + at + q), om = gload(omF + at + q), tp = gload(tpF + at + q),
+                      du = gload(duF + at + q);
+        up2 = up2 + (up.x * up.x + up.y * up.y);
+        if (q == 0) {   // the mean's imaginary parts take part as the complex products have them
+            ut = ut + ur.x * tp.x;
+            w2 = w2 + (om.x * om.x - om.y * om.y);
+            su = su + (ur.x * up.x - ur.y * up.y);
+            sd = sd + (ur.x * du.x - ur.y * du.y);
+        } else {
+            ut = ut + 2.0 * (ur.x * tp.x + ur.y * tp.y);
+            w2 = w2 + 2.0 * (om.x * om.x + om.y * om.y);
+            su = su + 2.0 * (ur.x * up.x + ur.y * up.y);
+            sd = sd + 2.0 * (ur.x * du.x + ur.y * du.y);
+        }
+    }
+    ut = wave_total(ut);
+    w2 = wave_total(w2);
+    up2 = wave_total(up2);
+    su = wave_total(su);
+    sd = wave_total(sd);
+    if (lane != 0) return;
+    double* o = out + (size_t)blockIdx.y * (4 + 3 * (size_t)N);
+    gstore((double2*)R.sy + S + at + 1, mk(ut, w2));
+    o[4 + 3 * j + 1] = -(sd + gload(rr + j) * su);
+    if (j == 0) o[0] = up2;
+    if (j == N - 1) o[1] = up2;
+}
+
 // writeKE_spectral: KE = 2 pi (radInt(sum_m |ur_m^2|) + radInt(sum_m |up_m^2|))
-// and the Nusselt numbers from d/dr of TFC (output.F90:232-265, integ.F90:36-76)
+// and the Nusselt numbers from d/dr of TFC (output.F90:232-265, integ.F90:36-76),
+// from the level sums of k_level_ke
 template <int NT, int MM>
 __global__ __launch_bounds__(NT) void k_diag(RunDesc* __restrict__ runs, const Shape sh0, const int record,
                                              double* __restrict__ out6)
 {
     extern __shared__ double2 smem[];
     const Shape sh = lds_twiddles<NT>(sh0, smem);     // twiddle table: smem[0..M)
-    const int N = sh.N, Nm1 = sh.Nm1;
+    const int N = sh.N;
     RunDesc& R = runs[blockIdx.x];
     double2* buf = smem + sh.M;
     double2* V0 = buf + sh.M + 4 * N;
@@ -4517,14 +4593,8 @@ __global__ __launch_bounds__(NT) void k_diag(RunDesc* __restrict__ runs, const S
     double* red = (double*)(V2 + N);
     const int tid = threadIdx.x;
     for (int j = tid; j < N; j += NT) {
-        double a = 0.0, b = 0.0;
-        for (int i = 0; i < Nm1; ++i) {
-            const double2 zr = R.urFR[i + (size_t)Nm1 * j], zp = R.upFR[i + (size_t)Nm1 * j];
-            const double2 sr = cmul(zr, zr), sp = cmul(zp, zp);
-            a = a + hypot(sr.x, sr.y);
-            b = b + hypot(sp.x, sp.y);
-        }
-        V1[j] = mk(a * sh.rad[j], b * sh.rad[j]);
+        const double2 s = R.sy[j];
+        V1[j] = mk(s.x * sh.rad[j], s.y * sh.rad[j]);
     }
     __syncthreads();
     cheb_fwd<NT, MM>(buf, V0, sh, [&](int i) { return V1[i]; });
@@ -4595,7 +4665,8 @@ __global__ __launch_bounds__(NT) void k_budget_dr(const RunDesc* __restrict__ ru
 }
 
 // The mean-flow energy, power budget and mean-flow balance of
-// writeKE_spectral (output.F90:122-324) for one run per workgroup:
+// writeKE_spectral (output.F90:122-324) for one run per workgroup, from the
+// level sums of k_level_budget:
 // out[0..3] = {2 pi radInt(<u_phi>^2), viscous dissipation (stress free:
 // less the wall terms 8 pi sum_m |up_m^2|), 2 pi Ra/Pr radInt(<u_r tt>), t},
 // out[4 + 3 j + c] the upbalance_ columns of level j.  Azimuthal means by
@@ -4618,39 +4689,17 @@ __global__ __launch_bounds__(NT) void k_budget(const RunDesc* __restrict__ runs,
     const int tid = threadIdx.x;
     const size_t S = (size_t)Nm1 * N;
     double* o = out + (size_t)blockIdx.x * (4 + 3 * (size_t)N);
-    __shared__ double wall_up2[2];
     for (int j = tid; j < N; j += NT) {
-        double ut = 0.0, w2 = 0.0, up2 = 0.0;
-        double2 su = mk(0.0, 0.0), sd = mk(0.0, 0.0);
-        for (int q = 0; q < Nm1; ++q) {
-            const size_t e = (size_t)q + (size_t)Nm1 * (size_t)j;
-            const double2 ur = R.urFR[e], up = R.upFR[e], om = R.omgFR[e], tp = R.tpass[e], du = R.sy[e];
-            const double2 u2 = cmul(up, up);
-            up2 = up2 + hypot(u2.x, u2.y);
-            if (q == 0) {
-                ut = ut + ur.x * tp.x;
-                w2 = w2 + cmul(om, om).x;
-                su = cadd(su, cmul(ur, up));
-                sd = cadd(sd, cmul(ur, du));
-            } else {
-                ut = ut + 2.0 * (ur.x * tp.x + ur.y * tp.y);
-                w2 = w2 + cadd(cmul(om, mk(om.x, -om.y)), cmul(mk(om.x, -om.y), om)).x;
-                su = cadd(su, cadd(cmul(ur, mk(up.x, -up.y)), cmul(mk(ur.x, -ur.y), up)));
-                sd = cadd(sd, cadd(cmul(ur, mk(du.x, -du.y)), cmul(mk(ur.x, -ur.y), du)));
-            }
-        }
+        const double2 lv = R.sy[S + (size_t)Nm1 * j + 1];
+        const double ut = lv.x, w2 = lv.y;
         const double2 u0 = R.upFR[(size_t)Nm1 * j];
         const double ua = u0.x;
         V0[j] = mk((ua * ua) * sh.rad[j], w2 * sh.rad[j]);
         V1[j] = mk(ut * sh.rad[j], 0.0);
-        if (j == 0) wall_up2[0] = up2;
-        if (j == N - 1) wall_up2[1] = up2;
-        const double2 ufa = cadd(sd, csc(rr[j], su));
         const double2 d1 = R.sy[(size_t)Nm1 * j], d2 = R.sy[S + (size_t)Nm1 * j];
         const double2 ud = cadd(csub(d2, csc(rr2[j], u0)), csc(rr[j], d1));
         const double2 u0p = R.up0prev[j];
         o[4 + 3 * j] = (u0.x - u0p.x) / R.dt;
-        o[4 + 3 * j + 1] = -ufa.x;
         o[4 + 3 * j + 2] = ud.x;
     }
     __syncthreads();
@@ -4684,9 +4733,9 @@ __global__ __launch_bounds__(NT) void k_budget(const RunDesc* __restrict__ runs,
     if (tid == 0) {
         const double pi = 3.14159265358979323846;
         const double upbark = sh.fact * red[0], vis1 = sh.fact * red[NT], buo = sh.fact * red[2 * NT];
+        const double up2i = o[0], up2o = o[1];   // at the walls
         o[0] = 2.0 * pi * upbark;
-        o[1] = R.mbc == 1 ? 2.0 * pi * vis1 - (4.0 * pi * 2.0 * wall_up2[1] - 4.0 * pi * 2.0 * wall_up2[0])
-                          : 2.0 * pi * vis1;
+        o[1] = R.mbc == 1 ? 2.0 * pi * vis1 - (4.0 * pi * 2.0 * up2o - 4.0 * pi * 2.0 * up2i) : 2.0 * pi * vis1;
         o[2] = 2.0 * pi * R.Ra / R.Pr * buo;
         o[3] = R.time;
     }
@@ -5091,6 +5140,7 @@ void launch_lu(double* A, int* perm, int n, size_t stride, int nmat, hipStream_t
 
 void launch_diag(const RunDesc* runs, int nrun, const Shape& sh, int record, double* out6, hipStream_t st)
 {
+    hipLaunchKernelGGL(k_level_ke, dim3((sh.N + LV_WAVES - 1) / LV_WAVES, nrun), dim3(64 * LV_WAVES), 0, st, runs, sh.Nm1, sh.N);
     TIER_DISPATCH(sh.M, hipLaunchKernelGGL((k_diag<B_, T_>), dim3(nrun), dim3(B_), diag_lds(sh), st, (RunDesc*)runs, sh, record, out6));
 }
 
@@ -5103,6 +5153,8 @@ void launch_keep(const RunDesc* runs, int nrun, const Shape& sh, int with_up, hi
 void launch_budget(const RunDesc* runs, int nrun, const Shape& sh, double* out, hipStream_t st)
 {
     RADIAL_LAUNCH(k_budget_dr);
+    hipLaunchKernelGGL(k_level_budget, dim3((sh.N + LV_WAVES - 1) / LV_WAVES, nrun), dim3(64 * LV_WAVES), 0, st, runs, sh.rr,
+                       sh.Nm1, sh.N, out);
     TIER_DISPATCH(sh.M, hipLaunchKernelGGL((k_budget<B_, T_>), dim3(nrun), dim3(B_), budget_lds(sh), st, runs, sh, out));
 }
 
