@@ -1257,6 +1257,7 @@ struct fdns_run {
     size_t bytes = 0;
     hipStream_t st = nullptr;
     int kstep = 0;             // host mirror of completed steps
+    bool staged = false;       // counted in g_stage
     bool has_state = false;
     bool in_ens = false;
     hipGraphExec_t gexec = nullptr;
@@ -1458,6 +1459,49 @@ int stage_ops(fdns_run* R, double dt)
     return 0;
 }
 
+// Small transfers of state go through one pinned megabyte: a copy to or from
+// pageable memory costs about 17 us whatever its size, and one from the
+// pinned block 12 for the fields together, which lie one behind the other
+// (tFR, omgFR, upFR, urFR, psi).  33 x 16, 45 kB: 90 -> 20 us for a state;
+// above a megabyte the second copy costs what the first call saves (97 x 256,
+// 2 MB: 142 us direct).  The block exists while there are runs; a thread that finds
+// it in use, or a process that could not pin it, copies directly.
+constexpr size_t STAGE_BYTES = 1 << 20;
+struct Stage {
+    std::mutex mu;
+    char* p = nullptr;
+    int users = 0;
+} g_stage;
+
+void stage_join(fdns_run* R)
+{
+    std::lock_guard<std::mutex> lk(g_stage.mu);
+    if (g_stage.users++ == 0 && hipHostMalloc((void**)&g_stage.p, STAGE_BYTES, hipHostMallocPortable) != hipSuccess) {
+        g_stage.p = nullptr;
+        (void)hipGetLastError();
+    }
+    R->staged = true;
+}
+
+void stage_leave(fdns_run* R)
+{
+    if (!R->staged) return;
+    std::lock_guard<std::mutex> lk(g_stage.mu);
+    if (--g_stage.users == 0 && g_stage.p) {
+        hipHostFree(g_stage.p);
+        g_stage.p = nullptr;
+    }
+    R->staged = false;
+}
+
+// The block for this call, null where it is too small or in use.
+char* stage_take(std::unique_lock<std::mutex>& lk, size_t bytes)
+{
+    if (bytes > STAGE_BYTES) return nullptr;
+    lk = std::unique_lock<std::mutex>(g_stage.mu, std::try_to_lock);
+    return lk.owns_lock() ? g_stage.p : nullptr;
+}
+
 int run_zero_dynamic(fdns_run* R)
 {
     // everything except the factors and constants starts at zero: fields,
@@ -1472,11 +1516,20 @@ int upload_desc(fdns_run* R)
     return 0;
 }
 
-int download_desc(fdns_run* R)
+// The run's counters, and the last pass's velocity maxima into cfl if given.
+int download_desc(fdns_run* R, double* cfl = nullptr)
 {
     RunDesc tmp;
-    HIPCHK(hipMemcpyAsync(&tmp, R->dev, sizeof(RunDesc), hipMemcpyDeviceToHost, R->st));
+    const size_t nc = cfl ? sizeof(double) * 2 * (size_t)R->p.Nr : 0;
+    std::unique_lock<std::mutex> lk;
+    char* stg = stage_take(lk, sizeof(RunDesc) + nc);
+    HIPCHK(hipMemcpyAsync(stg ? stg : (char*)&tmp, R->dev, sizeof(RunDesc), hipMemcpyDeviceToHost, R->st));
+    if (cfl) HIPCHK(hipMemcpyAsync(stg ? stg + sizeof(RunDesc) : (char*)cfl, R->h.cfl.p, nc, hipMemcpyDeviceToHost, R->st));
     HIPCHK(hipStreamSynchronize(R->st));
+    if (stg) {
+        std::memcpy((void*)&tmp, stg, sizeof(RunDesc));
+        if (cfl) std::memcpy(cfl, stg + sizeof(RunDesc), nc);
+    }
     R->h.head = tmp.head; R->h.kstep = tmp.kstep; R->h.time = tmp.time; R->h.nrec = tmp.nrec;
     return 0;
 }
@@ -1966,18 +2019,10 @@ int vardt_steps(fdns_run* R, int nsteps)
         if (!rk && ((imex && (!first || restart)) || (!imex && first && restart) || (!imex && !R->sc.sa && !first)))
             launch_nonlin(R->dev, 1, sh, R->st);
         HIPCHK(hipGetLastError());
-        if (rk) {
-            if (!first) {
-                HIPCHK(hipMemcpyAsync(cfl.data(), R->h.cfl.p, sizeof(double) * 2 * N, hipMemcpyDeviceToHost, R->st));
-                HIPCHK(hipStreamSynchronize(R->st));
-            }
-            new_dt_rk(R, cfl.data(), ks);
-        } else if (!first || restart) {
-            HIPCHK(hipMemcpyAsync(cfl.data(), R->h.cfl.p, sizeof(double) * 2 * N, hipMemcpyDeviceToHost, R->st));
-            HIPCHK(hipStreamSynchronize(R->st));
-            new_dt(R, cfl.data(), ks, !imex);
-        }
-        if ((rc = download_desc(R))) return rc;     // head, kstep, time, records
+        const bool pass = !first || (restart && !rk);
+        if ((rc = download_desc(R, pass ? cfl.data() : nullptr))) return rc;     // head, kstep, time, records
+        if (rk) new_dt_rk(R, cfl.data(), ks);
+        else if (pass) new_dt(R, cfl.data(), ks, !imex);
         RunDesc& h = R->h;
         h.dt = R->dt_new;
         double wl;
@@ -2096,6 +2141,7 @@ int fdns_create(const fdns_params* p, fdns_run** out)
     R->p = *p;
     R->sc = sc;
     if (hipStreamCreateWithFlags(&R->st, hipStreamNonBlocking) != hipSuccess) { delete R; return fail(FDNS_EHIP, "stream"); }
+    stage_join(R);
     if ((rc = R->side.create())) { fdns_destroy(R); return rc; }
     if ((rc = shape_get(p->Nr, p->Nm, p->eta, &R->shape))) { fdns_destroy(R); return rc; }
     double wl = 0.0;
@@ -2237,6 +2283,7 @@ int fdns_destroy(fdns_run* R)
     R->solo.release();
     R->side.destroy();
     if (R->st) hipStreamDestroy(R->st);
+    stage_leave(R);
     delete R;
     return 0;
 }
@@ -2249,10 +2296,17 @@ int fdns_set_state(fdns_run* R, const double* tFR, const double* omgFR, const do
     int rc;
     if ((rc = run_zero_dynamic(R))) return rc;
     RunDesc& h = R->h;
-    HIPCHK(hipMemcpyAsync(h.tFR, tFR, sizeof(double2) * S, hipMemcpyHostToDevice, R->st));
-    HIPCHK(hipMemcpyAsync(h.omgFR, omgFR, sizeof(double2) * S, hipMemcpyHostToDevice, R->st));
-    HIPCHK(hipMemcpyAsync(h.urFR, urFR, sizeof(double2) * S, hipMemcpyHostToDevice, R->st));
-    HIPCHK(hipMemcpyAsync(h.upFR, upFR, sizeof(double2) * S, hipMemcpyHostToDevice, R->st));
+    std::unique_lock<std::mutex> lk;   // held until the copies have run
+    if (char* stg = stage_take(lk, sizeof(double2) * 4 * S)) {
+        const double* const from[4] = {tFR, omgFR, upFR, urFR};
+        for (int k = 0; k < 4; ++k) std::memcpy(stg + k * sizeof(double2) * S, from[k], sizeof(double2) * S);
+        HIPCHK(hipMemcpyAsync(h.tFR, stg, sizeof(double2) * 4 * S, hipMemcpyHostToDevice, R->st));
+    } else {
+        HIPCHK(hipMemcpyAsync(h.tFR, tFR, sizeof(double2) * S, hipMemcpyHostToDevice, R->st));
+        HIPCHK(hipMemcpyAsync(h.omgFR, omgFR, sizeof(double2) * S, hipMemcpyHostToDevice, R->st));
+        HIPCHK(hipMemcpyAsync(h.urFR, urFR, sizeof(double2) * S, hipMemcpyHostToDevice, R->st));
+        HIPCHK(hipMemcpyAsync(h.upFR, upFR, sizeof(double2) * S, hipMemcpyHostToDevice, R->st));
+    }
     if (R->sc.kind != SK_IMEX) {
         // init_perturbation / init_fields: temp_spec = tFR, omg_spec = omgFR,
         // uphi_bar_spec = upFR(1,:) (init.F90:167-174, 393-397)
@@ -2356,6 +2410,18 @@ int fdns_get_state(fdns_run* R, double* tFR, double* omgFR, double* urFR, double
     if (!R) return fail(FDNS_EINVAL, "null run");
     const size_t S = (size_t)(R->p.Nm + 1) * R->p.Nr;
     const RunDesc& h = R->h;
+    {
+        std::unique_lock<std::mutex> lk;
+        const size_t F = sizeof(double2) * S;
+        if (char* stg = stage_take(lk, F * (psi ? 5 : 4))) {
+            HIPCHK(hipMemcpyAsync(stg, h.tFR, F * (psi ? 5 : 4), hipMemcpyDeviceToHost, R->st));
+            HIPCHK(hipStreamSynchronize(R->st));
+            double* const to[5] = {tFR, omgFR, upFR, urFR, psi};
+            for (int k = 0; k < 5; ++k)
+                if (to[k]) std::memcpy(to[k], stg + k * F, F);
+            return 0;
+        }
+    }
     HIPCHK(hipStreamSynchronize(R->st));
     if (tFR) HIPCHK(hipMemcpy(tFR, h.tFR, sizeof(double2) * S, hipMemcpyDeviceToHost));
     if (omgFR) HIPCHK(hipMemcpy(omgFR, h.omgFR, sizeof(double2) * S, hipMemcpyDeviceToHost));
