@@ -3281,6 +3281,14 @@ __device__ __forceinline__ void fu_rows(const double* A, const int ld, const int
     }
 }
 
+// The sum of a value over the wavefront's lanes.
+__device__ __forceinline__ double wave_total(double v)
+{
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) v = v + __shfl_xor(v, d);
+    return v;
+}
+
 // The other part (real <-> imaginary) of this lane's complex value.
 __device__ __forceinline__ double other_part(double v)
 {
@@ -3294,21 +3302,21 @@ __device__ __forceinline__ double other_part(double v)
 // wavefront 0 the real, wavefront 1 the imaginary part): right-hand side
 // x[4 i + part], solution to y.  The factor is staged in LDS from the kernel's
 // start in launches of one workgroup per CU, else read from memory.
-__device__ __forceinline__ void fu_m0_stage(const RunDesc& R, const int N, double* stg)
+__device__ __forceinline__ void fu_stage(const double* A, const int N, double* stg)
 {
     const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const BRes fr = bres(R.Ti, sizeof(double) * (size_t)N * N);
+    const BRes fr = bres(A, sizeof(double) * (size_t)N * N);
     for (int c = wv; 128 * c < N * N; c += (int)blockDim.x / 64) lds_dma(fr, (double2*)(stg + 128 * c), 16 * (64 * c + lane));
 }
 template <int SLOTS, class Col>
-__device__ __forceinline__ void fu_m0(const RunDesc& R, const int N, const double* x, double* y, Col col)
+__device__ __forceinline__ void fu_lu(const int* perm, const int N, const double* x, double* y, Col col)
 {
     const int lane = threadIdx.x & 63, im = (threadIdx.x >> 6) & 1;
     double v[SLOTS];
 #pragma unroll
     for (int q = 0; q < SLOTS; ++q) {
         const int r = lane + 64 * q;
-        v[q] = r < N ? ((const LDS_AS double*)x)[4 * gload(R.pT + r) + im] : 0.0;
+        v[q] = r < N ? ((const LDS_AS double*)x)[4 * gload(perm + r) + im] : 0.0;
     }
     lu_solve_wave<SLOTS, 8>(v, col, N);
 #pragma unroll
@@ -3424,14 +3432,14 @@ enum FuVec : int { FV_C = 0, FV_Y = 1, FV_R = 2, FV_P1 = 3, FV_P2 = 4, FV_P3 = 5
             if (staged) {                                                                               \
                 const LDS_AS double* fl = (const LDS_AS double*)V(FU_ZVEC);                             \
                 auto cl = [fl, lane, N](int p, int q) { return fl[lane + 64 * p + N * q]; };            \
-                if (N <= 64) fu_m0<1>(R, N, V(FV_R), V(FV_Y), cl);                                      \
-                else if (N <= 128) fu_m0<2>(R, N, V(FV_R), V(FV_Y), cl);                                \
-                else fu_m0<3>(R, N, V(FV_R), V(FV_Y), cl);                                              \
+                if (N <= 64) fu_lu<1>(R.pT + 0, N, V(FV_R), V(FV_Y), cl);                                      \
+                else if (N <= 128) fu_lu<2>(R.pT + 0, N, V(FV_R), V(FV_Y), cl);                                \
+                else fu_lu<3>(R.pT + 0, N, V(FV_R), V(FV_Y), cl);                                              \
             } else {                                                                                    \
                 const BRes fr = bres(R.Ti, sizeof(double) * (size_t)N * N);                             \
                 auto cg = [fr, lane, N](int p, int q) { return bload(fr, 8 * (lane + 64 * p + N * q)); }; \
-                if (N <= 128) fu_m0<2>(R, N, V(FV_R), V(FV_Y), cg);                                     \
-                else fu_m0<3>(R, N, V(FV_R), V(FV_Y), cg);                                              \
+                if (N <= 128) fu_lu<2>(R.pT + 0, N, V(FV_R), V(FV_Y), cg);                                     \
+                else fu_lu<3>(R.pT + 0, N, V(FV_R), V(FV_Y), cg);                                              \
             }                                                                                           \
         } else {                                                                                        \
             for (int t = wv - 2; t < nrb; t += NW - 2) fu_rows<1>(R.Ui, N, N, N, t, V(FV_R), V(FV_Y), V(FV_Y), N, 12, 0); \
@@ -3462,7 +3470,7 @@ __global__ __launch_bounds__(64 * FU_MAXW) void k_imex_modes(const RunDesc* __re
     auto hp = [&](int j) { return ub ? (size_t)(i < N ? i : 0) : e_[j]; };
     auto hget = [&](const double2* f, int o, int j) { return gload((const double*)(f + slot(o) * hs + hp(j)) + part); };
     auto hput = [&](double2* f, int j, double z) { gstore((double*)(f + slot(0) * hs + hp(j)) + part, z); };
-    if (zero && staged) fu_m0_stage(R, N, V(FU_ZVEC));
+    if (zero && staged) fu_stage(R.Ti, N, V(FU_ZVEC));
     fill(FV_C, tspec, wspec);
     fill(FV_Y, R.urT, R.urW);
     pad(FV_R);
@@ -3601,7 +3609,7 @@ __global__ __launch_bounds__(64 * FU_MAXW) void k_rk_modes(const RunDesc* __rest
     double2 *const tspec = R.tspec, *const wspec = R.wspec, *const TFC = R.TFC, *const ubar = R.ubar;
     double2 *const FaX = v ? (double2*)R.FaW : (double2*)R.FaT, *const FdX = v ? (double2*)R.FdW : (double2*)R.FdT;
     double2 *const FdT = R.FdT, *const FdW = R.FdW, *const Fb = R.Fb;
-    if (zero && staged) fu_m0_stage(R, N, V(FU_ZVEC));
+    if (zero && staged) fu_stage(R.Ti, N, V(FU_ZVEC));
     if (fa_prev) fill(FV_Y, R.urT, R.urW);
     else pad(FV_Y);
     pad(FV_R);
@@ -3714,6 +3722,287 @@ __global__ __launch_bounds__(64 * FU_MAXW) void k_rk_modes(const RunDesc* __rest
                 put(urFR, j, 0, imr(j, zo));
             }
         }
+    }
+}
+
+// ---- the schemes' other radial work, in the same manner (one mode per workgroup)
+// Up to FU1_MAXN rows, at every number of runs (a run's bits do not depend on
+// the others).  The kernels with one wavefront per mode (k_rk_init, k_rk_asm,
+// k_rkx_rhs, k_rkx_update) pass each vector through four to ten radial DFTs
+// and, in the mean flow, one wavefront over all modes: a chain of 18, 51, 59
+// and 42 us at 49 x 96, whatever the number of modes.  Products with the
+// Chebyshev matrices take 6, 18, 19 and 17.  Steps, there / here: RK4 420 / 173
+// us for one run of 49 x 96, 1211 / 890 for 64; BHR553 298 / 135 and 831 / 691.
+// Above 64 rows one run gains more (129 x 128 RK4 937 / 305), but the factor in
+// LDS leaves one workgroup on a CU and 64 runs lose (97 x 128 RK4 3121 / 4510,
+// BHR553 2244 / 2451; from memory 4599 and 2470): those keep the wavefronts.
+constexpr int FU1_MAXN = 64;
+#define FU1_SETUP                        \
+    constexpr int P = 1;                 \
+    FU_SETUP;                            \
+    auto at1 = [&](int k) { return at(k, 0); }; \
+    auto get1 = [&](const double2* f, size_t slot = 0) { return get(f, 0, slot); }; \
+    auto put1 = [&](double2* f, size_t slot, double z) { put(f, 0, slot, z); }; \
+    const bool mine = in[0]
+
+// psi's coefficients from LAPpsi psi = -omega, the right-hand side (walls
+// zero) in FV_R's second vector -> FV_Y's first; the factor staged behind
+// FU_ZVEC vectors by the kernel.  Then psi and its derivative -> FV_P1, FV_P2,
+// and omega at the walls from psi's interior by the Lagrange weights
+// (Johnston / stress free) -> FV_C[i ? 2 + part : part].
+#define FU_LAP                                                                                          \
+    do {                                                                                                \
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                                                \
+        __syncthreads();                                                                                \
+        if (wv < 2) {                                                                                   \
+            const int lane = tid & 63;                                                                  \
+            const LDS_AS double* fl = (const LDS_AS double*)V(FU_ZVEC);                                 \
+            auto cl = [fl, lane, N](int p, int q) { return fl[lane + 64 * p + N * q]; };                \
+            fu_lu<1>(R.pL + (size_t)m0 * N, N, V(FV_R) + 2, V(FV_Y), cl);   /* N <= FU1_MAXN */         \
+        }                                                                                               \
+        __syncthreads();                                                                                \
+        products(2, 0x10, 0x11, 0x43);                                                                  \
+        __syncthreads();                                                                                \
+        if (tid < 4) {                                                                                  \
+            const int top = tid >> 1, lm = R.lm;   /* wall, this thread's part */                       \
+            const GPtr<const double> lw = R.lagw;                                                       \
+            const double* const ps = V(FV_P1) + (tid & 1);                                              \
+            double dp = 0.0, d2p = 0.0;                                                                 \
+            for (int q = 0; q < lm; ++q) {                                                              \
+                const double z = ps[4 * (top ? N - 2 - q : 1 + q)];                                     \
+                dp = dp + lw[2 * top * LAGMAX + q] * z;                                                 \
+                d2p = d2p + lw[(2 * top + 1) * LAGMAX + q] * z;                                         \
+            }                                                                                           \
+            V(FV_C)[tid] = R.mbc == 0 ? -(d2p - (2.0 * lw[2 * top * LAGMAX]) * dp) : lw[4 * LAGMAX + top] * dp; \
+        }                                                                                               \
+        __syncthreads();                                                                                \
+    } while (0)
+
+// lap z of this thread's vector, z its value, d1 and d2 its derivatives
+#define FU_LAPLACIAN(z, d1, d2) ((rri * (d1) + (d2)) - ((mm[0] * mm[0]) * rr2i) * (z))
+
+// k_rk_init's terms
+__global__ __launch_bounds__(64 * FU_MAXW) void k_rk_init_modes(const RunDesc* __restrict__ runs, const Shape sh, const int nrun)
+{
+    FU1_SETUP;
+    const double Pr = R.Pr, raPr = R.Ra / R.Pr;
+    fill(FV_C, R.tFR, zero ? R.upFR : R.omgFR);
+    pad(FV_R);
+    __syncthreads();
+    const double z = at1(FV_C);
+    if (v == 0 && !zero && mine) put1(R.Fb, 0, (-raPr) * imr(0, other_part(z)));
+    if (R.need_fd[0] == 0) return;
+    products(1, 0x3, 0x0, 0x2);
+    __syncthreads();
+    products(2, 0x21, 0x22, 0x43);
+    __syncthreads();
+    if (!mine) return;
+    const double d1 = at1(FV_P1), d2 = at1(FV_P2);
+    if (v == 0) put1(R.FdT, 0, (1.0 / Pr) * FU_LAPLACIAN(z, d1, d2));
+    else if (zero) put1(R.FdW, 0, part ? 0.0 : (d2 - rr2i * z) + rri * d1);
+    else put1(R.FdW, 0, FU_LAPLACIAN(z, d1, d2));
+}
+
+// The mean flow u (FV_C's second vector, with the new temperature in the
+// first): coefficients -> FV_R, derivative -> FV_P1.
+#define FU_MEAN                          \
+    do {                                 \
+        __syncthreads();                 \
+        products(1, 0x3, 0x0, 0x2);      \
+        __syncthreads();                 \
+        products(1, 0x1, 0x2, 0x3);      \
+        __syncthreads();                 \
+    } while (0)
+
+// k_rk_asm's step end
+__global__ __launch_bounds__(64 * FU_MAXW) void k_rk_asm_modes(const RunDesc* __restrict__ runs, const Shape sh, const int nrun)
+{
+    FU1_SETUP;
+    const int SS = R.S;
+    const bool fa = R.fa_col[SS - 1] != 0, ub = zero && v == 1;
+    const double dt = R.dt;
+    if (!zero) fu_stage(R.Li + (size_t)m0 * N * N, N, V(FU_ZVEC));
+    if (fa) fill(FV_Y, R.urT, R.urW);
+    else pad(FV_Y);
+    pad(FV_C);
+    pad(FV_R);
+    const double2 *const FaX = v ? (const double2*)R.FaW : (const double2*)R.FaT, *const FdX = v ? (const double2*)R.FdW : (const double2*)R.FdT;
+    const double y0 = ub ? gload((const double*)(R.ubar + (i < N ? i : 0)) + part) : get1(v ? R.wspec : R.tspec);
+    double last = 0.0;   // the last stage's explicit term
+    if (fa) {
+        const double up = other_part(get1(v ? R.upW : R.upT)), uw = gload((const double*)R.urw + (i < N ? i : 0));
+        __syncthreads();
+        products(1, 0x4, 0x1, 0x3);
+        __syncthreads();
+        last = ub ? (part ? 0.0 : -uw) : -((imr(0, up) + at1(FV_P1)) + rri * at1(FV_Y));
+    }
+    double F = 0.0;
+    for (int k = 0; k < SS; ++k) {
+        const double a = k == SS - 1 && fa ? last : get1(FaX, (size_t)k);
+        F = (F + R.bA[k] * a) + R.bD[k] * get1(FdX, (size_t)k);
+        if (v == 1 && !zero) F = F + R.bD[k] * get1(R.Fb, (size_t)k);
+    }
+    const double y = v == 1 && !zero ? (wall ? y0 : y0 + dt * F)
+                                     : (wall ? (i == 0 && zero && col == 0 ? 1.0 : 0.0) : y0 + dt * F);
+    if (mine) {
+        if (v == 0) {
+            put1(R.tFR, 0, y);
+            put1(R.tspec, 0, y);
+        }
+        V(zero ? FV_C : FV_R)[4 * i + col] = zero ? y : (wall ? 0.0 : -1.0 * y);
+    }
+    if (zero) {
+        FU_MEAN;
+        if (!mine) return;
+        if (v == 0) {
+            gstore((double*)(R.TFC + i) + part, at1(FV_R));
+            return;
+        }
+        const double w = rri * y + at1(FV_P1);
+        gstore((double*)(R.ubar + i) + part, y);
+        put1(R.upFR, 0, y);
+        put1(R.urFR, 0, 0.0);
+        put1(R.omgFR, 0, w);
+        put1(R.wspec, 0, w);
+        return;
+    }
+    FU_LAP;
+    const double z = at1(FV_P1), zo = other_part(z);
+    if (!mine) return;
+    if (v == 0) {
+        put1(R.upFR, 0, -1.0 * at1(FV_P2));
+        put1(R.urFR, 0, imr(0, zo));
+    } else {
+        const double w = wall ? V(FV_C)[(i ? 2 : 0) + part] : y;
+        put1(R.omgFR, 0, w);
+        put1(R.wspec, 0, w);
+    }
+}
+
+// k_rkx_update's stage value or step end
+__global__ __launch_bounds__(64 * FU_MAXW) void k_rkx_update_modes(const RunDesc* __restrict__ runs, const Shape sh, const int nrun,
+                                                                   const int s)
+{
+    FU1_SETUP;
+    const int SS = R.S, K = s == SS ? SS : s;
+    const bool fin = s == SS, ub = zero && v == 1;
+    const double dt = R.dt;
+    if (!zero) fu_stage(R.Li + (size_t)m0 * N * N, N, V(FU_ZVEC));
+    pad(FV_C);
+    pad(FV_Y);
+    pad(FV_R);
+    pad(FV_P3);
+    const double2 *const FdX = v ? (const double2*)R.FdW : (const double2*)R.FdT;
+    const double y0 = ub ? gload((const double*)(R.ubar + (i < N ? i : 0)) + part) : get1(v ? R.wspec : R.tspec);
+    double F = 0.0;
+    for (int k = 0; k < K; ++k) F = F + (fin ? R.bA[k] : R.aA[s * MAXS + k]) * get1(FdX, (size_t)k);
+    double y = y0 + dt * F;
+    if (wall && (v == 0 || zero)) y = i == 0 && zero && col == 0 ? 1.0 : 0.0;
+    if (mine) {
+        if (v == 0) {
+            put1(R.tFR, 0, y);
+            if (fin) put1(R.tspec, 0, y);
+        }
+        V(zero ? FV_C : FV_R)[4 * i + col] = zero ? y : (wall ? 0.0 : -1.0 * y);
+    }
+    if (zero) {
+        FU_MEAN;
+        if (!mine) return;
+        const double c = at1(FV_R), d = at1(FV_P1);
+        if (v == 0) {
+            if (fin) gstore((double*)(R.TFC + i) + part, c);
+            return;
+        }
+        const double w = rri * y + d;
+        if (fin) gstore((double*)(R.ubar + i) + part, y);
+        put1(R.upFR, 0, y);
+        put1(R.urFR, 0, 0.0);
+        put1(R.upC, 0, c);
+        put1(R.d1u, 0, d);
+        put1(R.omgFR, 0, w);
+        if (fin) put1(R.wspec, 0, w);
+        return;
+    }
+    FU_LAP;
+    const double z = at1(FV_P1), zo = other_part(z), up = -1.0 * at1(FV_P2);
+    if (mine) {
+        if (v == 0) {
+            put1(R.psi, 0, z);
+            put1(R.upFR, 0, up);
+            put1(R.urFR, 0, imr(0, zo));
+            V(FV_R)[4 * i + col] = up;
+        } else {
+            const double w = wall ? V(FV_C)[(i ? 2 : 0) + part] : y;
+            put1(R.omgFR, 0, w);
+            if (fin) put1(R.wspec, 0, w);
+        }
+    }
+    // upFC = chebtransform(u_phi) (fourierloop_rk.F90:210, 411) and d/dr of it
+    __syncthreads();
+    products(1, 0x3, 0x2, 0x5);
+    __syncthreads();
+    products(1, 0x1, 0x5, 0x3);
+    __syncthreads();
+    if (mine && v == 0) {
+        put1(R.upC, 0, at1(FV_P3));
+        put1(R.d1u, 0, at1(FV_P1));
+    }
+}
+
+// k_rkx_rhs's stage right-hand sides; the mean flow's sums over the modes take
+// a wavefront per level
+__global__ __launch_bounds__(64 * FU_MAXW) void k_rkx_rhs_modes(const RunDesc* __restrict__ runs, const Shape sh, const int nrun,
+                                                                const int s)
+{
+    FU1_SETUP;
+    const double Pr = R.Pr, raPr = R.Ra / R.Pr;
+    const bool ub = zero && v == 1;
+    fill(FV_C, R.tFR, zero ? R.upFR : R.omgFR);
+    fill(FV_Y, R.urT, R.urW);
+    pad(FV_R);
+    const double up = other_part(get1(v ? R.upW : R.upT)), uc = zero ? get1(R.upC) : 0.0;
+    if (zero) {
+        const double2 *const urF = R.urFR, *const upF = R.upFR, *const duF = R.d1u;
+        for (int l = wv; l < N; l += NW) {
+            double su = 0.0, sd = 0.0;
+#pragma unroll 2
+            for (int q = tid & 63; q < Nm1; q += 64) {
+                const size_t o = (size_t)q + (size_t)Nm1 * l;
+                const double2 a = gload(urF + o), b = gload(upF + o), c = gload(duF + o);
+                if (q == 0) {
+                    su = su + (a.x * b.x - a.y * b.y);
+                    sd = sd + (a.x * c.x - a.y * c.y);
+                } else {
+                    su = su + 2.0 * (a.x * b.x + a.y * b.y);
+                    sd = sd + 2.0 * (a.x * c.x + a.y * c.y);
+                }
+            }
+            su = wave_total(su);
+            sd = wave_total(sd);
+            if ((tid & 63) == 0) {
+                V(FV_T)[2 * l] = su;
+                V(FV_T)[2 * l + 1] = sd;
+            }
+        }
+    }
+    __syncthreads();
+    products(2, 0x43, 0x10, 0x32);   // coefficients -> FV_R, flux derivatives -> FV_P1
+    __syncthreads();
+    const double z = at1(FV_C), fl = at1(FV_P1), ur = at1(FV_Y);
+    if (ub && mine) V(FV_R)[4 * i + col] = uc;   // the mean flow's own coefficients
+    __syncthreads();
+    products(2, 0x21, 0x22, 0x54);
+    __syncthreads();
+    if (!mine) return;
+    const double d1 = at1(FV_P2), d2 = at1(FV_P3), adv = (imr(0, up) + fl) + rri * ur;
+    if (v == 0) {
+        put1(R.FdT, (size_t)s, (1.0 / Pr) * FU_LAPLACIAN(z, d1, d2) - adv);
+    } else if (zero) {
+        const double ud = (d2 - rr2i * z) + rri * d1;
+        put1(R.FdW, (size_t)s, part ? 0.0 : ud - (V(FV_T)[2 * i + 1] + rri * V(FV_T)[2 * i]));
+    } else {
+        const double buo = raPr * imr(0, V(FV_C)[4 * i + (part ^ 1)]);
+        put1(R.FdW, (size_t)s, (FU_LAPLACIAN(z, d1, d2) - adv) - buo);
     }
 }
 
@@ -4505,13 +4794,6 @@ __global__ __launch_bounds__(64) void k_inv(const double* __restrict__ LU, const
 // modes of its levels by itself took 290 (k_diag) and 340 us (k_budget) at
 // 129 x 256, bound by one chain of loads; these take 4.5, and the kernels that
 // integrate the sums 17 and 15.  |z^2| is x^2 + y^2.
-__device__ __forceinline__ double wave_total(double v)
-{
-#pragma unroll
-    for (int d = 32; d > 0; d >>= 1) v = v + __shfl_xor(v, d);
-    return v;
-}
-
 constexpr int LV_WAVES = 4;   // levels per workgroup
 
 // sy[j] = (sum_m |ur_m^2|, sum_m |up_m^2|) of level j
@@ -4848,6 +5130,7 @@ int kernels_init()
 #undef SETLDS4
     SETLDS((k_lu<512, 1>)) SETLDS((k_lu<512, 3>)) SETLDS((k_lu_small<1, 4>)) SETLDS((k_lu_small<2, 4>))
     SETLDS((k_lu_small<3, 8>)) SETLDS((k_lu_small<4, 8>)) SETLDS((k_lu_small<5, 8>)) SETLDS(k_solve<0>) SETLDS(k_solve<1>) SETLDS(k_m0)
+    SETLDS(k_rk_init_modes) SETLDS(k_rk_asm_modes) SETLDS(k_rkx_update_modes) SETLDS(k_rkx_rhs_modes)
     SETLDS(k_imex_modes<1>) SETLDS(k_imex_modes<2>) SETLDS(k_rk_modes<1>) SETLDS(k_rk_modes<2>)
 #define SETTILE(k) SETLDS((k<4, true, false>)) SETLDS((k<8, true, false>))
 #define SETTILEPF(k) SETTILE(k) SETLDS((k<4, true, true>)) SETLDS((k<8, true, true>)) \
@@ -5021,9 +5304,18 @@ void launch_rk_post(const RunDesc* runs, int nrun, const Shape& sh, int s, hipSt
     TILE_LAUNCH(k_rk_post, 5, 2, 0, s);
 }
 
+// One mode per workgroup (FU1_SETUP's kernels); factor: those that solve, with it in LDS.
+template <class K, class... A>
+static void fu1_launch(K k, bool factor, const RunDesc* runs, int nrun, const Shape& sh, hipStream_t st, A... a)
+{
+    hipLaunchKernelGGL(k, dim3(padded_grid(nrun * sh.Nm1)), dim3(64 * fu_waves(sh.N, nrun * sh.Nm1 <= 256)), fu_lds(sh.N, 1, factor),
+                       st, runs, sh, nrun, a...);
+}
+
 void launch_rk_asm(const RunDesc* runs, int nrun, const Shape& sh, hipStream_t st)
 {
-    RADIAL_LAUNCH(k_rk_asm);
+    if (sh.N <= FU1_MAXN) fu1_launch(k_rk_asm_modes, true, runs, nrun, sh, st);
+    else RADIAL_LAUNCH(k_rk_asm);
 }
 
 void launch_asm_LAP(double* A, const double* t, const double* D, const double* D2, const Shape& sh, int m0, int count,
@@ -5034,7 +5326,8 @@ void launch_asm_LAP(double* A, const double* t, const double* D, const double* D
 
 void launch_rk_init(const RunDesc* runs, int nrun, const Shape& sh, hipStream_t st)
 {
-    RADIAL_LAUNCH(k_rk_init);
+    if (sh.N <= FU1_MAXN) fu1_launch(k_rk_init_modes, false, runs, nrun, sh, st);
+    else RADIAL_LAUNCH(k_rk_init);
 }
 
 void launch_rkx_init(const RunDesc* runs, int nrun, const Shape& sh, hipStream_t st)
@@ -5044,12 +5337,14 @@ void launch_rkx_init(const RunDesc* runs, int nrun, const Shape& sh, hipStream_t
 
 void launch_rkx_update(const RunDesc* runs, int nrun, const Shape& sh, int s, hipStream_t st)
 {
-    RADIAL_LAUNCH(k_rkx_update, s);
+    if (sh.N <= FU1_MAXN) fu1_launch(k_rkx_update_modes, true, runs, nrun, sh, st, s);
+    else RADIAL_LAUNCH(k_rkx_update, s);
 }
 
 void launch_rkx_rhs(const RunDesc* runs, int nrun, const Shape& sh, int s, hipStream_t st)
 {
-    RADIAL_LAUNCH(k_rkx_rhs, s);
+    if (sh.N <= FU1_MAXN) fu1_launch(k_rkx_rhs_modes, false, runs, nrun, sh, st, s);
+    else RADIAL_LAUNCH(k_rkx_rhs, s);
 }
 
 // LDS of k_solve: the staged right-hand sides of the widest chunk (w real
