@@ -5,7 +5,7 @@
 //               transforms, the four products and the four forward transforms
 //               of Nr_maxLOOP (nonlin.F90:134-190), all in LDS.
 //   k_imex_pre / k_imex_mid / k_imex_post
-//               one wavefront per (run, Fourier mode): the IMEX mode update of
+//               one workgroup per (run, 16 Fourier modes): the IMEX mode update of
 //               Nm_maxLOOP (fourierloop.F90:108-230 with rhs_create.F90:24-385)
 //               split around the two solve phases: Chebyshev transforms, RHS
 //               assembly into the run's solve area, the new fields.
@@ -16,7 +16,7 @@
 //   k_solve     one solve phase (temperature, or vorticity-streamfunction and
 //               mean flow) of a group of runs: FP64 MFMA products of the
 //               resident operator inverses with the right-hand sides of every
-//               run sharing the operator set, or dgetrs per (run, mode).
+//               run sharing the operator set.
 //   k_asm_*     operator matrices of mat_build / mat_build_IRK /
 //               mat_build_uphibar (mat_assembly.F90:68-413), one workgroup per
 //               (mode, column), a chunk of modes per launch.
@@ -26,6 +26,14 @@
 //   k_inv       the needed columns of each operator's inverse from its LU
 //               factor (dgetrs on unit vectors), a wavefront per block of
 //               columns.
+//   k_imex_modes / k_rk_modes
+//               small launches: one workgroup per (run, mode) does what the
+//               three tile kernels and the two solve phases do; the same bits.
+//   k_rk_init, k_rk_asm, k_rkx_* and, up to 64 rows, their *_modes forms
+//               the radial work of the other scheme families, per (run, mode).
+//   k_solve_lu  LU mode's solves, dgetrs' order, one workgroup per (run, mode).
+//   k_level_ke / k_level_budget
+//               the sums over the modes of one level, one wavefront each.
 //   k_diag      KE and Nusselt (output.F90:232-265), one workgroup per run.
 //
 // All DFTs are LDS-resident Stockham transforms with radices 2, 3, 4, 5.
