@@ -38,6 +38,7 @@
 //
 // All DFTs are LDS-resident Stockham transforms with radices 2, 3, 4, 5.
 #include "fdns_internal.h"
+#include "fdns_sweep.h"
 
 #include <float.h>
 
@@ -1108,9 +1109,6 @@ __device__ void lu_solve_wave(double (&xr)[SLOTS], Col col, const int n)
 // thread, 8-byte loads, every wavefront in every block: 294 and 2053 us; the
 // diagonal block's steps masked and divided by the compiler's divide, x_j by
 // v_readlane: 325 and 2936 us; 16-column blocks spill (1430 us).
-constexpr int LUX_NB = 8;      // columns per block
-constexpr int LUX_ROWS = 128;  // rows per wavefront
-__host__ __device__ constexpr int lux_waves(int n) { return (n + LUX_ROWS - 1) / LUX_ROWS; }
 constexpr int LUX_MAXT = 64 * lux_waves(2 * MAX_N);
 
 // Barrier of the LDS buffers only: the factor loads in flight stay in flight.
@@ -1195,10 +1193,10 @@ __device__ __forceinline__ void lux_diag(double2& x0, double2& x1, const double 
 __device__ __forceinline__ void lu_solve_reg(double2& x0, double2& x1, const double* __restrict__ A, const int n,
                                              double2* pub)
 {
-    constexpr int NB = LUX_NB, WB = LUX_ROWS / LUX_NB;   // blocks per wavefront
+    constexpr int NB = LUX_NB, WB = LUX_WB;
     const int tid = threadIdx.x, lane = tid & 63, r = 2 * tid;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int nblk = (n + NB - 1) / NB;
+    const int nblk = lux_blocks(n);
     __shared__ int first;
     // first block with a non-zero right-hand side
     if (tid == 0) first = nblk;
@@ -1255,10 +1253,10 @@ __device__ __forceinline__ void lu_solve_reg(double2& x0, double2& x1, const dou
         load(a0, a1, LOW ? b + 2 : b - 2, low);
     };
     // each sweep goes in pairs of blocks; a wavefront takes part up to its last
-    // (first) block and keeps the barriers after that
+    // (first) block and keeps the barriers after that (LuxShare)
     {
         constexpr auto low = std::true_type{};
-        const int pairs = (nblk - b0 + 1) / 2, mine = min(pairs, max(0, (WB * wv + WB - b0 + 1) / 2));
+        const auto [pairs, mine] = lux_forward(nblk, b0, wv);
         if (mine > 0) {
             load(p0, p1, b0, low);
             load(q0, q1, b0 + 1, low);
@@ -1273,7 +1271,7 @@ __device__ __forceinline__ void lu_solve_reg(double2& x0, double2& x1, const dou
     {
         constexpr auto up = std::false_type{};
         const int bt = nblk - 1;
-        const int pairs = (bt + 2) / 2, mine = (bt - WB * wv + 2) / 2;
+        const auto [pairs, mine] = lux_backward(nblk, wv);
         load(p0, p1, bt, up);
         load(q0, q1, bt - 1, up);
         lds_barrier();   // every read of the forward sweep's last values is done
