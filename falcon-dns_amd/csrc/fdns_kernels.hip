@@ -1119,6 +1119,16 @@ __device__ __forceinline__ void lds_barrier()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// Order for values that the lanes of one wavefront exchange through LDS: the
+// hardware keeps a wavefront's LDS operations in order, this keeps the
+// compiler from moving a lane's load ahead of another lane's store.
+__device__ __forceinline__ void wave_lds_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
 // The 8 x 8 diagonal block of a sweep on a quad of lanes: lane l of the quad
 // holds rows 2l and 2l + 1 of x and of the block (a0, a1); jb rows are inside
 // the matrix.  Columns ascending (LOW: unit lower triangle) or descending, each
@@ -4631,6 +4641,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W / 4)))
 #pragma unroll
                 for (int r = 0; r < 4; ++r) Ln[(16 * t + 4 * r + lk) * P + li] = C[r];
             });
+            wave_lds_sync();
             double a[RQ][NB];
 #pragma unroll
             for (int q = 0; q < RQ; ++q)
