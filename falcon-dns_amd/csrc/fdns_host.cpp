@@ -1265,7 +1265,7 @@ struct fdns_run {
     int tune_epoch = 0;        // launch choices the captured graph was made with
     double* series = nullptr;
     int series_cap = 0;
-    double* d_out6 = nullptr;
+    double* d_out = nullptr;   // fdns_diag's numbers and level sums
     SolveSched solo;           // solve plan of the run stepped alone
     double dt_new = 0.0;       // dt of the last step
     double dta[8] = {0};       // dt_array (variable dt), dta[0] the newest
@@ -2253,7 +2253,7 @@ int fdns_create(const fdns_params* p, fdns_run** out)
         }
     }
     h.series = R->series; h.cap = R->series_cap; h.nrec = 0;
-    if (hipMalloc((void**)&R->d_out6, sizeof(double) * 6) != hipSuccess) { fdns_destroy(R); return fail(FDNS_ENOMEM, "hipMalloc out"); }
+    if (hipMalloc((void**)&R->d_out, sizeof(double) * (6 + 2 * (size_t)N)) != hipSuccess) { fdns_destroy(R); return fail(FDNS_ENOMEM, "hipMalloc out"); }
     if ((rc = run_zero_dynamic(R)) || (rc = upload_desc(R))) { fdns_destroy(R); return rc; }
     if ((rc = plan_build(std::vector<fdns_run*>{R}, R->solo))) { fdns_destroy(R); return rc; }
     if (hipStreamSynchronize(R->st) != hipSuccess) { fdns_destroy(R); return fail(FDNS_EHIP, "factorisation failed"); }
@@ -2279,7 +2279,7 @@ int fdns_destroy(fdns_run* R)
     if (R->mem) hipFree(R->mem);
     if (R->own_dev) hipFree(R->own_dev);
     if (R->series) hipFree(R->series);
-    if (R->d_out6) hipFree(R->d_out6);
+    if (R->d_out) hipFree(R->d_out);
     R->solo.release();
     R->side.destroy();
     if (R->st) hipStreamDestroy(R->st);
@@ -2563,9 +2563,9 @@ int fdns_spectra(fdns_run* R, double* KEspec, double* Tspec)
 int fdns_diag(fdns_run* R, double* out6)
 {
     if (!R || !out6) return fail(FDNS_EINVAL, "null argument");
-    launch_diag(R->dev, 1, R->shape->sh, 0, R->d_out6, R->st);
+    launch_diag(R->dev, 1, R->shape->sh, 0, R->d_out, R->st);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(out6, R->d_out6, sizeof(double) * 6, hipMemcpyDeviceToHost, R->st));
+    HIPCHK(hipMemcpyAsync(out6, R->d_out, sizeof(double) * 6, hipMemcpyDeviceToHost, R->st));
     HIPCHK(hipStreamSynchronize(R->st));
     return 0;
 }

@@ -275,7 +275,10 @@ void launch_asm_U(double* A, const double* t, const double* D, const double* D2,
 void launch_lu(double* A, int* perm, int n, size_t stride, int nmat, hipStream_t st);
 void launch_inv(const double* LU, const int* perm, int n, size_t stride, int nmat, int col0, int ncols, double* out,
                 size_t ostride, hipStream_t st);
-void launch_diag(const RunDesc* runs, int nrun, const Shape& sh, int record, double* out6, hipStream_t st);
+// record: a row of the runs' series, as the last launch of their step (takes
+// their sy).  out (one run): the six numbers, and room for 2 N doubles behind
+// them; writes nothing of the run's, which may be stepping.
+void launch_diag(const RunDesc* runs, int nrun, const Shape& sh, int record, double* out, hipStream_t st);
 void launch_advance(RunDesc* runs, int nrun, hipStream_t st);
 int  kernels_init();   // raise dynamic LDS limits once
 

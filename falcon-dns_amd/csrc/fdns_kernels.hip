@@ -4813,8 +4813,10 @@ __global__ __launch_bounds__(64) void k_inv(const double* __restrict__ LU, const
 // integrate the sums 17 and 15.  |z^2| is x^2 + y^2.
 constexpr int LV_WAVES = 4;   // levels per workgroup
 
-// sy[j] = (sum_m |ur_m^2|, sum_m |up_m^2|) of level j
-__global__ __launch_bounds__(64 * LV_WAVES) void k_level_ke(const RunDesc* __restrict__ runs, const int Nm1, const int N)
+// lev[j] = (sum_m |ur_m^2|, sum_m |up_m^2|) of level j; lev null: the run's
+// sy, free at the end of its step
+__global__ __launch_bounds__(64 * LV_WAVES) void k_level_ke(const RunDesc* __restrict__ runs, const int Nm1, const int N,
+                                                            double2* lev)
 {
     const RunDesc& R = runs[blockIdx.y];
     const int lane = threadIdx.x & 63, j = blockIdx.x * LV_WAVES + (threadIdx.x >> 6);
@@ -4829,7 +4831,7 @@ __global__ __launch_bounds__(64 * LV_WAVES) void k_level_ke(const RunDesc* __res
     }
     a = wave_total(a);
     b = wave_total(b);
-    if (lane == 0) gstore((double2*)R.sy + j, mk(a, b));
+    if (lane == 0) gstore((lev ? lev : (double2*)R.sy) + j, mk(a, b));
 }
 
 // The budget's sums of level j (k_budget): sy[S + Nm1 j + 1] = (<u_r tt>,
@@ -4879,7 +4881,7 @@ __global__ __launch_bounds__(64 * LV_WAVES) void k_level_budget(const RunDesc* _
 // from the level sums of k_level_ke
 template <int NT, int MM>
 __global__ __launch_bounds__(NT) void k_diag(RunDesc* __restrict__ runs, const Shape sh0, const int record,
-                                             double* __restrict__ out6)
+                                             double* __restrict__ out6, const double2* __restrict__ lev)
 {
     extern __shared__ double2 smem[];
     const Shape sh = lds_twiddles<NT>(sh0, smem);     // twiddle table: smem[0..M)
@@ -4892,7 +4894,7 @@ __global__ __launch_bounds__(NT) void k_diag(RunDesc* __restrict__ runs, const S
     double* red = (double*)(V2 + N);
     const int tid = threadIdx.x;
     for (int j = tid; j < N; j += NT) {
-        const double2 s = R.sy[j];
+        const double2 s = gload((lev ? lev : (const double2*)R.sy) + j);
         V1[j] = mk(s.x * sh.rad[j], s.y * sh.rad[j]);
     }
     __syncthreads();
@@ -4921,8 +4923,7 @@ __global__ __launch_bounds__(NT) void k_diag(RunDesc* __restrict__ runs, const S
         const double Nut = V1[N - 1].x / ((1.0 - eta) / (log(eta)));
         const double Nub = V1[0].x / ((1.0 - eta) / (eta * log(eta)));
         if (out6) {
-            double* o = out6 + 6 * blockIdx.x;
-            o[0] = R.time; o[1] = KE; o[2] = Nut; o[3] = Nub; o[4] = 2.0 * pi * urk; o[5] = 2.0 * pi * upk;
+            out6[0] = R.time; out6[1] = KE; out6[2] = Nut; out6[3] = Nub; out6[4] = 2.0 * pi * urk; out6[5] = 2.0 * pi * upk;
         }
         if (record && R.series && R.nrec < R.cap) {
             double* row = R.series + 4 * (size_t)R.nrec;
@@ -5450,10 +5451,11 @@ void launch_lu(double* A, int* perm, int n, size_t stride, int nmat, hipStream_t
     else hipLaunchKernelGGL((k_lu<512, 3>), dim3(nmat), dim3(512), lu_lds(n, 8), st, A, perm, n, stride);
 }
 
-void launch_diag(const RunDesc* runs, int nrun, const Shape& sh, int record, double* out6, hipStream_t st)
+void launch_diag(const RunDesc* runs, int nrun, const Shape& sh, int record, double* out, hipStream_t st)
 {
-    hipLaunchKernelGGL(k_level_ke, dim3((sh.N + LV_WAVES - 1) / LV_WAVES, nrun), dim3(64 * LV_WAVES), 0, st, runs, sh.Nm1, sh.N);
-    TIER_DISPATCH(sh.M, hipLaunchKernelGGL((k_diag<B_, T_>), dim3(nrun), dim3(B_), diag_lds(sh), st, (RunDesc*)runs, sh, record, out6));
+    double2* const lev = out ? (double2*)(out + 6) : nullptr;
+    hipLaunchKernelGGL(k_level_ke, dim3((sh.N + LV_WAVES - 1) / LV_WAVES, nrun), dim3(64 * LV_WAVES), 0, st, runs, sh.Nm1, sh.N, lev);
+    TIER_DISPATCH(sh.M, hipLaunchKernelGGL((k_diag<B_, T_>), dim3(nrun), dim3(B_), diag_lds(sh), st, (RunDesc*)runs, sh, record, out, lev));
 }
 
 void launch_keep(const RunDesc* runs, int nrun, const Shape& sh, int with_up, hipStream_t st)

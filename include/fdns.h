@@ -145,7 +145,8 @@ int fdns_step(fdns_run* run, int nsteps);
 int fdns_get_dt(fdns_run* run, double* dt_new, double* dt_array);
 
 /* writeKE_spectral's KE and Nusselt numbers (output.F90:232-265) for the
- * current state: out = {t, KE, Nu_t, Nu_b, KE_r, KE_phi}. */
+ * current state: out = {t, KE, Nu_t, Nu_b, KE_r, KE_phi}.  Reads the run and
+ * writes nothing of it. */
 int fdns_diag(fdns_run* run, double* out6);
 /* Series recorded every n_KE steps: rows of {t, KE, Nu_t, Nu_b}. */
 int fdns_get_series(fdns_run* run, double* out, int cap_rows, int* nrows);
