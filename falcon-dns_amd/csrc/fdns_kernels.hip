@@ -967,17 +967,14 @@ constexpr int SOLVE_NB = 8;    // column block of lu_solve
 // columns 64 Q .. 64 Q + 63 (D ahead of their use, within the slot), so a
 // caller may stage one slot's columns at a time.
 
-// x / d by the reciprocal rcp = 1 / d (rounded): quotient, remainder,
-// correction (Markstein), which gives the correctly rounded quotient where
-// neither the reciprocal nor the remainder leaves the normal range.
-__device__ __forceinline__ double div_by(double x, double d, double rcp)
-{
-    const double q = x * rcp;
-    return fma(fma(-q, d, x), rcp, q);
-}
-
-// Whether a reciprocal may stand for the division by d (div_by).
-__device__ __forceinline__ bool rcp_safe(double d) { return fabs(d) > 0x1p-900 && fabs(d) < 0x1p900; }
+// The sweeps below spare their chains the masks (entries on the wrong side of
+// the diagonal count as zero) and the divisions (div_by).  Both are right as
+// long as every x_j is an ordinary number, and an x_j that is not shows in its
+// row of the solution (usual): a solve whose right-hand side is finite and
+// whose solution is not usual is done again with masks and divisions
+// (lu_wave_exact, lu_solve_exact), so that a run that overflows gets what
+// dgetrs gives it.  Right-hand sides that are not finite leave nothing finite
+// either way and are not repeated.
 
 // forward sweep over the columns of slot Q.  A step of the chain is the
 // broadcast of x_j and one fma: the entries on and above the diagonal count as
@@ -1030,7 +1027,7 @@ __device__ __forceinline__ void lu_wave_bwd(double (&xr)[SLOTS], Col col, const 
     double dg = col(Q, jlo + min(lane, jtop));
     if (!row) dg = 1.0;
     const double rcp = 1.0 / dg;
-    auto sweep = [&](auto div) {
+    auto sweep = [&](auto div, auto last) {
         double c[D][SLOTS];
         auto column = [&](double (&cv)[SLOTS], int j) {
             j = min(max(j, jlo), jhi);
@@ -1058,10 +1055,57 @@ __device__ __forceinline__ void lu_wave_bwd(double (&xr)[SLOTS], Col col, const 
                 }
             }
         }
-        xr[Q] = div(xr[Q]);
+        xr[Q] = last(xr[Q]);
     };
-    if (__any(!rcp_safe(dg))) sweep([&](double x) { return x / dg; });
-    else sweep([&](double x) { return div_by(x, dg, rcp); });
+    const auto exact = [&](double x) { return x / dg; };
+    if (__any(!rcp_safe(dg))) sweep(exact, exact);
+    else sweep([&](double x) { return div_by(x, dg, rcp); }, [&](double x) { return div_last(x, dg, rcp); });
+}
+
+// The solve by one wavefront with masks and divisions, from the factor in memory.
+template <int SLOTS>
+__device__ __forceinline__ void lu_wave_exact(double (&xr)[SLOTS], const double* __restrict__ A, const int n)
+{
+    const int lane = threadIdx.x & 63;
+#pragma unroll 1
+    for (int k = 0; k < 2 * n; ++k) {
+        const bool low = k < n;
+        const int j = low ? k : 2 * n - 1 - k;
+        double xj = 0.0, a[SLOTS];
+#pragma unroll
+        for (int q = 0; q < SLOTS; ++q) {
+            const int r = lane + 64 * q;
+            a[q] = r < n ? gload(A + (size_t)r + (size_t)n * j) : 0.0;
+            if (!low && r == j) xr[q] = xr[q] / a[q];
+            if (j >> 6 == q) xj = rdl(xr[q], j & 63);
+        }
+#pragma unroll
+        for (int q = 0; q < SLOTS; ++q) {
+            const int r = lane + 64 * q;
+            if (low ? r > j && r < n : r < j) xr[q] = fma(-xj, a[q], xr[q]);
+        }
+    }
+}
+
+// After the sweeps: xr stands, or the solve is done again from the right-hand side rhs(q).
+template <int SLOTS, class Rhs>
+__device__ __forceinline__ void lu_wave_check(double (&xr)[SLOTS], const double* A, const int n, Rhs rhs)
+{
+    bool ok = true;
+#pragma unroll
+    for (int q = 0; q < SLOTS; ++q) ok = ok && ((int)(threadIdx.x & 63) + 64 * q >= n || usual(xr[q]));
+    if (!__any(!ok)) return;
+    double b[SLOTS];
+    ok = true;
+#pragma unroll
+    for (int q = 0; q < SLOTS; ++q) {
+        b[q] = rhs(q);
+        ok = ok && fabs(b[q]) <= DBL_MAX;
+    }
+    if (__any(!ok)) return;
+    lu_wave_exact<SLOTS>(b, A, n);
+#pragma unroll
+    for (int q = 0; q < SLOTS; ++q) xr[q] = b[q];
 }
 
 // The whole solve with every column readable by col.
@@ -1136,7 +1180,9 @@ __device__ __forceinline__ void wave_lds_sync()
 // zero, so that a step of the chain is the broadcast of x_j and one fma per
 // row and part, without a mask or a branch; the division is three
 // multiply-adds by a reciprocal formed ahead of the chain, on every lane at
-// once, and the divided values are formed again for all lanes at the end.
+// once, and the divided values are formed again for all lanes at the end (a
+// quotient that rounds to the smallest subnormal may come out zero: telling
+// the two apart, as div_last does, cost 1 % of the solve).
 // Called by a whole wavefront, mine: the lane is in the block's quad; the
 // other lanes' x is left as it is.
 template <bool LOW>
@@ -1294,50 +1340,118 @@ __device__ __forceinline__ void lu_solve_reg(double2& x0, double2& x1, const dou
     }
 }
 
+// lu_solve_reg with masks and divisions, a column at a time.
+__device__ __forceinline__ void lu_solve_exact(double2& x0, double2& x1, const double* __restrict__ A, const int n, double2* pub)
+{
+    const int r = 2 * (int)threadIdx.x;
+    auto at = [&](int i, int j) { return i < n ? gload(A + (size_t)i + (size_t)n * j) : 0.0; };
+    lds_barrier();   // every read of the sweeps' last values is done
+#pragma unroll 1
+    for (int k = 0; k < 2 * n; ++k) {
+        const bool low = k < n;
+        const int j = low ? k : 2 * n - 1 - k;
+        const double a0 = at(r, j), a1 = at(r + 1, j);
+        if (r == (j & ~1)) {
+            double2& xj = j & 1 ? x1 : x0;
+            const double d = j & 1 ? a1 : a0;
+            if (!low) xj = mk(xj.x / d, xj.y / d);
+            lstore(pub + (k & 1), xj);
+        }
+        lds_barrier();
+        const double2 xj = lload(pub + (k & 1));
+        if (low ? r > j : r < j) x0 = mk(fma(-xj.x, a0, x0.x), fma(-xj.y, a0, x0.y));
+        if (low ? r + 1 > j : r + 1 < j) x1 = mk(fma(-xj.x, a1, x1.x), fma(-xj.y, a1, x1.y));
+    }
+}
+
+// The system that workgroup blk of a LU-mode launch solves: modes go round the
+// XCDs and a mode's runs, which may share its factor, stay on one XCD's L2.
+struct LuxSystem {
+    const double* A;
+    const int* perm;
+    const double2* v;   // right-hand side and solution: its row 0 of the solve areas
+    double2* y;
+    int m, n, z;        // mode (past the last: nothing to do); order; rows below z have zero right-hand sides
+    __device__ __forceinline__ double2 rhs(int r) const   // row r of the permuted right-hand side, zero past n
+    {
+        const int p = r < n ? gload(perm + r) : -1;
+        return p >= z ? gload(v + p) : mk(0.0, 0.0);
+    }
+};
+template <int phase>
+__device__ __forceinline__ LuxSystem lux_system(const RunDesc* __restrict__ runs, const int nrun, const Shape& sh,
+                                                const int stage, const int blk)
+{
+    const int N = sh.N, k = blk >> 3, ri = k % nrun;
+    LuxSystem s;
+    s.m = 8 * (k / nrun) + (blk & 7);
+    s.n = N;
+    s.z = 0;
+    if (s.m >= sh.Nm1) return s;
+    const RunDesc& R = runs[ri];
+    const size_t MS = 2 * (size_t)N;     // solve-area entries per mode
+    s.v = (const double2*)R.sx + (size_t)s.m * MS;
+    s.y = (double2*)R.sy + (size_t)s.m * MS;
+    if (phase == 0) {
+        s.A = R.TiS[stage] + (size_t)s.m * N * N;
+        s.perm = R.pTS[stage] + (size_t)s.m * N;
+    } else if (s.m == 0) {
+        s.A = R.UiS[stage];
+        s.perm = R.pUS[stage];
+        s.v += N;
+        s.y += N;
+    } else {
+        s.A = R.FiS[stage] + (size_t)(s.m - 1) * 4 * N * N;
+        s.perm = R.pFS[stage] + (size_t)(s.m - 1) * 2 * N;
+        s.n = 2 * N;
+        s.z = N;   // the psi rows of the coupled system
+    }
+    return s;
+}
+
 // The implicit solves of one phase in LU mode (fdns_params.solver): one
-// workgroup per (run, mode), dgetrs in its operation order.  Modes go round
-// the XCDs and a mode's runs, which may share its factor, stay on one XCD's
-// L2.
+// workgroup per (run, mode), dgetrs in its operation order.  The solution is
+// stored, then looked over; where it has to be done again the system is looked
+// up again too (an opaque block index), so that the sweeps' registers hold
+// nothing for it: kept across the sweeps, and behind a barrier that waits for
+// the stores, looking over cost 3 % of the coupled solves at 257 x 768, so 1 %
+// (249.3 -> 251.5 us).
 template <int phase>
 __global__ __launch_bounds__(LUX_MAXT) __attribute__((amdgpu_waves_per_eu(5))) void k_solve_lu(
     const RunDesc* __restrict__ runs, const int nrun, const Shape sh, const int stage)
 {
     __shared__ double2 pub[2 * LUX_NB];
-    const int N = sh.N, tid = threadIdx.x;
-    const int k = (int)blockIdx.x >> 3;
-    const int m = 8 * (k / nrun) + ((int)blockIdx.x & 7), ri = k % nrun;
-    if (m >= sh.Nm1) return;
-    const RunDesc& R = runs[ri];
-    const size_t MS = 2 * (size_t)N;     // solve-area entries per mode
-    const double2* v = (const double2*)R.sx + (size_t)m * MS;
-    double2* y = (double2*)R.sy + (size_t)m * MS;
-    // o: the system's row 0 in the solve area; z: rows below z have zero
-    // right-hand sides (the psi rows of the coupled system)
-    const double* A;
-    const int* perm;
-    int n = N, o = 0, z = 0;
-    if (phase == 0) {
-        A = R.TiS[stage] + (size_t)m * N * N;
-        perm = R.pTS[stage] + (size_t)m * N;
-    } else if (m == 0) {
-        A = R.UiS[stage];
-        perm = R.pUS[stage];
-        o = N;
-    } else {
-        A = R.FiS[stage] + (size_t)(m - 1) * 4 * N * N;
-        perm = R.pFS[stage] + (size_t)(m - 1) * 2 * N;
-        n = 2 * N;
-        z = N;
-    }
-    auto rhs = [&](int r) {
-        const int p = r < n ? gload(perm + r) : -1;
-        return p >= z ? gload(v + o + p) : mk(0.0, 0.0);
+    __shared__ int odd;
+    const int r = 2 * (int)threadIdx.x;
+    auto store = [&](const LuxSystem& s, const double2& x0, const double2& x1) {
+        const bool real_out = phase == 1 && s.m == 0;
+        if (r < s.n) gstore(s.y + r, mk(x0.x, real_out ? 0.0 : x0.y));
+        if (r + 1 < s.n) gstore(s.y + r + 1, mk(x1.x, real_out ? 0.0 : x1.y));
     };
-    double2 x0 = rhs(2 * tid), x1 = rhs(2 * tid + 1);
-    lu_solve_reg(x0, x1, A, n, pub);
-    const bool real_out = phase == 1 && m == 0;
-    if (2 * tid < n) gstore(y + o + 2 * tid, mk(x0.x, real_out ? 0.0 : x0.y));
-    if (2 * tid + 1 < n) gstore(y + o + 2 * tid + 1, mk(x1.x, real_out ? 0.0 : x1.y));
+    if (threadIdx.x == 0) odd = 0;
+    {
+        const LuxSystem s = lux_system<phase>(runs, nrun, sh, stage, blockIdx.x);
+        if (s.m >= sh.Nm1) return;
+        double2 x0 = s.rhs(r), x1 = s.rhs(r + 1);
+        lu_solve_reg(x0, x1, s.A, s.n, pub);
+        store(s, x0, x1);   // in flight past the barrier
+        if ((r < s.n && !(usual(x0.x) && usual(x0.y))) || (r + 1 < s.n && !(usual(x1.x) && usual(x1.y)))) odd = 1;
+    }
+    lds_barrier();
+    if (!odd) return;
+    __syncthreads();
+    if (threadIdx.x == 0) odd = 0;
+    __syncthreads();
+    int blk = blockIdx.x;
+    asm volatile("" : "+s"(blk));
+    const LuxSystem s = lux_system<phase>(runs, nrun, sh, stage, blk);
+    double2 x0 = s.rhs(r), x1 = s.rhs(r + 1);
+    const auto finite = [](double2 z) { return fabs(z.x) <= DBL_MAX && fabs(z.y) <= DBL_MAX; };
+    if (!(finite(x0) && finite(x1))) odd = 1;
+    __syncthreads();
+    if (odd) return;
+    lu_solve_exact(x0, x1, s.A, s.n, pub);
+    store(s, x0, x1);
 }
 
 constexpr int SOLVE_KC = 16;   // MFMA k-steps (4 columns of A each) loaded ahead per wavefront
@@ -1447,13 +1561,14 @@ __device__ void m0_solve(const RunDesc& R, const Shape& sh, double2* smem)
     for (int i = tid; i < N; i += NT) lstore(x + i, gload((const double2*)R.sx + i));
     stage(0, min(64, N));
     double xr[2] = {0.0, 0.0};
+    auto rhs = [&](int q) {
+        const int i = lane + 64 * q;
+        const double2 v = (i < N) ? lload(x + gload(R.pT + i)) : mk(0.0, 0.0);
+        return im ? v.y : v.x;
+    };
     if (tid < 128) {
 #pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            const int i = lane + 64 * q;
-            const double2 v = (i < N) ? lload(x + gload(R.pT + i)) : mk(0.0, 0.0);
-            xr[q] = im ? v.y : v.x;
-        }
+        for (int q = 0; q < 2; ++q) xr[q] = rhs(q);
     }
     auto colA = [fl, lane, N](int p, int j) { return fl[lane + 64 * p + N * j]; };
     auto colB = [fl, lane, N](int p, int j) { return fl[lane + 64 * p + N * (j - 64)]; };
@@ -1468,7 +1583,10 @@ __device__ void m0_solve(const RunDesc& R, const Shape& sh, double2* smem)
     }
     if (tid < 128) {
         lu_wave_bwd<0, 2, 4>(xr, colA, N);
-        // every gather of x was before the stagings' barriers
+        lu_wave_check<2>(xr, R.Ti, N, rhs);
+    }
+    __syncthreads();   // every gather of x is done
+    if (tid < 128) {
         LDS_AS double* xd = (LDS_AS double*)x + im;
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
@@ -1594,16 +1712,15 @@ __global__ __launch_bounds__(NT) void k_m0(const RunDesc* __restrict__ runs, con
         // of any store), swept, stored
         const int lane = tid & 63, im = (tid >> 6) & 1;
         double xr[3] = {0.0, 0.0, 0.0};
+        auto rhs = [&](int q) {
+            const int i = lane + 64 * q;
+            const double2 v = (i < N) ? lload(x + gload(R.pT + i)) : mk(0.0, 0.0);
+            return im ? v.y : v.x;
+        };
         if (tid < 128) {
 #pragma unroll
-            for (int q = 0; q < 3; ++q) {
-                const int i = lane + 64 * q;
-                const double2 v = (i < N) ? lload(x + gload(R.pT + i)) : mk(0.0, 0.0);
-                xr[q] = im ? v.y : v.x;
-            }
-        }
-        __syncthreads();
-        if (tid < 128) {
+            for (int q = 0; q < 3; ++q) xr[q] = rhs(q);
+
             const LDS_AS double* fl = (const LDS_AS double*)f;
             auto col = [fl, lane, N](int p, int j) { return fl[lane + 64 * p + N * j]; };
             if (N <= 128) {
@@ -1614,6 +1731,10 @@ __global__ __launch_bounds__(NT) void k_m0(const RunDesc* __restrict__ runs, con
             } else {
                 lu_solve_wave<3, 4>(xr, col, N);
             }
+            lu_wave_check<3>(xr, R.Ti, N, rhs);
+        }
+        __syncthreads();   // every gather of x is done
+        if (tid < 128) {
             LDS_AS double* xd = (LDS_AS double*)x + im;
 #pragma unroll
             for (int q = 0; q < 3; ++q) {
@@ -3325,16 +3446,18 @@ __device__ __forceinline__ void fu_stage(const double* A, const int N, double* s
     for (int c = wv; 128 * c < N * N; c += (int)blockDim.x / 64) lds_dma(fr, (double2*)(stg + 128 * c), 16 * (64 * c + lane));
 }
 template <int SLOTS, class Col>
-__device__ __forceinline__ void fu_lu(const int* perm, const int N, const double* x, double* y, Col col)
+__device__ __forceinline__ void fu_lu(const double* A, const int* perm, const int N, const double* x, double* y, Col col)
 {
     const int lane = threadIdx.x & 63, im = (threadIdx.x >> 6) & 1;
     double v[SLOTS];
-#pragma unroll
-    for (int q = 0; q < SLOTS; ++q) {
+    auto rhs = [&](int q) {
         const int r = lane + 64 * q;
-        v[q] = r < N ? ((const LDS_AS double*)x)[4 * gload(perm + r) + im] : 0.0;
-    }
+        return r < N ? ((const LDS_AS double*)x)[4 * gload(perm + r) + im] : 0.0;
+    };
+#pragma unroll
+    for (int q = 0; q < SLOTS; ++q) v[q] = rhs(q);
     lu_solve_wave<SLOTS, 8>(v, col, N);
+    lu_wave_check<SLOTS>(v, A, N, rhs);
 #pragma unroll
     for (int q = 0; q < SLOTS; ++q) {
         const int r = lane + 64 * q;
@@ -3448,14 +3571,14 @@ enum FuVec : int { FV_C = 0, FV_Y = 1, FV_R = 2, FV_P1 = 3, FV_P2 = 4, FV_P3 = 5
             if (staged) {                                                                               \
                 const LDS_AS double* fl = (const LDS_AS double*)V(FU_ZVEC);                             \
                 auto cl = [fl, lane, N](int p, int q) { return fl[lane + 64 * p + N * q]; };            \
-                if (N <= 64) fu_lu<1>(R.pT + 0, N, V(FV_R), V(FV_Y), cl);                                      \
-                else if (N <= 128) fu_lu<2>(R.pT + 0, N, V(FV_R), V(FV_Y), cl);                                \
-                else fu_lu<3>(R.pT + 0, N, V(FV_R), V(FV_Y), cl);                                              \
+                if (N <= 64) fu_lu<1>(R.Ti, R.pT, N, V(FV_R), V(FV_Y), cl);                             \
+                else if (N <= 128) fu_lu<2>(R.Ti, R.pT, N, V(FV_R), V(FV_Y), cl);                       \
+                else fu_lu<3>(R.Ti, R.pT, N, V(FV_R), V(FV_Y), cl);                                     \
             } else {                                                                                    \
                 const BRes fr = bres(R.Ti, sizeof(double) * (size_t)N * N);                             \
                 auto cg = [fr, lane, N](int p, int q) { return bload(fr, 8 * (lane + 64 * p + N * q)); }; \
-                if (N <= 128) fu_lu<2>(R.pT + 0, N, V(FV_R), V(FV_Y), cg);                                     \
-                else fu_lu<3>(R.pT + 0, N, V(FV_R), V(FV_Y), cg);                                              \
+                if (N <= 128) fu_lu<2>(R.Ti, R.pT, N, V(FV_R), V(FV_Y), cg);                            \
+                else fu_lu<3>(R.Ti, R.pT, N, V(FV_R), V(FV_Y), cg);                                     \
             }                                                                                           \
         } else {                                                                                        \
             for (int t = wv - 2; t < nrb; t += NW - 2) fu_rows<1>(R.Ui, N, N, N, t, V(FV_R), V(FV_Y), V(FV_Y), N, 12, 0); \
@@ -3774,7 +3897,7 @@ constexpr int FU1_MAXN = 64;
             const int lane = tid & 63;                                                                  \
             const LDS_AS double* fl = (const LDS_AS double*)V(FU_ZVEC);                                 \
             auto cl = [fl, lane, N](int p, int q) { return fl[lane + 64 * p + N * q]; };                \
-            fu_lu<1>(R.pL + (size_t)m0 * N, N, V(FV_R) + 2, V(FV_Y), cl);   /* N <= FU1_MAXN */         \
+            fu_lu<1>(R.Li + (size_t)m0 * N * N, R.pL + (size_t)m0 * N, N, V(FV_R) + 2, V(FV_Y), cl);   /* N <= FU1_MAXN */         \
         }                                                                                               \
         __syncthreads();                                                                                \
         products(2, 0x10, 0x11, 0x43);                                                                  \

@@ -1,10 +1,13 @@
 // fdns_sweep.h -- how the wavefronts of a workgroup share the column-block
-// sweeps of the LU-mode solves (plain C++, so that the host can go over it).
+// sweeps of the LU-mode solves, and the sweeps' division (plain C++, so that
+// the host can go over them).
 #pragma once
 
 #ifdef __HIPCC__
+#define SWEEP_DEV __host__ __device__
 #define SWEEP_FN __host__ __device__ constexpr
 #else
+#define SWEEP_DEV
 #define SWEEP_FN constexpr
 #endif
 
@@ -36,5 +39,25 @@ SWEEP_FN LuxShare lux_backward(int nblk, int wv)
     const int mine = (nblk - LUX_WB * wv + 1) / 2;
     return {(nblk + 1) / 2, mine < 0 ? 0 : mine};
 }
+
+// x / d by the reciprocal rcp = 1 / d (rounded): quotient, remainder,
+// correction (Markstein), which gives the correctly rounded quotient where
+// neither the reciprocal (rcp_safe) nor the quotient or the remainder (usual)
+// leaves the normal range.  Beyond it an infinity, and a quotient next to the
+// largest number, give NaN.
+SWEEP_DEV inline double div_by(double x, double d, double rcp)
+{
+    const double q = x * rcp;
+    return __builtin_fma(__builtin_fma(-q, d, x), rcp, q);
+}
+// the quotient that stays in the solution: where it is zero the number itself,
+// zero or not usual
+SWEEP_DEV inline double div_last(double x, double d, double rcp)
+{
+    const double q = div_by(x, d, rcp);
+    return q == 0.0 ? x : q;
+}
+SWEEP_DEV inline bool rcp_safe(double d) { return __builtin_fabs(d) > 0x1p-400 && __builtin_fabs(d) < 0x1p400; }
+SWEEP_DEV inline bool usual(double q) { return q == 0.0 || (__builtin_fabs(q) > 0x1p-500 && __builtin_fabs(q) < 0x1p500); }
 
 }  // namespace fdns
