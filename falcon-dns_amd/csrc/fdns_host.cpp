@@ -1603,6 +1603,7 @@ int plan_build(const std::vector<fdns_run*>& runs, SolveSched& S)
 // summed per kernel class (FDNS_KC_* of include/fdns.h).
 struct KTimer {
     static constexpr int NCLS = FDNS_NKCLASS;
+    int tiles = 0;   // families (1 IMEX, 2 IMEXRK) that take the column tiles also where whole mode updates run
     std::vector<hipEvent_t> ev;
     std::vector<int> cls;
     size_t used = 0;
@@ -1680,8 +1681,8 @@ void imex_launches(const RunDesc* dev, int n, const Shape& sh, const SolveSched&
                    KTimer* kt, const Side* sd = nullptr)
 {
     if (first) TIMED(kt, FDNS_KC_OTHER, st, launch_imex_prep(dev, n, sh, st));
-    if (!kt && !ss.lu && mode_fused(sh, n)) {
-        launch_imex_modes(dev, n, sh, st);
+    if (!ss.lu && mode_fused(sh, n) && !(kt && (kt->tiles & 1))) {
+        TIMED(kt, FDNS_KC_IMEX_MID, st, launch_imex_modes(dev, n, sh, st));
         return;
     }
     TIMED(kt, FDNS_KC_IMEX_PRE, st, launch_imex_pre(dev, n, sh, st));
@@ -1695,8 +1696,8 @@ void imex_launches(const RunDesc* dev, int n, const Shape& sh, const SolveSched&
 void stage_launches(const RunDesc* dev, int n, const Shape& sh, const SolveSched& ss, int s, hipStream_t st,
                     KTimer* kt, const Side* sd = nullptr)
 {
-    if (!kt && !ss.lu && mode_fused(sh, n)) {
-        launch_rk_modes(dev, n, sh, s, st);
+    if (!ss.lu && mode_fused(sh, n) && !(kt && (kt->tiles & 2))) {
+        TIMED(kt, FDNS_KC_RK_MID, st, launch_rk_modes(dev, n, sh, s, st));
         return;
     }
     TIMED(kt, FDNS_KC_RK_PRE, st, launch_rk_pre(dev, n, sh, s, st));
@@ -3206,13 +3207,13 @@ int fdns_ens_step(fdns_ens* E, int nsteps, int use_graph)
 // Batched steps launched one kernel at a time with a HIP event pair around
 // every launch, the groups one after another on the ensemble's stream.
 // kernel_ms[c] / launches[c]: summed duration and count per kernel class
-// FDNS_KC_*; wall_ms: host wall time of the call.
-int fdns_ens_step_timed(fdns_ens* E, int nsteps, double* kernel_ms, int* launches, double* wall_ms)
+// FDNS_KC_*; wall_ms: host wall time of the call.  tiles: KTimer's.
+static int ens_step_timed(fdns_ens* E, int nsteps, double* kernel_ms, int* launches, double* wall_ms, int tiles)
 {
-    if (!E) return fail(FDNS_EINVAL, "null ensemble");
     if (E->kstep == 0)
         if (int rc = groups_retune(E->groups, E->tune_epoch, E->sg)) return rc;
     KTimer kt;
+    kt.tiles = tiles;
     HIPCHK(hipStreamSynchronize(E->st));
     const auto t0 = std::chrono::steady_clock::now();
     for (int k = 0; k < nsteps; ++k) {
@@ -3235,6 +3236,12 @@ int fdns_ens_step_timed(fdns_ens* E, int nsteps, double* kernel_ms, int* launche
         if (launches) launches[c] = cnt[c];
     }
     return 0;
+}
+
+int fdns_ens_step_timed(fdns_ens* E, int nsteps, double* kernel_ms, int* launches, double* wall_ms)
+{
+    if (!E) return fail(FDNS_EINVAL, "null ensemble");
+    return ens_step_timed(E, nsteps, kernel_ms, launches, wall_ms, 0);
 }
 
 int fdns_ens_destroy(fdns_ens* E)
@@ -3309,6 +3316,19 @@ int fdns_ens_autotune(fdns_ens* E, int steps, fdns_tuning* chosen, double* repor
     }
     if (!rc) rc = fdns_ens_create(clones.data(), (int)clones.size(), &S);
     if (!rc) rc = fdns_ens_step(S, 1, 0);   // the first step (prologue) untimed
+    // the ensemble's scheme families (KTimer::tiles), and those of the groups
+    // that launch tiles and batched solves: the tiles of a family whose groups
+    // all take whole mode updates are timed by themselves, for the report, and
+    // their choices kept
+    int families = 0, tiled = 0;
+    if (!rc) rc = ens_regroup(S);
+    if (!rc)
+        for (auto& g : S->groups) {
+            const int f = g.sc.kind == SK_IMEX ? 1 : (g.sc.kind == SK_IMEXRK ? 2 : 0);
+            families |= f;
+            if (g.solve.lu || !mode_fused(g.shape->sh, (int)g.runs.size())) tiled |= f;
+        }
+    const auto family = [](int c) { return c < 3 ? 1 : 2; };   // of tile kernel c
     double t_split[2] = {-1.0, -1.0};
     for (int pass = 0; pass < NT && !rc; ++pass) {
         fdns_tuning t = was;
@@ -3318,16 +3338,23 @@ int fdns_ens_autotune(fdns_ens* E, int steps, fdns_tuning* chosen, double* repor
         if ((rc = fdns_tuning_set(N, Nm, &t))) break;
         double ms[FDNS_NKCLASS];
         int cnt[FDNS_NKCLASS];
-        if ((rc = fdns_ens_step_timed(S, 1, ms, cnt, nullptr))) break;   // warm-up with these choices
-        if ((rc = fdns_ens_step_timed(S, steps, ms, cnt, nullptr))) break;
-        t_nl[pass % 2] += ms[FDNS_KC_NONLIN] / steps;
-        n_nl[pass % 2]++;
-        for (int c = 0; c < 6; ++c)
-            if (cnt[FDNS_KC_IMEX_PRE + c] > 0) {
-                t_tile[c][pass] += ms[FDNS_KC_IMEX_PRE + c] / steps;
-                n_tile[c][pass]++;
+        // as the steps run, then the families whose tiles they do not launch
+        for (int report_only = 0; report_only < 2; ++report_only) {
+            const int fam = report_only ? families & ~tiled : tiled;
+            if (report_only && !fam) break;
+            if ((rc = ens_step_timed(S, 1, ms, cnt, nullptr, report_only ? fam : 0))) break;   // warm-up with these choices
+            if ((rc = ens_step_timed(S, steps, ms, cnt, nullptr, report_only ? fam : 0))) break;
+            if (!report_only) {
+                t_nl[pass % 2] += ms[FDNS_KC_NONLIN] / steps;
+                n_nl[pass % 2]++;
             }
-        t_ch[pass % nch] += (ms[FDNS_KC_SOLVE_T] + ms[FDNS_KC_SOLVE_F]) / steps;
+            for (int c = 0; c < 6; ++c)
+                if ((fam & family(c)) && cnt[FDNS_KC_IMEX_PRE + c] > 0) {
+                    t_tile[c][pass] += ms[FDNS_KC_IMEX_PRE + c] / steps;
+                    n_tile[c][pass]++;
+                }
+            if (!report_only || !tiled) t_ch[pass % nch] += (ms[FDNS_KC_SOLVE_T] + ms[FDNS_KC_SOLVE_F]) / steps;
+        }
         n_ch[pass % nch]++;
     }
     // lane_split changes the concurrency of the groups, which the per-kernel
@@ -3348,7 +3375,7 @@ int fdns_ens_autotune(fdns_ens* E, int steps, fdns_tuning* chosen, double* repor
         if (t_nl[i] / n_nl[i] < t_nl[b] / n_nl[b]) b = i;
     best.nl_tpb = nl[b];
     for (int c = 0; c < 6; ++c) {
-        if (n_tile[c][0] == 0) continue;   // not launched by this ensemble: keep
+        if (!(tiled & family(c)) || n_tile[c][0] == 0) continue;   // not launched by this ensemble: keep
         b = 0;
         for (int i = 1; i < NT; ++i)
             if (t_tile[c][i] < t_tile[c][b]) b = i;
@@ -3359,7 +3386,7 @@ int fdns_ens_autotune(fdns_ens* E, int steps, fdns_tuning* chosen, double* repor
     b = 0;
     for (int i = 1; i < nch; ++i)
         if (t_ch[i] / n_ch[i] < t_ch[b] / n_ch[b]) b = i;
-    best.solve_chunk = ch[b];
+    if (tiled) best.solve_chunk = ch[b];
     best.lane_split = (t_split[1] > 0.0 && t_split[1] < t_split[0]) ? 1 : 0;
     // the per-kernel times miss how the groups' kernels share the chip: time
     // graph-replayed steps with the new choice and with the one in force

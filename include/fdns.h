@@ -249,7 +249,9 @@ int fdns_ens_step(fdns_ens* ens, int nsteps, int use_graph);
 /* the same batched steps launched without a graph and with the groups one
  * after another on the ensemble's stream, with a HIP event pair around every
  * kernel launch: kernel_ms[c] and launches[c] (FDNS_NKCLASS entries each) are
- * the summed duration and count per kernel class */
+ * the summed duration and count per kernel class.  A small group in inverse
+ * mode takes the whole mode update of a step or stage in one launch, counted
+ * in IMEX_MID or RK_MID; its other mode classes have none. */
 #define FDNS_KC_NONLIN    0   /* nonlinear pass (Nr_maxLOOP) */
 #define FDNS_KC_IMEX_PRE  1   /* IMEX temperature right-hand sides */
 #define FDNS_KC_IMEX_MID  2   /* IMEX new temperature, vorticity right-hand sides */
@@ -299,8 +301,10 @@ int fdns_tuning_set(int Nr, int Nm, const fdns_tuning* t);
  * step; then `steps` graph-replayed steps with lane_split off and on, keeping
  * the faster; last, 4 `steps` graph-replayed steps with the choice so found
  * and with the choice in force before the call, keeping the faster (the
- * per-kernel times do not see how groups share the chip).  Needs members of
- * one (Nr_max, Nm_max).  *chosen = the stored
+ * per-kernel times do not see how groups share the chip).  Where every group
+ * of a family (IMEX, IMEXRK) takes its mode updates in one launch (small
+ * groups in inverse mode), its tiles are timed for the report only and their
+ * choices left as they were; so solve_chunk where no group launches solves.  Needs members of one (Nr_max, Nm_max).  *chosen = the stored
  * choice; report (may be NULL) gets FDNS_TUNE_REPORT per-step milliseconds,
  * -1 for an option not tried or a kernel not launched:
  *   [0..1]        nonlinear pass, nl_tpb 128 / 256
