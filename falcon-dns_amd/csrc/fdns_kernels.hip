@@ -4934,74 +4934,102 @@ __global__ __launch_bounds__(64) void k_inv(const double* __restrict__ LU, const
 // modes of its levels by itself took 290 (k_diag) and 340 us (k_budget) at
 // 129 x 256, bound by one chain of loads; these take 4.5, and the kernels that
 // integrate the sums 17 and 15.  |z^2| is x^2 + y^2.
+// A few are not worth that launch (2 - 3 us of a call): where a lane per level
+// goes over at most 16 modes in all, k_diag and k_budget form the sums
+// themselves.  fdns_diag with / without the launch: 5 x 1 31.2 / 28.5 us,
+// 33 x 15 33.0 / 31.0, 129 x 15 37.8 / 37.7; fdns_budget 42.6 / 39.6,
+// 46.2 / 46.2, 57.0 / 65.7.
 constexpr int LV_WAVES = 4;   // levels per workgroup
+__host__ __device__ inline bool lv_few(int N, int Nm1) { return Nm1 * ((N + 63) / 64) <= 16; }
 
-// lev[j] = (sum_m |ur_m^2|, sum_m |up_m^2|) of level j; lev null: the run's
-// sy, free at the end of its step
+// (sum_m |ur_m^2|, sum_m |up_m^2|) of level j over the modes q, q + dq, ...
+__device__ __forceinline__ double2 level_ke(const RunDesc& R, const int Nm1, const int j, int q, const int dq)
+{
+    const double2 *ur = R.urFR, *up = R.upFR;
+    double a = 0.0, b = 0.0;
+#pragma unroll 4
+    for (; q < Nm1; q += dq) {
+        const double2 zr = gload(ur + q + (size_t)Nm1 * j), zp = gload(up + q + (size_t)Nm1 * j);
+        a = a + (zr.x * zr.x + zr.y * zr.y);
+        b = b + (zp.x * zp.x + zp.y * zp.y);
+    }
+    return mk(a, b);
+}
+
+// lev[j] = the sums of level j over all modes; lev null: the run's sy, free at
+// the end of its step
 __global__ __launch_bounds__(64 * LV_WAVES) void k_level_ke(const RunDesc* __restrict__ runs, const int Nm1, const int N,
                                                             double2* lev)
 {
     const RunDesc& R = runs[blockIdx.y];
     const int lane = threadIdx.x & 63, j = blockIdx.x * LV_WAVES + (threadIdx.x >> 6);
     if (j >= N) return;
-    const double2 *ur = R.urFR, *up = R.upFR;
-    double a = 0.0, b = 0.0;
-#pragma unroll 4
-    for (int q = lane; q < Nm1; q += 64) {
-        const double2 zr = gload(ur + q + (size_t)Nm1 * j), zp = gload(up + q + (size_t)Nm1 * j);
-        a = a + (zr.x * zr.x + zr.y * zr.y);
-        b = b + (zp.x * zp.x + zp.y * zp.y);
-    }
-    a = wave_total(a);
-    b = wave_total(b);
-    if (lane == 0) gstore((lev ? lev : (double2*)R.sy) + j, mk(a, b));
+    double2 s = level_ke(R, Nm1, j, lane, 64);
+    s.x = wave_total(s.x);
+    s.y = wave_total(s.y);
+    if (lane == 0) gstore((lev ? lev : (double2*)R.sy) + j, s);
 }
 
-// The budget's sums of level j (k_budget): sy[S + Nm1 j + 1] = (<u_r tt>,
-// <omega^2>), the Reynolds-stress column of the output, and at the walls
-// sum_m |up_m^2| in out[0], out[1].  sy holds k_budget_dr's derivatives.
+// The budget's sums of level j over the modes q, q + dq, ...: <u_r tt>,
+// <omega^2>, sum_m |up_m^2|, <u_r u_phi>, <u_r du_phi/dr>.  sy holds
+// k_budget_dr's derivatives.
+struct LevelBudget {
+    double ut, w2, up2, su, sd;
+};
+__device__ __forceinline__ LevelBudget level_budget(const RunDesc& R, const int Nm1, const int j, int q, const int dq)
+{
+    const size_t at = (size_t)Nm1 * j;
+    const double2 *urF = R.urFR, *upF = R.upFR, *omF = R.omgFR, *tpF = R.tpass, *duF = R.sy;
+    LevelBudget s = {0.0, 0.0, 0.0, 0.0, 0.0};
+#pragma unroll 2
+    for (; q < Nm1; q += dq) {
+        const double2 ur = gload(urF + at + q), up = gload(upF + at + q), om = gload(omF + at + q), tp = gload(tpF + at + q),
+                      du = gload(duF + at + q);
+        s.up2 = s.up2 + (up.x * up.x + up.y * up.y);
+        if (q == 0) {   // the mean's imaginary parts take part as the complex products have them
+            s.ut = s.ut + ur.x * tp.x;
+            s.w2 = s.w2 + (om.x * om.x - om.y * om.y);
+            s.su = s.su + (ur.x * up.x - ur.y * up.y);
+            s.sd = s.sd + (ur.x * du.x - ur.y * du.y);
+        } else {
+            s.ut = s.ut + 2.0 * (ur.x * tp.x + ur.y * tp.y);
+            s.w2 = s.w2 + 2.0 * (om.x * om.x + om.y * om.y);
+            s.su = s.su + 2.0 * (ur.x * up.x + ur.y * up.y);
+            s.sd = s.sd + 2.0 * (ur.x * du.x + ur.y * du.y);
+        }
+    }
+    return s;
+}
+// into the run's output o: the Reynolds-stress column of level j, and at the
+// walls sum_m |up_m^2| in o[0], o[1]
+__device__ __forceinline__ void put_level_budget(double* o, const LevelBudget& s, const double rr, const int j, const int N)
+{
+    o[4 + 3 * j + 1] = -(s.sd + rr * s.su);
+    if (j == 0) o[0] = s.up2;
+    if (j == N - 1) o[1] = s.up2;
+}
+
+// the sums of level j over all modes; sy[S + Nm1 j + 1] = (<u_r tt>, <omega^2>)
 __global__ __launch_bounds__(64 * LV_WAVES) void k_level_budget(const RunDesc* __restrict__ runs, const double* __restrict__ rr,
                                                                 const int Nm1, const int N, double* __restrict__ out)
 {
     const RunDesc& R = runs[blockIdx.y];
     const int lane = threadIdx.x & 63, j = blockIdx.x * LV_WAVES + (threadIdx.x >> 6);
     if (j >= N) return;
-    const size_t S = (size_t)Nm1 * N, at = (size_t)Nm1 * j;
-    const double2 *urF = R.urFR, *upF = R.upFR, *omF = R.omgFR, *tpF = R.tpass, *duF = R.sy;
-    double ut = 0.0, w2 = 0.0, up2 = 0.0, su = 0.0, sd = 0.0;
-#pragma unroll 2
-    for (int q = lane; q < Nm1; q += 64) {
-        const double2 ur = gload(urF + at + q), up = gload(upF + at + q), om = gload(omF + at + q), tp = gload(tpF + at + q),
-                      du = gload(duF + at + q);
-        up2 = up2 + (up.x * up.x + up.y * up.y);
-        if (q == 0) {   // the mean's imaginary parts take part as the complex products have them
-            ut = ut + ur.x * tp.x;
-            w2 = w2 + (om.x * om.x - om.y * om.y);
-            su = su + (ur.x * up.x - ur.y * up.y);
-            sd = sd + (ur.x * du.x - ur.y * du.y);
-        } else {
-            ut = ut + 2.0 * (ur.x * tp.x + ur.y * tp.y);
-            w2 = w2 + 2.0 * (om.x * om.x + om.y * om.y);
-            su = su + 2.0 * (ur.x * up.x + ur.y * up.y);
-            sd = sd + 2.0 * (ur.x * du.x + ur.y * du.y);
-        }
-    }
-    ut = wave_total(ut);
-    w2 = wave_total(w2);
-    up2 = wave_total(up2);
-    su = wave_total(su);
-    sd = wave_total(sd);
+    LevelBudget s = level_budget(R, Nm1, j, lane, 64);
+    s.ut = wave_total(s.ut);
+    s.w2 = wave_total(s.w2);
+    s.up2 = wave_total(s.up2);
+    s.su = wave_total(s.su);
+    s.sd = wave_total(s.sd);
     if (lane != 0) return;
-    double* o = out + (size_t)blockIdx.y * (4 + 3 * (size_t)N);
-    gstore((double2*)R.sy + S + at + 1, mk(ut, w2));
-    o[4 + 3 * j + 1] = -(sd + gload(rr + j) * su);
-    if (j == 0) o[0] = up2;
-    if (j == N - 1) o[1] = up2;
+    gstore((double2*)R.sy + (size_t)Nm1 * N + (size_t)Nm1 * j + 1, mk(s.ut, s.w2));
+    put_level_budget(out + (size_t)blockIdx.y * (4 + 3 * (size_t)N), s, gload(rr + j), j, N);
 }
 
 // writeKE_spectral: KE = 2 pi (radInt(sum_m |ur_m^2|) + radInt(sum_m |up_m^2|))
 // and the Nusselt numbers from d/dr of TFC (output.F90:232-265, integ.F90:36-76),
-// from the level sums of k_level_ke
+// from the level sums (level_ke)
 template <int NT, int MM>
 __global__ __launch_bounds__(NT) void k_diag(RunDesc* __restrict__ runs, const Shape sh0, const int record,
                                              double* __restrict__ out6, const double2* __restrict__ lev)
@@ -5017,7 +5045,7 @@ __global__ __launch_bounds__(NT) void k_diag(RunDesc* __restrict__ runs, const S
     double* red = (double*)(V2 + N);
     const int tid = threadIdx.x;
     for (int j = tid; j < N; j += NT) {
-        const double2 s = gload((lev ? lev : (const double2*)R.sy) + j);
+        const double2 s = lv_few(N, sh.Nm1) ? level_ke(R, sh.Nm1, j, 0, 1) : gload((lev ? lev : (const double2*)R.sy) + j);
         V1[j] = mk(s.x * sh.rad[j], s.y * sh.rad[j]);
     }
     __syncthreads();
@@ -5089,7 +5117,7 @@ __global__ __launch_bounds__(NT) void k_budget_dr(const RunDesc* __restrict__ ru
 
 // The mean-flow energy, power budget and mean-flow balance of
 // writeKE_spectral (output.F90:122-324) for one run per workgroup, from the
-// level sums of k_level_budget:
+// level sums (level_budget):
 // out[0..3] = {2 pi radInt(<u_phi>^2), viscous dissipation (stress free:
 // less the wall terms 8 pi sum_m |up_m^2|), 2 pi Ra/Pr radInt(<u_r tt>), t},
 // out[4 + 3 j + c] the upbalance_ columns of level j.  Azimuthal means by
@@ -5113,8 +5141,17 @@ __global__ __launch_bounds__(NT) void k_budget(const RunDesc* __restrict__ runs,
     const size_t S = (size_t)Nm1 * N;
     double* o = out + (size_t)blockIdx.x * (4 + 3 * (size_t)N);
     for (int j = tid; j < N; j += NT) {
-        const double2 lv = R.sy[S + (size_t)Nm1 * j + 1];
-        const double ut = lv.x, w2 = lv.y;
+        double ut, w2;
+        if (lv_few(N, Nm1)) {
+            const LevelBudget s = level_budget(R, Nm1, j, 0, 1);
+            put_level_budget(o, s, rr[j], j, N);
+            ut = s.ut;
+            w2 = s.w2;
+        } else {
+            const double2 s = R.sy[S + (size_t)Nm1 * j + 1];
+            ut = s.x;
+            w2 = s.y;
+        }
         const double2 u0 = R.upFR[(size_t)Nm1 * j];
         const double ua = u0.x;
         V0[j] = mk((ua * ua) * sh.rad[j], w2 * sh.rad[j]);
@@ -5577,7 +5614,8 @@ void launch_lu(double* A, int* perm, int n, size_t stride, int nmat, hipStream_t
 void launch_diag(const RunDesc* runs, int nrun, const Shape& sh, int record, double* out, hipStream_t st)
 {
     double2* const lev = out ? (double2*)(out + 6) : nullptr;
-    hipLaunchKernelGGL(k_level_ke, dim3((sh.N + LV_WAVES - 1) / LV_WAVES, nrun), dim3(64 * LV_WAVES), 0, st, runs, sh.Nm1, sh.N, lev);
+    if (!lv_few(sh.N, sh.Nm1))
+        hipLaunchKernelGGL(k_level_ke, dim3((sh.N + LV_WAVES - 1) / LV_WAVES, nrun), dim3(64 * LV_WAVES), 0, st, runs, sh.Nm1, sh.N, lev);
     TIER_DISPATCH(sh.M, hipLaunchKernelGGL((k_diag<B_, T_>), dim3(nrun), dim3(B_), diag_lds(sh), st, (RunDesc*)runs, sh, record, out, lev));
 }
 
@@ -5590,7 +5628,8 @@ void launch_keep(const RunDesc* runs, int nrun, const Shape& sh, int with_up, hi
 void launch_budget(const RunDesc* runs, int nrun, const Shape& sh, double* out, hipStream_t st)
 {
     RADIAL_LAUNCH(k_budget_dr);
-    hipLaunchKernelGGL(k_level_budget, dim3((sh.N + LV_WAVES - 1) / LV_WAVES, nrun), dim3(64 * LV_WAVES), 0, st, runs, sh.rr,
+    if (!lv_few(sh.N, sh.Nm1))
+        hipLaunchKernelGGL(k_level_budget, dim3((sh.N + LV_WAVES - 1) / LV_WAVES, nrun), dim3(64 * LV_WAVES), 0, st, runs, sh.rr,
                        sh.Nm1, sh.N, out);
     TIER_DISPATCH(sh.M, hipLaunchKernelGGL((k_budget<B_, T_>), dim3(nrun), dim3(B_), budget_lds(sh), st, runs, sh, out));
 }
