@@ -1062,11 +1062,35 @@ __device__ __forceinline__ void lu_wave_bwd(double (&xr)[SLOTS], Col col, const 
     else sweep([&](double x) { return div_by(x, dg, rcp); }, [&](double x) { return div_last(x, dg, rcp); });
 }
 
-// The solve by one wavefront with masks and divisions, from the factor in memory.
+// Whether this lane's rows of a solution are usual.
 template <int SLOTS>
-__device__ __forceinline__ void lu_wave_exact(double (&xr)[SLOTS], const double* __restrict__ A, const int n)
+__device__ __forceinline__ bool lu_wave_usual(const double (&xr)[SLOTS], const int n)
 {
+    bool ok = true;
+#pragma unroll
+    for (int q = 0; q < SLOTS; ++q) ok = ok && ((int)(threadIdx.x & 63) + 64 * q >= n || usual(xr[q]));
+    return ok;
+}
+
+// The solve again, by one wavefront with masks and divisions, from the factor
+// in memory (n <= 192) and the right-hand side rhs(row); out(row, value).  A
+// workgroup comes here behind a barrier after its sweeps, on a flag: the
+// sweeps' code and registers hold nothing for it (kept beside them, the flag's
+// test alone cost the m = 0 sweep of 129 rows 2 us of 32).
+template <class Rhs, class Out>
+__device__ __forceinline__ void lu_wave_exact(const double* __restrict__ A, const int* __restrict__ perm, const int n, Rhs rhs,
+                                              Out out)
+{
+    constexpr int SLOTS = 3;
     const int lane = threadIdx.x & 63;
+    double x[SLOTS];
+    bool ok = true;
+#pragma unroll
+    for (int q = 0; q < SLOTS; ++q) {
+        x[q] = lane + 64 * q < n ? rhs(gload(perm + lane + 64 * q)) : 0.0;
+        ok = ok && fabs(x[q]) <= DBL_MAX;
+    }
+    if (__any(!ok)) return;
 #pragma unroll 1
     for (int k = 0; k < 2 * n; ++k) {
         const bool low = k < n;
@@ -1076,36 +1100,18 @@ __device__ __forceinline__ void lu_wave_exact(double (&xr)[SLOTS], const double*
         for (int q = 0; q < SLOTS; ++q) {
             const int r = lane + 64 * q;
             a[q] = r < n ? gload(A + (size_t)r + (size_t)n * j) : 0.0;
-            if (!low && r == j) xr[q] = xr[q] / a[q];
-            if (j >> 6 == q) xj = rdl(xr[q], j & 63);
+            if (!low && r == j) x[q] = x[q] / a[q];
+            if (j >> 6 == q) xj = rdl(x[q], j & 63);
         }
 #pragma unroll
         for (int q = 0; q < SLOTS; ++q) {
             const int r = lane + 64 * q;
-            if (low ? r > j && r < n : r < j) xr[q] = fma(-xj, a[q], xr[q]);
+            if (low ? r > j && r < n : r < j) x[q] = fma(-xj, a[q], x[q]);
         }
     }
-}
-
-// After the sweeps: xr stands, or the solve is done again from the right-hand side rhs(q).
-template <int SLOTS, class Rhs>
-__device__ __forceinline__ void lu_wave_check(double (&xr)[SLOTS], const double* A, const int n, Rhs rhs)
-{
-    bool ok = true;
 #pragma unroll
-    for (int q = 0; q < SLOTS; ++q) ok = ok && ((int)(threadIdx.x & 63) + 64 * q >= n || usual(xr[q]));
-    if (!__any(!ok)) return;
-    double b[SLOTS];
-    ok = true;
-#pragma unroll
-    for (int q = 0; q < SLOTS; ++q) {
-        b[q] = rhs(q);
-        ok = ok && fabs(b[q]) <= DBL_MAX;
-    }
-    if (__any(!ok)) return;
-    lu_wave_exact<SLOTS>(b, A, n);
-#pragma unroll
-    for (int q = 0; q < SLOTS; ++q) xr[q] = b[q];
+    for (int q = 0; q < SLOTS; ++q)
+        if (lane + 64 * q < n) out(lane + 64 * q, x[q]);
 }
 
 // The whole solve with every column readable by col.
@@ -1561,14 +1567,13 @@ __device__ void m0_solve(const RunDesc& R, const Shape& sh, double2* smem)
     for (int i = tid; i < N; i += NT) lstore(x + i, gload((const double2*)R.sx + i));
     stage(0, min(64, N));
     double xr[2] = {0.0, 0.0};
-    auto rhs = [&](int q) {
-        const int i = lane + 64 * q;
-        const double2 v = (i < N) ? lload(x + gload(R.pT + i)) : mk(0.0, 0.0);
-        return im ? v.y : v.x;
-    };
     if (tid < 128) {
 #pragma unroll
-        for (int q = 0; q < 2; ++q) xr[q] = rhs(q);
+        for (int q = 0; q < 2; ++q) {
+            const int i = lane + 64 * q;
+            const double2 v = (i < N) ? lload(x + gload(R.pT + i)) : mk(0.0, 0.0);
+            xr[q] = im ? v.y : v.x;
+        }
     }
     auto colA = [fl, lane, N](int p, int j) { return fl[lane + 64 * p + N * j]; };
     auto colB = [fl, lane, N](int p, int j) { return fl[lane + 64 * p + N * (j - 64)]; };
@@ -1583,15 +1588,16 @@ __device__ void m0_solve(const RunDesc& R, const Shape& sh, double2* smem)
     }
     if (tid < 128) {
         lu_wave_bwd<0, 2, 4>(xr, colA, N);
-        lu_wave_check<2>(xr, R.Ti, N, rhs);
-    }
-    __syncthreads();   // every gather of x is done
-    if (tid < 128) {
+        // every gather of x was before the stagings' barriers
         LDS_AS double* xd = (LDS_AS double*)x + im;
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
             const int i = lane + 64 * q;
             if (i < N) xd[2 * i] = xr[q];
+        }
+        if (__any(!lu_wave_usual<2>(xr, N))) {
+            const double* v = (const double*)(const double2*)R.sx + im;
+            lu_wave_exact(R.Ti, R.pT, N, [&](int i) { return gload(v + 2 * i); }, [&](int i, double z) { xd[2 * i] = z; });
         }
     }
     __syncthreads();
@@ -1712,15 +1718,16 @@ __global__ __launch_bounds__(NT) void k_m0(const RunDesc* __restrict__ runs, con
         // of any store), swept, stored
         const int lane = tid & 63, im = (tid >> 6) & 1;
         double xr[3] = {0.0, 0.0, 0.0};
-        auto rhs = [&](int q) {
-            const int i = lane + 64 * q;
-            const double2 v = (i < N) ? lload(x + gload(R.pT + i)) : mk(0.0, 0.0);
-            return im ? v.y : v.x;
-        };
         if (tid < 128) {
 #pragma unroll
-            for (int q = 0; q < 3; ++q) xr[q] = rhs(q);
-
+            for (int q = 0; q < 3; ++q) {
+                const int i = lane + 64 * q;
+                const double2 v = (i < N) ? lload(x + gload(R.pT + i)) : mk(0.0, 0.0);
+                xr[q] = im ? v.y : v.x;
+            }
+        }
+        __syncthreads();
+        if (tid < 128) {
             const LDS_AS double* fl = (const LDS_AS double*)f;
             auto col = [fl, lane, N](int p, int j) { return fl[lane + 64 * p + N * j]; };
             if (N <= 128) {
@@ -1731,15 +1738,15 @@ __global__ __launch_bounds__(NT) void k_m0(const RunDesc* __restrict__ runs, con
             } else {
                 lu_solve_wave<3, 4>(xr, col, N);
             }
-            lu_wave_check<3>(xr, R.Ti, N, rhs);
-        }
-        __syncthreads();   // every gather of x is done
-        if (tid < 128) {
             LDS_AS double* xd = (LDS_AS double*)x + im;
 #pragma unroll
             for (int q = 0; q < 3; ++q) {
                 const int i = lane + 64 * q;
                 if (i < N) xd[2 * i] = xr[q];
+            }
+            if (__any(!lu_wave_usual<3>(xr, N))) {
+                const double* v = (const double*)(const double2*)R.sx + im;
+                lu_wave_exact(R.Ti, R.pT, N, [&](int i) { return gload(v + 2 * i); }, [&](int i, double z) { xd[2 * i] = z; });
             }
         }
         __syncthreads();
@@ -3446,23 +3453,31 @@ __device__ __forceinline__ void fu_stage(const double* A, const int N, double* s
     for (int c = wv; 128 * c < N * N; c += (int)blockDim.x / 64) lds_dma(fr, (double2*)(stg + 128 * c), 16 * (64 * c + lane));
 }
 template <int SLOTS, class Col>
-__device__ __forceinline__ void fu_lu(const double* A, const int* perm, const int N, const double* x, double* y, Col col)
+__device__ __forceinline__ void fu_lu(const int* perm, const int N, const double* x, double* y, Col col, int& odd)
 {
     const int lane = threadIdx.x & 63, im = (threadIdx.x >> 6) & 1;
     double v[SLOTS];
-    auto rhs = [&](int q) {
-        const int r = lane + 64 * q;
-        return r < N ? ((const LDS_AS double*)x)[4 * gload(perm + r) + im] : 0.0;
-    };
 #pragma unroll
-    for (int q = 0; q < SLOTS; ++q) v[q] = rhs(q);
+    for (int q = 0; q < SLOTS; ++q) {
+        const int r = lane + 64 * q;
+        v[q] = r < N ? ((const LDS_AS double*)x)[4 * gload(perm + r) + im] : 0.0;
+    }
     lu_solve_wave<SLOTS, 8>(v, col, N);
-    lu_wave_check<SLOTS>(v, A, N, rhs);
 #pragma unroll
     for (int q = 0; q < SLOTS; ++q) {
         const int r = lane + 64 * q;
         if (r < N) y[4 * r + im] = v[q];
     }
+    if (!lu_wave_usual<SLOTS>(v, N)) odd = 1;
+}
+// after a barrier, where odd tells that it has to be done again
+__device__ __forceinline__ void fu_lu_exact(const double* A, const int* perm, const int N, const double* x, double* y)
+{
+    const int im = threadIdx.x >> 6;
+    if (im < 2)
+        lu_wave_exact(A, perm, N, [&](int i) { return ((const LDS_AS double*)x)[4 * i + im]; },
+                      [&](int i, double z) { y[4 * i + im] = z; });
+    __syncthreads();
 }
 
 // Set-up shared by the two kernels.  The workgroup's modes m0 .. m0 + nmo - 1
@@ -3496,6 +3511,8 @@ __device__ __forceinline__ void fu_lu(const double* A, const int* perm, const in
         e_[j] = m + (size_t)Nm1 * (i < N ? i : 0);                                                      \
     }                                                                                                   \
     extern __shared__ double2 stg_[];                                                                   \
+    __shared__ int odd;   /* the m = 0 (or psi) solve has to be done again */                           \
+    if (tid == 0) odd = 0;                                                                              \
     auto V = [&](int k, int j = 0) { return (double*)stg_ + k * 4 * K4 + j * VS; };                     \
     /* the modes' columns of fields a and b into vector k */                                            \
     auto fill = [&](int k, const double2* a, const double2* b) {                                        \
@@ -3571,19 +3588,20 @@ enum FuVec : int { FV_C = 0, FV_Y = 1, FV_R = 2, FV_P1 = 3, FV_P2 = 4, FV_P3 = 5
             if (staged) {                                                                               \
                 const LDS_AS double* fl = (const LDS_AS double*)V(FU_ZVEC);                             \
                 auto cl = [fl, lane, N](int p, int q) { return fl[lane + 64 * p + N * q]; };            \
-                if (N <= 64) fu_lu<1>(R.Ti, R.pT, N, V(FV_R), V(FV_Y), cl);                             \
-                else if (N <= 128) fu_lu<2>(R.Ti, R.pT, N, V(FV_R), V(FV_Y), cl);                       \
-                else fu_lu<3>(R.Ti, R.pT, N, V(FV_R), V(FV_Y), cl);                                     \
+                if (N <= 64) fu_lu<1>(R.pT, N, V(FV_R), V(FV_Y), cl, odd);                              \
+                else if (N <= 128) fu_lu<2>(R.pT, N, V(FV_R), V(FV_Y), cl, odd);                        \
+                else fu_lu<3>(R.pT, N, V(FV_R), V(FV_Y), cl, odd);                                      \
             } else {                                                                                    \
                 const BRes fr = bres(R.Ti, sizeof(double) * (size_t)N * N);                             \
                 auto cg = [fr, lane, N](int p, int q) { return bload(fr, 8 * (lane + 64 * p + N * q)); }; \
-                if (N <= 128) fu_lu<2>(R.Ti, R.pT, N, V(FV_R), V(FV_Y), cg);                            \
-                else fu_lu<3>(R.Ti, R.pT, N, V(FV_R), V(FV_Y), cg);                                     \
+                if (N <= 128) fu_lu<2>(R.pT, N, V(FV_R), V(FV_Y), cg, odd);                             \
+                else fu_lu<3>(R.pT, N, V(FV_R), V(FV_Y), cg, odd);                                      \
             }                                                                                           \
         } else {                                                                                        \
             for (int t = wv - 2; t < nrb; t += NW - 2) fu_rows<1>(R.Ui, N, N, N, t, V(FV_R), V(FV_Y), V(FV_Y), N, 12, 0); \
         }                                                                                               \
         __syncthreads();                                                                                \
+        if (odd) fu_lu_exact(R.Ti, R.pT, N, V(FV_R), V(FV_Y));                                          \
     } while (0)
 
 // One IMEX step of the workgroup's modes: k_imex_pre, the temperature solve,
@@ -3897,9 +3915,10 @@ constexpr int FU1_MAXN = 64;
             const int lane = tid & 63;                                                                  \
             const LDS_AS double* fl = (const LDS_AS double*)V(FU_ZVEC);                                 \
             auto cl = [fl, lane, N](int p, int q) { return fl[lane + 64 * p + N * q]; };                \
-            fu_lu<1>(R.Li + (size_t)m0 * N * N, R.pL + (size_t)m0 * N, N, V(FV_R) + 2, V(FV_Y), cl);   /* N <= FU1_MAXN */         \
+            fu_lu<1>(R.pL + (size_t)m0 * N, N, V(FV_R) + 2, V(FV_Y), cl, odd);   /* N <= FU1_MAXN */    \
         }                                                                                               \
         __syncthreads();                                                                                \
+        if (odd) fu_lu_exact(R.Li + (size_t)m0 * N * N, R.pL + (size_t)m0 * N, N, V(FV_R) + 2, V(FV_Y)); \
         products(2, 0x10, 0x11, 0x43);                                                                  \
         __syncthreads();                                                                                \
         if (tid < 4) {                                                                                  \

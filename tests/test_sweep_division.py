@@ -73,13 +73,16 @@ def test_quotients(tmp_path):
 
 
 def test_every_solve_by_sweeps_is_checked():
-    """Each place that sweeps ends in the check of its solution."""
+    """Each place that sweeps looks over its solution, and has the solve that
+    stands in for it."""
     src = open(os.path.join(CSRC, "fdns_kernels.hip")).read()
     for name in ("void m0_solve(", "void k_m0(", "void fu_lu("):
         body = src[src.index(name):]
         body = body[:body.index("\n}\n")]
         sweeps = [m.end() for m in re.finditer(r"lu_solve_wave<|lu_wave_bwd<", body)]
-        assert sweeps and body.index("lu_wave_check<") > max(sweeps), name
+        assert sweeps and body.index("lu_wave_usual<") > max(sweeps), name
+        assert name == "void fu_lu(" or "lu_wave_exact(" in body, name
+    assert src.count("if (odd) fu_lu_exact(") == 2   # the m = 0 temperature, and psi
     body = src[src.index("void k_solve_lu("):]
     body = body[:body.index("\n}\n")]
     assert body.index("lu_solve_reg(") < body.index("usual(x0.x)") < body.index("lu_solve_exact(")
