@@ -3452,8 +3452,15 @@ __device__ __forceinline__ void fu_stage(const double* A, const int N, double* s
     const BRes fr = bres(A, sizeof(double) * (size_t)N * N);
     for (int c = wv; 128 * c < N * N; c += (int)blockDim.x / 64) lds_dma(fr, (double2*)(stg + 128 * c), 16 * (64 * c + lane));
 }
+// Whether the solve has to be done again: a flag behind the staged factor (its
+// last load ends within 128 doubles of it), or in its place.  (A variable of
+// its own moved the vectors: k_imex_modes<2>, 129 x 64, 57.8 -> 59.7 us.)
+__device__ __forceinline__ LDS_AS int* fu_odd(double* factor, const int N, const bool staged)
+{
+    return (LDS_AS int*)(factor + (staged ? N * N + 160 : 0));
+}
 template <int SLOTS, class Col>
-__device__ __forceinline__ void fu_lu(const int* perm, const int N, const double* x, double* y, Col col, int& odd)
+__device__ __forceinline__ void fu_lu(const int* perm, const int N, const double* x, double* y, Col col, LDS_AS int& odd)
 {
     const int lane = threadIdx.x & 63, im = (threadIdx.x >> 6) & 1;
     double v[SLOTS];
@@ -3511,8 +3518,6 @@ __device__ __forceinline__ void fu_lu_exact(const double* A, const int* perm, co
         e_[j] = m + (size_t)Nm1 * (i < N ? i : 0);                                                      \
     }                                                                                                   \
     extern __shared__ double2 stg_[];                                                                   \
-    __shared__ int odd;   /* the m = 0 (or psi) solve has to be done again */                           \
-    if (tid == 0) odd = 0;                                                                              \
     auto V = [&](int k, int j = 0) { return (double*)stg_ + k * 4 * K4 + j * VS; };                     \
     /* the modes' columns of fields a and b into vector k */                                            \
     auto fill = [&](int k, const double2* a, const double2* b) {                                        \
@@ -3582,6 +3587,8 @@ enum FuVec : int { FV_C = 0, FV_Y = 1, FV_R = 2, FV_P1 = 3, FV_P2 = 4, FV_P3 = 5
 #define FU_ZERO                                                                                         \
     do {                                                                                                \
         if (staged) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                                    \
+        LDS_AS int& odd = *fu_odd(V(FU_ZVEC), N, staged != 0);                                          \
+        if (tid == 0) odd = 0;                                                                          \
         __syncthreads();                                                                                \
         if (wv < 2) {                                                                                   \
             const int lane = tid & 63;                                                                  \
@@ -3910,6 +3917,8 @@ constexpr int FU1_MAXN = 64;
 #define FU_LAP                                                                                          \
     do {                                                                                                \
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                                                \
+        LDS_AS int& odd = *fu_odd(V(FU_ZVEC), N, true);                                                 \
+        if (tid == 0) odd = 0;                                                                          \
         __syncthreads();                                                                                \
         if (wv < 2) {                                                                                   \
             const int lane = tid & 63;                                                                  \
