@@ -808,9 +808,8 @@ __device__ __forceinline__ void lds_dma(BRes r, double2* lds, int off)
 // receives its column updates in dgetrs' column order.  Each thread's first
 // GEMV row of a block is loaded before the diagonal solve, so that the two
 // factor reads of a block overlap.
-template <int NT, int NB, int KR>
-__device__ void lu_solve_k(double2* x, double2* xs, const double* __restrict__ A, const int* __restrict__ perm,
-                           const int n)
+template <int NT, int NB>
+__device__ __forceinline__ void lu_solve(double2* x, double2* xs, const double* __restrict__ A, const int* __restrict__ perm, const int n)
 {
     const int tid = threadIdx.x;
     // dgetrs' row interchanges as one gather through the LDS scratch xs
@@ -822,17 +821,10 @@ __device__ void lu_solve_k(double2* x, double2* xs, const double* __restrict__ A
     // unit lower triangle
     for (int j0 = 0; j0 < n; j0 += NB) {
         const int jb = min(NB, n - j0);
-        // the factor entries of this thread's first KR GEMV rows (i0 + k NT),
-        // all loaded while wavefront 0 solves the diagonal block; further rows
-        // in groups of KR, each group's loads issued together
         const int i0 = j0 + jb + tid;
-        double l0[KR][NB];
+        double l0[NB];
 #pragma unroll
-        for (int k = 0; k < KR; ++k) {
-            const int i = i0 + k * NT;
-#pragma unroll
-            for (int j = 0; j < NB; ++j) l0[k][j] = (i < n && j < jb) ? gload(A + (size_t)i + ld * (size_t)(j0 + j)) : 0.0;
-        }
+        for (int j = 0; j < NB; ++j) l0[j] = (i0 < n && j < jb) ? gload(A + (size_t)i0 + ld * (size_t)(j0 + j)) : 0.0;
         if (tid < 64) {
             const int l = tid;
             double a[NB];
@@ -862,21 +854,13 @@ __device__ void lu_solve_k(double2* x, double2* xs, const double* __restrict__ A
             }
             lstore(x + i, xi);
         };
-#pragma unroll
-        for (int k = 0; k < KR; ++k)
-            if (i0 + k * NT < n) lrow(i0 + k * NT, l0[k]);
+        if (i0 < n) lrow(i0, l0);
 #pragma unroll 1
-        for (int ib = i0 + KR * NT; ib < n; ib += KR * NT) {
-            double lv[KR][NB];
+        for (int i = i0 + NT; i < n; i += NT) {
+            double lv[NB];
 #pragma unroll
-            for (int k = 0; k < KR; ++k) {
-                const int i = ib + k * NT;
-#pragma unroll
-                for (int j = 0; j < NB; ++j) lv[k][j] = (i < n && j < jb) ? gload(A + (size_t)i + ld * (size_t)(j0 + j)) : 0.0;
-            }
-#pragma unroll
-            for (int k = 0; k < KR; ++k)
-                if (ib + k * NT < n) lrow(ib + k * NT, lv[k]);
+            for (int j = 0; j < NB; ++j) lv[j] = (i < n && j < jb) ? gload(A + (size_t)i + ld * (size_t)(j0 + j)) : 0.0;
+            lrow(i, lv);
         }
         __syncthreads();
     }
@@ -885,13 +869,9 @@ __device__ void lu_solve_k(double2* x, double2* xs, const double* __restrict__ A
     for (int bi = nblk - 1; bi >= 0; --bi) {
         const int j0 = bi * NB;
         const int jb = min(NB, n - j0);
-        double u0[KR][NB];
+        double u0[NB];
 #pragma unroll
-        for (int k = 0; k < KR; ++k) {
-            const int i = tid + k * NT;
-#pragma unroll
-            for (int j = 0; j < NB; ++j) u0[k][j] = (i < j0 && j < jb) ? gload(A + (size_t)i + ld * (size_t)(j0 + j)) : 0.0;
-        }
+        for (int j = 0; j < NB; ++j) u0[j] = (tid < j0 && j < jb) ? gload(A + (size_t)tid + ld * (size_t)(j0 + j)) : 0.0;
         if (tid < 64) {
             const int l = tid;
             double a[NB];
@@ -922,32 +902,16 @@ __device__ void lu_solve_k(double2* x, double2* xs, const double* __restrict__ A
             }
             lstore(x + i, xi);
         };
-#pragma unroll
-        for (int k = 0; k < KR; ++k)
-            if (tid + k * NT < j0) urow(tid + k * NT, u0[k]);
+        if (tid < j0) urow(tid, u0);
 #pragma unroll 1
-        for (int ib = tid + KR * NT; ib < j0; ib += KR * NT) {
-            double uv[KR][NB];
+        for (int i = tid + NT; i < j0; i += NT) {
+            double uv[NB];
 #pragma unroll
-            for (int k = 0; k < KR; ++k) {
-                const int i = ib + k * NT;
-#pragma unroll
-                for (int j = 0; j < NB; ++j) uv[k][j] = (i < j0 && j < jb) ? gload(A + (size_t)i + ld * (size_t)(j0 + j)) : 0.0;
-            }
-#pragma unroll
-            for (int k = 0; k < KR; ++k)
-                if (ib + k * NT < j0) urow(ib + k * NT, uv[k]);
+            for (int j = 0; j < NB; ++j) uv[j] = (i < j0 && j < jb) ? gload(A + (size_t)i + ld * (size_t)(j0 + j)) : 0.0;
+            urow(i, uv);
         }
         __syncthreads();
     }
-}
-
-// lu_solve_k with the GEMV rows of a thread loaded one at a time (the radial
-// kernels, whose registers are spoken for).
-template <int NT, int NB>
-__device__ void lu_solve(double2* x, double2* xs, const double* __restrict__ A, const int* __restrict__ perm, const int n)
-{
-    lu_solve_k<NT, NB, 1>(x, xs, A, perm, n);
 }
 
 constexpr int SOLVE_NB = 8;    // column block of lu_solve
