@@ -3309,10 +3309,12 @@ __global__ __launch_bounds__(64 * TW) __attribute__((amdgpu_waves_per_eu(2))) vo
 // In a launch of few modes a workgroup has one; above one mode per CU it has
 // two (P), which share the loads of the shared operators.
 //
-// What bounds it: the operators through the CU's L1 (about 24 cycles per 1 KiB
-// load of four columns' 32 rows, 16 where the columns start on a cache line:
-// the leading dimension LE), the latency of the few loads of a phase, and for
-// m = 0 the sweeps of its temperature, solved in dgetrs' order.  Measured, one
+// What bounds it: the operators through the CU's L1, 18 - 20 cycles per 1 KiB
+// load of four columns' 32 rows (fewest where the columns start on a cache
+// line: the leading dimension LE), which by the counters keeps a busy CU's
+// address unit occupied 40 % of the time at 65 x 128 and 53 % at 129 x 128; the
+// latency of the few loads of a phase; and for m = 0 the sweeps of its
+// temperature, solved in dgetrs' order.  Measured, one
 // run's CNAB2 step (nonlinear pass included), tiles -> here: 33 x 16 46 -> 27
 // us, 65 x 128 70 -> 35, 97 x 256 105 -> 53, 129 x 128 150 -> 53; ARS443:
 // 169 -> 85, 237 -> 119, 382 -> 191, 527 -> 189.
@@ -5402,12 +5404,13 @@ size_t tile_stage_bytes(const Shape& sh, int nx)
 //     (49 x 96), 1.03 at 520 (64 x 128), 1.4 at 528 (17 x 64); 1.0 at 784;
 //   - one run, whose column tiles are few: 1.1 - 1.4 at 385 (65, 97, 129 x
 //     768), but 0.97 at 513 (65 x 1024).
+constexpr int NCU = 256;   // compute units of an MI355X
 static int fu_modes(const Shape& sh, int nrun)
 {
     if (sh.N > FU_MAXN) return 0;
-    if (nrun * sh.Nm1 <= 256) return 1;
+    if (nrun * sh.Nm1 <= NCU) return 1;
     const int G = nrun * fu_groups(sh.Nm1, 2);
-    return G <= (sh.N <= 64 ? 512 : (nrun == 1 ? 400 : 256)) ? 2 : 0;
+    return G <= (sh.N <= 64 ? 2 * NCU : (nrun == 1 ? 400 : NCU)) ? 2 : 0;
 }
 
 bool mode_fused(const Shape& sh, int nrun) { return fu_modes(sh, nrun) != 0; }
@@ -5417,7 +5420,7 @@ template <class K1, class K2, class... A>
 static void fu_launch(K1 k1, K2 k2, const RunDesc* runs, int nrun, const Shape& sh, hipStream_t st, A... a)
 {
     const int P = fu_modes(sh, nrun), G = nrun * fu_groups(sh.Nm1, P);
-    const bool one = G <= 256;   // alone on its CU: more wavefronts, m = 0's factor in LDS
+    const bool one = G <= NCU;   // alone on its CU: more wavefronts, m = 0's factor in LDS
     const dim3 grid(padded_grid(G)), block(64 * fu_waves(sh.N, one));
     const size_t lds = fu_lds(sh.N, P, one);
     if (P == 1) hipLaunchKernelGGL(k1, grid, block, lds, st, runs, sh, nrun, (int)one, a...);
@@ -5478,7 +5481,7 @@ void launch_rk_post(const RunDesc* runs, int nrun, const Shape& sh, int s, hipSt
 template <class K, class... A>
 static void fu1_launch(K k, bool factor, const RunDesc* runs, int nrun, const Shape& sh, hipStream_t st, A... a)
 {
-    hipLaunchKernelGGL(k, dim3(padded_grid(nrun * sh.Nm1)), dim3(64 * fu_waves(sh.N, nrun * sh.Nm1 <= 256)), fu_lds(sh.N, 1, factor),
+    hipLaunchKernelGGL(k, dim3(padded_grid(nrun * sh.Nm1)), dim3(64 * fu_waves(sh.N, nrun * sh.Nm1 <= NCU)), fu_lds(sh.N, 1, factor),
                        st, runs, sh, nrun, a...);
 }
 
