@@ -1568,18 +1568,17 @@ __device__ void m0_solve(const RunDesc& R, const Shape& sh, double2* smem)
     for (int i = tid; i < N; i += NT) gstore((double2*)R.sy + i, lload(x + i));
 }
 
-// The implicit solves of one phase of a step for a group of runs:
-// phase 0 the temperature (AT), phase 1 the vorticity-streamfunction (AF) of
+// The implicit solves of one phase of a step for a group of runs in inverse
+// mode (LU mode: k_solve_lu): phase 0 the temperature (AT), phase 1 the vorticity-streamfunction (AF) of
 // modes m >= 1 and the mean flow (A_uphi) of m = 0.  Right-hand sides come
 // from each run's solve area sx, solutions go to its solution area sy, both
 // mode-major: rows 0..2N-1 of mode m at +2N m (temperature or psi in rows
 // 0..N-1, omega or mean flow in rows N..2N-1).
-//   LU mode: one workgroup per (run, mode), dgetrs in its operation order.
-//   Inverse mode: one workgroup per (chunk of up to SOLVE_RHS runs that share
+//   One workgroup per (chunk of up to SOLVE_RHS runs that share
 //   an operator set, mode, group of four 16-row strips of the inverse), the
 //   MFMA product over the chunk's right-hand sides.  The m = 0 temperature,
 //   whose wall derivative is the Nusselt number, keeps dgetrs: with m0n > 0
-//   (phase 0, inverse mode) the launch's first blocks solve it for runs
+//   (phase 0) the launch's first blocks solve it for runs
 //   0..m0n-1 (m0_solve), the rest do the batched solves; otherwise k_m0
 //   solves it beside this kernel.
 template <int phase>

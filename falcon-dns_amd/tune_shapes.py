@@ -7,7 +7,10 @@ BPR353 by default: the schemes of the served stream) is stepped twice, the
 autotuner times every option on clones of it, and the ensemble's time per
 step (graph replays) is then measured with the plain choice and with the
 chosen one, so each line states its own gain.  Results are bit for bit the
-same under every choice; only the time changes.
+same under every choice; only the time changes.  Groups small enough for whole
+mode updates launch no tiles and no batched solves, and the autotuner leaves
+those choices as they were: take --runs large enough for the groups in question
+(the stored lines of the served shapes are from when such groups took tiles).
 
     python3 falcon-dns_amd/tune_shapes.py                     # the served shapes
     python3 falcon-dns_amd/tune_shapes.py --shapes 97x256 --runs 64
