@@ -43,7 +43,9 @@ SWEEP_FN LuxShare lux_backward(int nblk, int wv)
 // x / d by the reciprocal rcp = 1 / d (rounded): quotient, remainder,
 // correction (Markstein), which gives the correctly rounded quotient where
 // neither the reciprocal (rcp_safe) nor the quotient or the remainder (usual)
-// leaves the normal range.  Beyond it an infinity, and a quotient next to the
+// leaves the normal range: |x| >= 2^-900 keeps the remainder's 106 bits above
+// 2^-1022, and runs that decay go a long way before they leave it (1e-241).
+// Beyond it an infinity, and a quotient next to the
 // largest number, give NaN.
 SWEEP_DEV inline double div_by(double x, double d, double rcp)
 {
@@ -57,7 +59,7 @@ SWEEP_DEV inline double div_last(double x, double d, double rcp)
     const double q = div_by(x, d, rcp);
     return q == 0.0 ? x : q;
 }
-SWEEP_DEV inline bool rcp_safe(double d) { return __builtin_fabs(d) > 0x1p-400 && __builtin_fabs(d) < 0x1p400; }
-SWEEP_DEV inline bool usual(double q) { return q == 0.0 || (__builtin_fabs(q) > 0x1p-500 && __builtin_fabs(q) < 0x1p500); }
+SWEEP_DEV inline bool rcp_safe(double d) { return __builtin_fabs(d) > 0x1p-100 && __builtin_fabs(d) < 0x1p100; }
+SWEEP_DEV inline bool usual(double q) { return q == 0.0 || (__builtin_fabs(q) > 0x1p-800 && __builtin_fabs(q) < 0x1p900); }
 
 }  // namespace fdns
